@@ -63,6 +63,62 @@ def test_conv_forward_and_backward(ctx, ci, co, ks, shape):
     assert close(gw.to_host().reshape(gw0.shape), gw0, 1e-5)
 
 
+def to_bf16(a):
+    """a rounded to BF16 (nearest even), as FP64."""
+    u = np.ascontiguousarray(a, np.float32).view(np.uint32).astype(np.uint64)
+    u = (u + 0x7FFF + ((u >> 16) & 1)) & 0xFFFF0000
+    return u.astype(np.uint32).view(np.float32).astype(np.float64)
+
+
+# edges of the position tiles (16 x 4 x 4, 8 x 8 x 4, 8 x 4 x 2), of the channel
+# groups (8, 16, 32 in BF16; 4, 8, 16 in FP32) and of the row tiles (16, 32, 64);
+# the last ones have the 256 workgroups that take the large tiles
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("ci,co,ks,shape", [(1, 1, 3, (1, 1, 1)), (2, 16, 3, (5, 4, 17)),
+                                            (8, 17, 3, (3, 9, 16)), (9, 33, 3, (4, 5, 15)),
+                                            (17, 65, 3, (2, 3, 8)), (33, 64, 1, (3, 5, 9)),
+                                            (16, 16, 3, (33, 33, 64)), (20, 40, 3, (34, 40, 41)),
+                                            (4, 20, 1, (18, 66, 65)), (5, 50, 3, (17, 65, 60))])
+def test_conv_tiles_match_oracle(ctx, ci, co, ks, shape, bf16):
+    """Forward, data and weight gradients at the edges of the tiling, in both
+    arithmetic modes.  BF16: the oracle takes the rounded operands, so what
+    remains is FP32 accumulation, as in FP32 mode: a sum of m products differs
+    by at most m 2^-24 of the sum of their magnitudes, about sqrt(m) in
+    practice; 1e-5 of the largest entry holds 10 times that for the 74,000
+    positions of the largest weight gradient here."""
+    rng = np.random.default_rng(1000 * ci + co + shape[2])
+    rnd = to_bf16 if bf16 else lambda a: np.asarray(a, np.float32).astype(np.float64)
+    x = rnd(rng.standard_normal((ci,) + shape))
+    w = rnd(rng.standard_normal((co, ci, ks ** 3)) / np.sqrt(ci * ks ** 3))
+    b = rng.standard_normal(co).astype(np.float32).astype(np.float64)
+    dy = rnd(rng.standard_normal((co,) + shape))
+    L, h, P = E.lib(), ctx.h, int(np.prod(shape))
+    print(f"conv3d ci={ci} co={co} ks={ks} shape={shape} bf16={bf16}", flush=True)
+    dx_, dw_, db_, ddy = f32(ctx, x), f32(ctx, w), f32(ctx, b), f32(ctx, dy)
+    y, gx = E.DeviceArray(ctx, (co * P,), np.float32), f32(ctx, np.ones(ci * P))
+    gw, gb = E.DeviceArray(ctx, (w.size,), np.float32), f32(ctx, np.ones(co))
+    E._check(L.ttdft_nn_set_math(h, E.NN_BF16 if bf16 else E.NN_FP32))
+    try:
+        E._check(L.ttdft_nn_conv3d_forward(h, dx_.ptr, ci, dims(shape), dw_.ptr, db_.ptr, co, ks,
+                                           y.ptr, 0))
+        E._check(L.ttdft_nn_conv3d_backward_data(h, ddy.ptr, co, dims(shape), dw_.ptr, ci, ks,
+                                                 gx.ptr, 1))
+        E._check(L.ttdft_nn_conv3d_backward_weight(h, dx_.ptr, ci, dims(shape), ddy.ptr, co, ks,
+                                                   gw.ptr, None, 0))
+        first = gw.to_host()
+        E._check(L.ttdft_nn_conv3d_backward_weight(h, dx_.ptr, ci, dims(shape), ddy.ptr, co, ks,
+                                                   gw.ptr, gb.ptr, 1))
+    finally:
+        E._check(L.ttdft_nn_set_math(h, E.NN_FP32))
+    gx0, gw0, gb0 = U.conv3d_backward(x, w, dy, ks)
+    y0 = U.conv3d(x, w, b, ks)
+    assert close(y.to_host().reshape(y0.shape), y0, 1e-5)
+    assert close(gx.to_host().reshape(gx0.shape), gx0 + 1, 1e-5)
+    assert close(first.reshape(gw0.shape), gw0, 1e-5)
+    assert close(gw.to_host().reshape(gw0.shape), 2 * gw0, 1e-5)
+    assert close(gb.to_host(), gb0 + 1, 1e-5)
+
+
 def test_activation_pool_upsample_loss_adam(ctx):
     rng = np.random.default_rng(7)
     L, h = E.lib(), ctx.h
