@@ -652,6 +652,45 @@ def test_dense_product_tilings(ctx, dims, k):
         assert np.all(Y[:, k:] == 7.0)  # columns past k untouched
 
 
+@pytest.mark.parametrize("n", [1, 31, 33, 127, 129, 255, 257, 300])
+@pytest.mark.parametrize("k", [1, 17, 96, 97])
+def test_dense_product_row_blocks_and_parts(ctx, monkeypatch, n, k):
+    """Row blocks of 128 (FP64) and 256 (FP32) rows, stages of 32 columns and
+    one to three parts of them at their edges, in a filter whose steps hand
+    the block on as operand fragments.  FP32 keeps FP32 accuracy: m - 1 steps
+    with sums of n products each, an error of 2^-24 per operation that adds
+    up like a random walk, times the filter's growth (4 here)."""
+    rng = np.random.default_rng(n + k)
+    A = rng.standard_normal((n, n)) / np.sqrt(n)
+    A = A + A.T
+    ham = E.Hamiltonian(ctx, n, np.arange(n + 1, dtype=np.int64) * n,
+                        np.tile(np.arange(n, dtype=np.int32), n), A.reshape(-1), 0, None, None,
+                        None, None, copies=E.HAM_F64 | E.HAM_F32)
+    assert ham.format()[0] == 2
+    X = rng.standard_normal((n, k))
+    m, a, b, a0 = 4, -1.0, 3.0, -3.0
+    e, c = (b - a) / 2, (b + a) / 2
+    for dtype, npdt, tol in ((E.F64, np.float64, 1e-13),
+                             (E.F32, np.float32, 4 * 2.0 ** -24 * np.sqrt(3.0 * n + 16))):
+        Xc = X.astype(npdt)
+        A_c = A.astype(npdt).astype(np.float64)
+        sigma = e / (a0 - c)
+        gamma = 2.0 / sigma
+        prev = Xc.astype(np.float64)
+        cur = (sigma / e) * (A_c @ prev - c * prev)
+        for _ in range(2, m):
+            nxt = 1.0 / (gamma - sigma)
+            prev, cur = cur, (2 * nxt / e) * (A_c @ cur - c * cur) - sigma * nxt * prev
+            sigma = nxt
+        for parts in ("1", "2", "3"):
+            monkeypatch.setenv("TTDFT_DENSE_LDS", parts)
+            dX = dev(ctx, Xc, npdt)
+            print(f"dense row blocks n={n} k={k} dtype={dtype} parts={parts}", flush=True)
+            ctx.cheb_filter(ham, dX.ptr, k, k, m, a, b, a0, 1, dtype)
+            assert rel(dX.to_host().astype(np.float64), cur) < tol
+    ham.free()
+
+
 def test_dense_storage_reuse_across_hamiltonians(ctx):
     """Hamiltonians of different sizes built and freed in turn on one context:
     the dense storage and the projector fold come from the context's block

@@ -857,7 +857,7 @@ int ttdft_cheb_filter(ttdft_ctx ctx, ttdft_ham H, void *X, int64_t ldx, int32_t 
         double alpha = sigma1 / e, beta = alpha * (-c);
         // Y_1 = alpha H X + beta X   -> B
         TT_TRY(ham_step(ctx, H, Ac, ldx, Bc, ldx, nullptr, 0, cols, dtype, alpha, beta, 0.0, 1,
-                        0));
+                        0, nullptr, 0, {false, target > 1}));
         char *cur = Bc, *prev = Ac;
         for (int it = 2; it <= target; ++it) {
             const double sigma2 = 1.0 / (gamma - sigma);
@@ -866,7 +866,7 @@ int ttdft_cheb_filter(ttdft_ctx ctx, ttdft_ham H, void *X, int64_t ldx, int32_t 
             const double delta = -sigma * sigma2;
             // Y_it = alpha H Y_{it-1} + beta Y_{it-1} + delta Y_{it-2}, written over Y_{it-2}
             TT_TRY(ham_step(ctx, H, cur, ldx, prev, ldx, prev, ldx, cols, dtype, alpha, beta,
-                            delta, 1, 1));
+                            delta, 1, 1, nullptr, 0, {true, it < target}));
             char *t = cur;
             cur = prev;
             prev = t;

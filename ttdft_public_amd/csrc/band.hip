@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "lds_ring.h"
 
 namespace ttdft {
 namespace {
@@ -81,29 +82,6 @@ struct BrickArgs {
     int use_beta, use_delta;
     int32_t light_last;  // ragged last x-chunk's units after all full ones, per XCD
 };
-
-typedef __attribute__((address_space(3))) void lds_void;
-
-// s_waitcnt immediate: vmcnt in bits [3:0] and [15:14], expcnt [6:4], lgkmcnt [11:8].
-// Waits until at most n vector-memory operations of this wave are outstanding
-// and all LDS operations are done.
-#define TT_WAIT_VM_LDS(n)                                                                   \
-    do {                                                                                    \
-        asm volatile("" ::: "memory");                                                      \
-        __builtin_amdgcn_s_waitcnt(((n) & 15) | ((((n) >> 4) & 3) << 14) | (7 << 4) | (0 << 8)); \
-    } while (0)
-#define TT_WAIT_ALL() __builtin_amdgcn_s_waitcnt(0)
-
-// Workgroup barrier without the memory fence of __syncthreads(): that fence
-// would also wait for the line loads still in flight into LDS.  The waits
-// the barrier needs are issued explicitly before it; the empty asm keeps the
-// compiler from moving memory operations across.
-__device__ __forceinline__ void line_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 
 // N LDS loads of T from byte offsets OFF0 + i STRIDE past p, completed inside
 // the asm block (s_waitcnt lgkmcnt(0)); every output is used by the caller.
@@ -738,6 +716,11 @@ bool band_shape(int32_t rx, int32_t ry, int32_t rz, int bx, int by, int bz, int6
     const int64_t band_slots = n * (int64_t)(2 * bx + 1) * (2 * by + 1) * (2 * bz + 1);
     const double fill = band_slots > 0 ? (double)nnz / (double)band_slots : 0.0;
     if (bx < 1 || bx > 7 || fill < 0.15 || rx < 4) return false;
+    // Bands that reach across the whole basis (at most 8 functions in x) leave
+    // nothing to skip: a matrix that qualifies for dense storage goes there,
+    // where no column is padding and small products spread over more
+    // workgroups (512 x 16 FP64: 0.012 against 0.069 ms).
+    if (bx >= rx - 1 && by >= ry - 1 && bz >= rz - 1 && dense_storage_fits(n, nnz)) return false;
     b->ks = (4 + 2 * bx + 3) / 4;
     b->gxn = (rx + 3) / 4;
     b->hyn = (ry + 3) / 4;

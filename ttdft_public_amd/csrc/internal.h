@@ -185,6 +185,7 @@ int dev_fill_uniform(ttdft_ctx ctx, double *f, int64_t n, uint64_t seed, double 
 int small_orth(ttdft_ctx ctx, double *Y, int32_t n, int32_t b);
 // Dense storage (format 2) of H_loc when it is nearly full and small enough
 // (no-op otherwise); drop_dense frees it.
+bool dense_storage_fits(int64_t n, int64_t nnz);
 int maybe_build_dense(ttdft_ctx ctx, ttdft_ham_s *H, int copies);
 int finish_dense(ttdft_ctx ctx, ttdft_ham_s *H, int copies);
 // Device blocks that live and die with Hamiltonians, rebuilt every SCF
@@ -217,13 +218,21 @@ int launch_band_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t
                      const void *W, void *Y, int64_t ldy, const void *Z, int64_t ldz,
                      int32_t k, int dtype, double alpha, double beta, double delta,
                      int use_beta, int use_delta);
+// Consecutive applications of one H, each to the result of the one before
+// (same states, leading dimensions and work space, nothing else using that
+// work space between them): have: the previous step left its result in the
+// product's own operand layout there; want: do so for the next one.  Storage
+// forms without such a layout ignore it.
+struct StepChain {
+    bool have = false, want = false;
+};
 // Full H application (nl projection + fused SpMM) with the given epilogue.
 // The projections go to ws (ws_bytes long; an error if they do not fit) when
 // ws is given, else to the context's scratch.
 int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, void *Y,
              int64_t ldy, const void *Z, int64_t ldz, int32_t k, int dtype, double alpha,
              double beta, double delta, int use_beta, int use_delta, void *ws = nullptr,
-             size_t ws_bytes = 0);
+             size_t ws_bytes = 0, StepChain chain = StepChain());
 
 // S = X^T Y, k x k column-major FP64 (device)
 int launch_gram(ttdft_ctx ctx, const void *X, int64_t ldx, const void *Y, int64_t ldy,

@@ -9,6 +9,7 @@
 // HBM exactly once per application; the row's (value, column) pairs are read
 // 64 at a time with one coalesced load and broadcast with v_readlane.
 #include "internal.h"
+#include "lds_ring.h"
 
 namespace ttdft {
 namespace {
@@ -400,152 +401,382 @@ __global__ __launch_bounds__(512) void dense_hx_kernel(
     }
 }
 
-// Dense H_loc X with X staged through LDS, in two kernels.
-// dense_hx_part_kernel: workgroup (p, row block, state block) owns 64 rows (a
-// 16-row tile per wave, 4 waves) by 16 JT states over part p of the inner
-// dimension l (nparts parts of whole 32-wide steps, so there are enough
-// workgroups to fill the chip).  Per step the workgroup copies X[l0 .. l0 +
-// 31][its states] into LDS once (coalesced loads of VX consecutive states,
-// pairs in FP32 when aligned), so every X value read from L2 serves four
-// row tiles; each wave loads its 16 rows of H as before
-// (lane (i, q): H[i][l0 + 8q .. 8q + 7]) and MFMA step u pairs l = l0 + 8q + u
-// in both operands, the X operand read from LDS (row 8q + u, 16 consecutive
-// states per quarter-wave; the row pitch of 16 JT + 18 elements puts the
-// quarter-waves' rows 8 apart on distinct banks: 8 pitches are 16 mod 64
-// dwords in FP32, 32 in FP64).  One accumulator per state tile.
-// The next step's X and H loads are issued before this step's products
-// (pinned there by a scheduling barrier, and unconditional so that the wait
-// before the products covers only their LDS reads); the X stage alternates
-// between two buffers with one barrier per step.  The
-// part's sums go to P[p][r][c] in FP64.  Rows past n read row n - 1 (never
-// stored); X rows past n meet zero H padding.
+// Dense H_loc X through a ring of LDS stages, in two or three kernels.
+//
+// What bounds it: H is read once per product and fits no cache, so HBM does
+// (6.1 TB/s for a plain read), beside the matrix cores in FP64 from about 64
+// states on.  dense_ring_kernel therefore keeps two further stages of loads in
+// flight while one is multiplied: workgroup (row block, state block, part)
+// owns ROWS rows (8 waves of 16 in FP64, of 32 in FP32) by 16 JT states over
+// part p of the inner dimension l.  A stage is 32 values of l: 32 KB of H,
+// each wave its own rows, loaded straight into LDS 16 bytes a lane in whole
+// row runs; and the same 32 rows of X, shared by the waves.  One barrier per
+// stage.  The 16-byte chunks of an H row are stored at (chunk ^ row), so that
+// the operand reads of 16 rows spread over the banks.
+//
+// X comes as MFMA fragments (layout below; 1 KB pieces that are loaded and
+// read lane-contiguous), made by x_fragments_kernel or, within a filter, by
+// dense_combine_kernel as it writes the previous product's result.
+//
+// FP64: D[j][i] = sum_l X[l][j] H[i][l] on 16x16x4 FP64 MFMA.
+//
+// FP32: FP32 MFMA has a sixteenth of the BF16 rate and bounded this product
+// (27,000 x 96: 1.33 ms where the read of H takes 0.48).  Every FP32 value is
+// the exact sum of three BF16 values (x0 = bf16(x), x1 = bf16(x - x0),
+// x2 = x - x0 - x1); the products h0 x0, h0 x1, h1 x0, h1 x1, h0 x2, h2 x0
+// on 16x16x32 BF16 MFMA with FP32 accumulation leave out terms below 2^-24 of
+// |h x|, the rounding of one FP32 product.  H stays in FP32 in memory and is
+// split in registers after the LDS read, X once per product.
+//
 // dense_combine_kernel: Y = alpha (sum_p P[p] + C^T W) (+ beta X) (+ delta Z),
-// the parts summed in a fixed order.
-template <typename T, int JT, int VX>
-__global__ __launch_bounds__(256) void dense_hx_part_kernel(int64_t n, int64_t ldh, int32_t k,
-                                                            const T *__restrict__ H,
-                                                            const T *__restrict__ X,
-                                                            int64_t ldx, int32_t nparts,
-                                                            double *__restrict__ P) {
-    typedef typename DenseMma<T>::acc_t acc_t;
-    typedef T xv_t __attribute__((ext_vector_type(VX)));
-    constexpr int NS = 16 * JT;                 // states per workgroup
-    constexpr int XR = NS + 18;                 // LDS row pitch (elements)
-    constexpr int NX = 32 * NS / (256 * VX);    // X vectors per thread per step
-    static_assert(32 * NS % (256 * VX) == 0, "every thread stages the same count");
-    typedef T v4 __attribute__((ext_vector_type(4)));
-    __shared__ __align__(16) T xs[2][32 * XR];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int li = lane & 15, q = lane >> 4;
-    const int64_t i0 = (int64_t)blockIdx.x * 64 + wave * 16;
-    const int c0 = blockIdx.y * NS;
-    const int part = blockIdx.z;
-    const int64_t nst = ldh / 32;
-    const int64_t sb = nst * part / nparts, se = nst * (part + 1) / nparts;
-    const int64_t row = i0 + li < n ? i0 + li : n - 1;
-    const T *hrow = H + row * ldh + 8 * q;
-    // X vector e of this thread: row idx / (NS / VX) of the step, VX
-    // consecutive states from col (the last vector of a ragged k is clamped
-    // inside the row: states past k are never stored, and with VX = 2 k is even)
-    auto xrow = [&](int e) { return (t + 256 * e) / (NS / VX); };
-    auto xcol = [&](int e) { return VX * ((t + 256 * e) % (NS / VX)); };
-    xv_t xv[NX];
-    v4 ha[2], hb[2];
-    auto load_x = [&](int64_t l0) {
-#pragma unroll
-        for (int e = 0; e < NX; ++e) {
-            int64_t l = l0 + xrow(e);
-            l = l < n ? l : n - 1;
-            const int c = c0 + xcol(e) < k ? c0 + xcol(e) : k - VX;
-            xv[e] = *reinterpret_cast<const xv_t *>(X + l * ldx + c);
-        }
-    };
-    auto store_x = [&](int buf) {
-#pragma unroll
-        for (int e = 0; e < NX; ++e)
-            *reinterpret_cast<xv_t *>(&xs[buf][xrow(e) * XR + xcol(e)]) = xv[e];
-    };
-    auto load_h = [&](int64_t l0, v4 (&h)[2]) {
-        h[0] = *reinterpret_cast<const v4 *>(hrow + l0);
-        h[1] = *reinterpret_cast<const v4 *>(hrow + l0 + 4);
-    };
-    // one accumulator per state tile: consecutive products go to different
-    // tiles, so a tile's chain has JT - 1 other products between its steps
-    acc_t acc[JT];
-#pragma unroll
-    for (int jt = 0; jt < JT; ++jt) acc[jt] = acc_t{0, 0, 0, 0};
-    auto mma = [&](int buf, const v4 (&h)[2]) {
-        const T *xb = xs[buf] + 8 * q * XR + li;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const T hu = h[u >> 2][u & 3];
-#pragma unroll
-            for (int jt = 0; jt < JT; ++jt)
-                acc[jt] = DenseMma<T>::step(xb[u * XR + 16 * jt], hu, acc[jt]);
-        }
-    };
-    if (sb < se) {
-        load_x(32 * sb);
-        load_h(32 * sb, hb);
-        store_x(0);
-        // (ha is copied, not loaded, at the loop entry too: the wait the
-        // copy needs then stays here and not before every step's products)
-        ha[0] = hb[0];
-        ha[1] = hb[1];
-        __syncthreads();
-        int buf = 0;
-        for (int64_t st = sb; st < se; ++st) {
-            // the last step reloads its own operands (unconditional loads keep
-            // the wait before the products to this step's LDS reads)
-            const int64_t nx = st + 1 < se ? st + 1 : st;
-            load_x(32 * nx);
-            load_h(32 * nx, hb);
-            // keep the next step's loads ahead of this step's products (the
-            // scheduler would otherwise sink the H loads past them into the
-            // registers the products free, exposing their latency)
-            __builtin_amdgcn_sched_barrier(0);
-            mma(buf, ha);
-            store_x(buf ^ 1);
-            ha[0] = hb[0];
-            ha[1] = hb[1];
-            __syncthreads();
-            buf ^= 1;
-        }
-    }
-    // D[j][i]: element v of lane L holds state DenseMma::state(L/16, v), row L%16
-    const int64_t r = i0 + li;
-    if (r >= n) return;
-    double *Pr = P + ((int64_t)part * n + r) * k;
-#pragma unroll
-    for (int jt = 0; jt < JT; ++jt)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int c = c0 + 16 * jt + DenseMma<T>::state(q, v);
-            if (c < k) Pr[c] = (double)acc[jt][v];
-        }
+// the parts summed in FP64 in a fixed order.
+constexpr int kRingStep = 32;  // values of l per stage
+
+typedef __bf16 bfv8 __attribute__((ext_vector_type(8)));
+typedef unsigned uv4 __attribute__((ext_vector_type(4)));
+
+// Fragments of 32 rows of X and one 16-state tile, lane = state + 16 q:
+//   FP64: four 1 KB pieces u2 of two doubles per lane, X[8 u2 + 2 q + {0, 1}];
+//   FP32: three 1 KB pieces (x0, x1, x2) of eight BF16 per lane, X[8 q + 0..7].
+// Pieces of one tile are consecutive, then tiles, then steps.
+template <typename T> struct RingCfg;
+template <> struct RingCfg<double> {
+    static constexpr int RT = 1;      // 16-row tiles per wave
+    static constexpr int PIECES = 4;  // 1 KB pieces per tile and step
+};
+template <> struct RingCfg<float> {
+    static constexpr int RT = 2;
+    static constexpr int PIECES = 3;
+};
+constexpr int kRingWaves = 8;
+template <typename T> constexpr int ring_rows() { return 16 * kRingWaves * RingCfg<T>::RT; }
+
+// Two FP32 values as sums of three BF16 values each, packed in pairs.
+__device__ __forceinline__ unsigned bf16_pair(float x, float y) {
+    typedef float v2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(v2{x, y}, b2));
+}
+__device__ __forceinline__ void split_bf16(float x, float y, unsigned &a, unsigned &b,
+                                           unsigned &c) {
+    a = bf16_pair(x, y);
+    const float rx = x - __builtin_bit_cast(float, a << 16);
+    const float ry = y - __builtin_bit_cast(float, a & 0xffff0000u);
+    b = bf16_pair(rx, ry);
+    c = bf16_pair(rx - __builtin_bit_cast(float, b << 16),
+                  ry - __builtin_bit_cast(float, b & 0xffff0000u));
 }
 
+// Writes the fragment entries of rows 8 o .. 8 o + 7 of state c.
+__device__ __forceinline__ void store_fragment(const double (&y)[8], int64_t o, int c,
+                                               int32_t ntiles, double *F) {
+    typedef double v2 __attribute__((ext_vector_type(2)));
+    double *f = F + (((o >> 2) * ntiles + (c >> 4)) * 4 + (o & 3)) * 128 + 2 * (c & 15);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) *reinterpret_cast<v2 *>(f + 32 * q) = v2{y[2 * q], y[2 * q + 1]};
+}
+__device__ __forceinline__ void store_fragment(const float (&y)[8], int64_t o, int c,
+                                               int32_t ntiles, float *F) {
+    uv4 a, b, d;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        unsigned p, q, r;
+        split_bf16(y[2 * i], y[2 * i + 1], p, q, r);
+        a[i] = p;
+        b[i] = q;
+        d[i] = r;
+    }
+    // (a piece is 64 lanes x 16 bytes)
+    uv4 *f = reinterpret_cast<uv4 *>(F) + ((o >> 2) * ntiles + (c >> 4)) * 3 * 64 + (c & 15) +
+             16 * (o & 3);
+    f[0] = a;
+    f[64] = b;
+    f[128] = d;
+}
+
+// X to fragments: one thread per eight rows of one state; rows n .. ldh - 1
+// are zero (they meet the zero padding of H), states past k are left as they
+// are (they only reach results that are not stored).
+template <typename T>
+__global__ __launch_bounds__(256) void x_fragments_kernel(int64_t n, int64_t ldh, int32_t k,
+                                                          const T *__restrict__ X, int64_t ldx,
+                                                          int32_t ntiles, T *__restrict__ F) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= ldh / 8 * k) return;
+    const int64_t o = e / k;
+    const int c = (int)(e - o * k);
+    T y[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] = 8 * o + i < n ? X[(8 * o + i) * ldx + c] : T(0);
+    store_fragment(y, o, c, ntiles, F);
+}
+
+// A wave's H operands of one stage in registers
+template <typename T> struct RingH;
+template <> struct RingH<double> {
+    v4f_t raw[4];
+    __device__ __forceinline__ void read(const unsigned char *hb, int wave, int lane) {
+        const int li = lane & 15, q = lane >> 4;
+        // row li of the wave's tile, chunk 4 u2 + q at position (4 u2 + q) ^ li
+        const unsigned a = lds_addr(hb) + (16 * wave + li) * 256 + ((q ^ li) * 16);
+        lds_read4(a, a ^ 64, a ^ 128, a ^ 192, raw[0], raw[1], raw[2], raw[3]);
+    }
+    __device__ __forceinline__ void split(int, int) {}
+};
+template <> struct RingH<float> {
+    v4f_t raw[4];
+    uv4 h0[2], h1[2], h2[2];  // BF16 pieces of rows li, li + 16
+    __device__ __forceinline__ void read(const unsigned char *hb, int wave, int lane) {
+        const int li = lane & 15, q = lane >> 4;
+        // rows li and li + 16 of the wave, chunks 2 q and 2 q + 1 (entries 8 q .. 8 q + 7)
+        const unsigned a = lds_addr(hb) + (32 * wave + li) * 128 + (((2 * q) ^ (li & 7)) * 16);
+        lds_read4(a, a ^ 16, a + 2048, (a ^ 16) + 2048, raw[0], raw[1], raw[2], raw[3]);
+    }
+    // pairs lo .. hi - 1 of the lane's eight
+    __device__ __forceinline__ void split(int lo, int hi) {
+#pragma unroll
+        for (int e = lo; e < hi; ++e) {
+            unsigned a, b, c;
+            split_bf16(raw[e >> 1][2 * (e & 1)], raw[e >> 1][2 * (e & 1) + 1], a, b, c);
+            // (pins the conversion here: it would sink past the stage's barrier)
+            asm volatile("" : "+v"(a), "+v"(b), "+v"(c));
+            h0[e >> 2][e & 3] = a;
+            h1[e >> 2][e & 3] = b;
+            h2[e >> 2][e & 3] = c;
+        }
+    }
+};
+
+// Products of one stage.  While they run, `next` reads (and splits) the H
+// operands of the stage after: all waves leave the stage's barrier together,
+// and would otherwise first queue for LDS, then convert, and only then give
+// the matrix cores work (FP32, 27,000 x 96: 0.79 ms against 0.82 before the
+// vector adds below, 0.84 with them).
+template <int JT>
+__device__ __forceinline__ void ring_products(const RingH<double> &cur, RingH<double> &next,
+                                              const unsigned char *hnext, const unsigned char *xb,
+                                              int wave, int lane, dv4 (&acc)[1][JT]) {
+    typedef double v2 __attribute__((ext_vector_type(2)));
+    const unsigned xa = lds_addr(xb) + lane * 16;
+#pragma unroll
+    for (int jt = 0; jt < JT; ++jt) {
+        v4f_t x[4];
+        const unsigned a = xa + jt * 4096;
+        lds_read4(a, a + 1024, a + 2048, a + 3072, x[0], x[1], x[2], x[3]);
+#pragma unroll
+        for (int u2 = 0; u2 < 4; ++u2) {
+            const v2 hv = __builtin_bit_cast(v2, cur.raw[u2]), xv = __builtin_bit_cast(v2, x[u2]);
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                acc[0][jt] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[u], hv[u], acc[0][jt], 0, 0, 0);
+        }
+    }
+    next.read(hnext, wave, lane);
+}
+
+template <int JT>
+__device__ __forceinline__ void ring_products(const RingH<float> &cur, RingH<float> &next,
+                                              const unsigned char *hnext, const unsigned char *xb,
+                                              int wave, int lane, fv4 (&acc)[2][JT]) {
+    const unsigned xa = lds_addr(xb) + lane * 16;
+    v4f_t xr[2][3];
+    lds_read3<1024, 2048>(xa, xr[0][0], xr[0][1], xr[0][2]);
+    next.read(hnext, wave, lane);
+    // The stage's sums start from zero and are added to the running ones by
+    // vector adds: these round to nearest, where the accumulator of a BF16
+    // product is truncated, a bias that grows with the number of products
+    // (27,000 x 96, degree 20: error 5.9e-5 in place of 1.6e-5, as on FP32 products).
+    fv4 sum[2][2];
+#pragma unroll
+    for (int jt = 0; jt < JT; ++jt) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (jt + 1 < JT) {
+            v4f_t(&x)[3] = xr[(jt + 1) & 1];
+            lds_read3<1024, 2048>(xa + (jt + 1) * 3072, x[0], x[1], x[2]);
+        }
+        const bfv8 x0 = __builtin_bit_cast(bfv8, xr[jt & 1][0]),
+                   x1 = __builtin_bit_cast(bfv8, xr[jt & 1][1]),
+                   x2 = __builtin_bit_cast(bfv8, xr[jt & 1][2]);
+        fv4(&s)[2] = sum[jt & 1];
+        s[0] = s[1] = fv4{0, 0, 0, 0};
+#define RING_MMA(XV, HV)                                                                    \
+    for (int rt = 0; rt < 2; ++rt)                                                          \
+        s[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(                                    \
+            XV, __builtin_bit_cast(bfv8, cur.HV[rt]), s[rt], 0, 0, 0);
+        // smallest terms first
+        RING_MMA(x2, h0)
+        RING_MMA(x0, h2)
+        RING_MMA(x1, h1)
+        RING_MMA(x1, h0)
+        RING_MMA(x0, h1)
+        RING_MMA(x0, h0)
+#undef RING_MMA
+        if (jt > 0)
+            for (int rt = 0; rt < 2; ++rt) acc[rt][jt - 1] += sum[(jt - 1) & 1][rt];
+        next.split(8 * jt / JT, 8 * (jt + 1) / JT);
+        // one product, then three vector instructions of the adds and the
+        // split, in turn
+#pragma unroll
+        for (int i = 0; i < 12; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    for (int rt = 0; rt < 2; ++rt) acc[rt][JT - 1] += sum[(JT - 1) & 1][rt];
+}
+
+template <typename T, int JT>
+__global__ __launch_bounds__(64 * kRingWaves) void dense_ring_kernel(
+    int64_t n, int64_t ldh, int32_t k, const T *__restrict__ H, const T *__restrict__ F,
+    int32_t ntiles, int32_t nparts, T *__restrict__ P) {
+    typedef typename DenseMma<T>::acc_t acc_t;
+    constexpr int RT = RingCfg<T>::RT, ROWB = kRingStep * sizeof(T);
+    constexpr int XB = JT * RingCfg<T>::PIECES * 1024, HB = ring_rows<T>() * ROWB;
+    static_assert(HB == 32768, "each wave loads 4 KB of H per stage");
+    constexpr int STAGE = HB + XB;
+    constexpr int NB = 3 * STAGE <= 160 * 1024 ? 3 : 2;  // stages in LDS
+    constexpr int NQX = (XB / 1024 + kRingWaves - 1) / kRingWaves;
+    constexpr int NQ = 4 + NQX;  // loads per wave per stage (a fixed count)
+    __shared__ __align__(1024) unsigned char ring[NB * STAGE];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t i0 = (int64_t)blockIdx.x * ring_rows<T>();
+    const int part = blockIdx.z;
+    const int64_t nst = ldh / kRingStep;
+    const int64_t sb = nst * part / nparts, se = nst * (part + 1) / nparts;
+    // H: load r of this wave takes 1024 / ROWB rows, one run of ROWB bytes
+    // each; the lane at position p of row i takes chunk p ^ (i mod chunks).
+    // Rows past n load row n - 1 (never stored).
+    constexpr int CPR = ROWB / 16, RPL = 1024 / ROWB;
+    int32_t hoff[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int i = 16 * RT * wave + RPL * r + lane / CPR;
+        const int64_t last = n - 1 - i0;
+        const int64_t ic = i < last ? i : last;
+        hoff[r] = (int32_t)(ic * ldh * (int64_t)sizeof(T)) + 16 * ((lane % CPR) ^ (i % CPR));
+    }
+    const char *hbase = reinterpret_cast<const char *>(H + i0 * ldh);
+    const char *fbase = reinterpret_cast<const char *>(F) + (int64_t)blockIdx.y * XB + lane * 16;
+    const int64_t fstep = (int64_t)ntiles * RingCfg<T>::PIECES * 1024;
+    // stage st to LDS place b; past the last stage: that one again (every
+    // wave issues NQ loads a stage)
+    auto place = [&](int b) { return ring + b * STAGE; };
+    auto fetch_h = [&](int64_t st, int b) {
+        unsigned char *d = place(b) + wave * 4096;
+        const char *src = hbase + (st < se ? st : se - 1) * ROWB;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) load_lds_16(src + hoff[r], d + 1024 * r);
+    };
+    auto fetch_x = [&](int64_t st, int b) {
+        unsigned char *d = place(b) + HB;
+        const char *src = fbase + (st < se ? st : se - 1) * fstep;
+#pragma unroll
+        for (int i = 0; i < NQX; ++i) {
+            int c = wave + kRingWaves * i;
+            c = c < XB / 1024 ? c : XB / 1024 - 1;  // past the last piece: that one again
+            load_lds_16(src + 1024 * c, d + 1024 * c);
+        }
+    };
+    acc_t acc[RT][JT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int jt = 0; jt < JT; ++jt) acc[rt][jt] = acc_t{0, 0, 0, 0};
+    RingH<T> h[2];
+    fetch_h(sb, 0);
+#pragma unroll
+    for (int s = 0; s < NB - 1; ++s) {
+        fetch_x(sb + s, s);
+        fetch_h(sb + s + 1, s + 1);
+    }
+    TT_WAIT_VM_LDS((NB - 1) * NQ);  // H of the first stage, this wave's own rows
+    h[0].read(place(0), wave, lane);
+    h[0].split(0, 8);
+    int b = 0;  // place of stage st
+    auto step = [&](int64_t st, const RingH<T> &cur, RingH<T> &next) {
+        // X of stage st and this wave's H of stage st + 1 are complete when at
+        // most the loads of NB - 2 further stages are outstanding; behind the
+        // barrier every wave's X is, and every wave has read X of stage
+        // st - 1, whose place the next loads take (H of stage st was read
+        // during stage st - 1, by the wave that loaded it)
+        TT_WAIT_VM_LDS((NB - 2) * NQ);
+        line_barrier();
+        fetch_x(st + NB - 1, b == 0 ? NB - 1 : b - 1);
+        fetch_h(st + NB, b);
+        const int bn = b + 1 == NB ? 0 : b + 1;
+        ring_products<JT>(cur, next, place(bn), place(b) + HB, wave, lane, acc);
+        b = bn;
+    };
+    for (int64_t st = sb; st < se; st += 2) {
+        step(st, h[0], h[1]);
+        if (st + 1 >= se) break;
+        step(st + 1, h[1], h[0]);
+    }
+    TT_WAIT_ALL();  // no load into LDS may outlive the workgroup
+    const int li = lane & 15, q = lane >> 4;
+    const int c0 = blockIdx.y * 16 * JT;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int64_t r = i0 + 16 * (RT * wave + rt) + li;
+        if (r >= n) continue;
+        T *Pr = P + ((int64_t)part * n + r) * k;
+#pragma unroll
+        for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int c = c0 + 16 * jt + DenseMma<T>::state(q, v);
+                if (c < k) Pr[c] = acc[rt][jt][v];
+            }
+    }
+}
+
+// One thread per eight rows of one state (the rows of a fragment entry)
 template <typename T>
 __global__ __launch_bounds__(256) void dense_combine_kernel(
-    int64_t n, int32_t k, int32_t nparts, const double *__restrict__ P, const T *X, int64_t ldx,
-    const int64_t *__restrict__ ct_rowptr, const int32_t *__restrict__ ct_col,
+    int64_t n, int64_t ldh, int32_t k, int32_t nparts, const T *__restrict__ P, const T *X,
+    int64_t ldx, const int64_t *__restrict__ ct_rowptr, const int32_t *__restrict__ ct_col,
     const T *__restrict__ ct_val, const T *__restrict__ W, T *Y, int64_t ldy, const T *Z,
-    int64_t ldz, double alpha, double beta, double delta, int use_beta, int use_delta) {
-    const int64_t total = n * k;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t r = e / k;
-        const int c = (int)(e - r * k);
-        double s = P[e];
-        for (int p = 1; p < nparts; ++p) s += P[(int64_t)p * total + e];
+    int64_t ldz, double alpha, double beta, double delta, int use_beta, int use_delta,
+    int32_t ntiles, T *__restrict__ F) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= ldh / 8 * k) return;
+    const int64_t o = e / k, total = n * k;
+    const int c = (int)(e - o * k);
+    T yv[8];
+    double s[8], xb[8], zb[8];
+    // (all loads of the eight rows before the first result is stored)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int64_t r = 8 * o + i < n ? 8 * o + i : n - 1;
+        s[i] = (double)P[r * k + c];
+        xb[i] = use_beta ? (double)X[r * ldx + c] : 0.0;
+        zb[i] = use_delta ? (double)Z[r * ldz + c] : 0.0;
+    }
+    for (int p = 1; p < nparts; ++p)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int64_t r = 8 * o + i < n ? 8 * o + i : n - 1;
+            s[i] += (double)P[(int64_t)p * total + r * k + c];
+        }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int64_t r = 8 * o + i;
+        if (r >= n) {
+            yv[i] = T(0);
+            continue;
+        }
         if (ct_rowptr)
             for (int64_t f = ct_rowptr[r]; f < ct_rowptr[r + 1]; ++f)
-                s += (double)ct_val[f] * (double)W[(int64_t)ct_col[f] * k + c];
-        double y = s * alpha;
-        if (use_beta) y += beta * (double)X[r * ldx + c];
-        if (use_delta) y += delta * (double)Z[r * ldz + c];
-        Y[r * ldy + c] = (T)y;
+                s[i] += (double)ct_val[f] * (double)W[(int64_t)ct_col[f] * k + c];
+        double y = s[i] * alpha;
+        if (use_beta) y += beta * xb[i];
+        if (use_delta) y += delta * zb[i];
+        yv[i] = (T)y;
+        Y[r * ldy + c] = yv[i];
     }
+    if (F) store_fragment(yv, o, c, ntiles, F);
 }
 
 __global__ __launch_bounds__(256) void dense_to_f32_kernel(const double *__restrict__ s,
@@ -670,12 +901,14 @@ void drop_dense(ttdft_ham_s *H) {
 // the block's k states on one wavefront, while a matrix product streams the
 // n^2 values once at full bandwidth.
 constexpr double kDenseMaxBytes = 48.0 * 1024 * 1024 * 1024;
+bool dense_storage_fits(int64_t n, int64_t nnz) {
+    return n >= 1 && 8.0 * (double)n * (double)n <= kDenseMaxBytes &&
+           (double)nnz >= 0.2 * (double)n * (double)n;
+}
 int maybe_build_dense(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
     (void)copies;
     const int64_t n = H->n;
-    if (H->format != 0 || n < 1 || 8.0 * (double)n * (double)n > kDenseMaxBytes ||
-        (double)H->nnz < 0.2 * (double)n * n)
-        return TTDFT_OK;
+    if (H->format != 0 || !dense_storage_fits(n, H->nnz)) return TTDFT_OK;
     // rows padded to 16 and the leading dimension to 32 (the product's tiles)
     const int64_t ld = (n + 31) / 32 * 32;
     const size_t n2 = (size_t)((n + 15) / 16 * 16) * (size_t)ld;
@@ -759,63 +992,86 @@ int finish_dense(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
     return TTDFT_OK;
 }
 
-constexpr int kDenseParts = 4;  // most parts of l in the split dense product
+constexpr int kDenseParts = 16;  // most parts of l in the split dense product
 
 // 0: one-kernel dense product; 1: split product, parts picked; 2..4: split
 // product with that many parts
-int dense_split_form(int dtype) {
-    (void)dtype;  // both precisions take the split product by default
+static int dense_split_form() {
     const char *env = std::getenv("TTDFT_DENSE_LDS");
     return env ? std::atoi(env) : 1;
+}
+
+// Tiling of the dense product of k states: fewest columns of at most 96
+// states, then the fewest 16-state tiles that cover k in that many columns
+// (each column streams H once).
+struct DenseTiling {
+    int ncol, jt, nparts;
+    size_t partial_bytes, bytes;  // partial sums; with the fragments of X behind them
+};
+static DenseTiling dense_tiling(const ttdft_ham_s *H, int32_t k, int dtype) {
+    DenseTiling d;
+    d.ncol = (k + 95) / 96;
+    d.jt = (k + 16 * d.ncol - 1) / (16 * d.ncol);
+    const int rows = dtype == TTDFT_F64 ? ring_rows<double>() : ring_rows<float>();
+    const int64_t nst = H->dense_ld / kRingStep, wgs = (H->n + rows - 1) / rows * d.ncol;
+    // Parts of l: one workgroup fills a CU (its LDS stages), so parts p take
+    // ceil(wgs p / 256) rounds of nst / p stages and about four to fill and
+    // drain the ring; a part's sums cost n k / (64 rows) stages of the chip's
+    // bandwidth (written and read back).  The cheapest count is taken.
+    double best = 0.0;
+    d.nparts = 1;
+    for (int p = 1; p <= kDenseParts && p <= nst; ++p) {
+        const double cost = (double)((wgs * p + 255) / 256) * (double)((nst + p - 1) / p + 4) +
+                            p * (double)H->n * k / (256.0 * 16 * rows);
+        if (p == 1 || cost < best) {
+            best = cost;
+            d.nparts = p;
+        }
+    }
+    const int form = dense_split_form();
+    if (form > 1) d.nparts = (int)std::min<int64_t>(std::min(form, kDenseParts), nst);
+    const size_t es = dtype_size(dtype);
+    d.partial_bytes = ((size_t)d.nparts * H->n * k * es + 255) / 256 * 256;
+    d.bytes = d.partial_bytes + (size_t)nst * d.ncol * d.jt * 1024 *
+                                    (dtype == TTDFT_F64 ? RingCfg<double>::PIECES
+                                                        : RingCfg<float>::PIECES);
+    return d;
 }
 
 template <typename T, int JT>
 static void dense_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const T *Hd, const T *ctv,
                          const void *X, int64_t ldx, const void *W, void *Y, int64_t ldy,
                          const void *Z, int64_t ldz, int32_t k, double alpha, double beta,
-                         double delta, int use_beta, int use_delta, double *P) {
+                         double delta, int use_beta, int use_delta, void *P, StepChain chain) {
     const int64_t n = H->n;
     const dim3 grid((unsigned)((n + 15) / 16), (unsigned)((k + 16 * JT - 1) / (16 * JT)));
     const int64_t *ctr = H->p > 0 && !H->dense_nl ? H->ct_rowptr : nullptr;
+    // Split product against the one-kernel form, which stays for callers whose
+    // work space cannot hold the partial sums: FP32 27,000 x 96 0.84 + 0.03
+    // (sum of the parts) against 2.54 ms, FP64 8,000 x 24 0.108 + 0.007 against
+    // 0.153.  TTDFT_DENSE_LDS=0 turns the split off, 1 picks the parts, 2..4
+    // fixes them.
+    if (P) {
+        const DenseTiling d = dense_tiling(H, k, sizeof(T) == 8 ? TTDFT_F64 : TTDFT_F32);
+        const int ntiles = d.ncol * JT;
+        T *Pt = (T *)P, *F = (T *)((char *)P + d.partial_bytes);
+        const unsigned cb = (unsigned)((H->dense_ld / 8 * k + 255) / 256);
+        if (!chain.have)
+            hipLaunchKernelGGL((x_fragments_kernel<T>), dim3(cb), dim3(256), 0, ctx->stream, n,
+                               H->dense_ld, k, (const T *)X, ldx, ntiles, F);
+        const dim3 g((unsigned)((n + ring_rows<T>() - 1) / ring_rows<T>()), (unsigned)d.ncol,
+                     (unsigned)d.nparts);
+        hipLaunchKernelGGL((dense_ring_kernel<T, JT>), g, dim3(64 * kRingWaves), 0,
+                           ctx->stream, n, H->dense_ld, k, Hd, F, ntiles, d.nparts, Pt);
+        hipLaunchKernelGGL((dense_combine_kernel<T>), dim3(cb), dim3(256), 0, ctx->stream, n,
+                           H->dense_ld, k, d.nparts, Pt, (const T *)X, ldx, ctr, H->ct_col, ctv,
+                           (const T *)W, (T *)Y, ldy, (const T *)Z, ldz, alpha, beta, delta,
+                           use_beta, use_delta, ntiles, chain.want ? F : nullptr);
+        return;
+    }
     // six-state runs per lane, fetched as pairs, when every tile is full and
     // every row of X starts on a pair boundary (even leading dimension and a
     // pair-aligned X: a filter block may start at an odd column)
-    // The split product with X staged in LDS, against the one-kernel form:
-    // FP32 27,000 x 96 1.39 against 2.54 ms, 27,000 x 48 0.74 against 1.26,
-    // 8,000 x 24 0.077 against 0.089; FP64 27,000 x 96 3.02 against 3.26,
-    // 27,000 x 48 1.58 against 2.14, 8,000 x 24 0.133 against 0.153.
-    // TTDFT_DENSE_LDS=0 turns the split off, 1 picks the parts, 2..4 fixes
-    // them.
-    const int lds_form = dense_split_form(sizeof(T) == 8 ? TTDFT_F64 : TTDFT_F32);
-    if (lds_form >= 1 && P) {
-        // parts of l for about 4.5 workgroups per CU, 6 for FP64 at 80-96
-        // states (measured best at 27,000: FP64 x 96 3.17 ms at four parts,
-        // 3.33 at three; FP64 x 48 1.62 ms at three, 1.74 at four)
-        const int64_t wgs = (n + 63) / 64 * grid.y;
-        const int64_t target = sizeof(T) == 8 && JT >= 5 ? 1536 : 1152;
-        int nparts = (int)((target + wgs - 1) / wgs);
-        if (lds_form > 1) nparts = lds_form;
-        const int64_t nst = H->dense_ld / 32;
-        if (nparts > nst) nparts = (int)nst;
-        if (nparts > kDenseParts) nparts = kDenseParts;
-        const dim3 g((unsigned)((n + 63) / 64), grid.y, (unsigned)nparts);
-        // X staged in pairs when every pair is aligned and whole
-        const bool pairs = k % 2 == 0 && ldx % 2 == 0 &&
-                           reinterpret_cast<uintptr_t>(X) % (2 * sizeof(T)) == 0;
-        if (pairs)
-            hipLaunchKernelGGL((dense_hx_part_kernel<T, JT, 2>), g, dim3(256), 0, ctx->stream,
-                               n, H->dense_ld, k, Hd, (const T *)X, ldx, nparts, P);
-        else
-            hipLaunchKernelGGL((dense_hx_part_kernel<T, JT, 1>), g, dim3(256), 0, ctx->stream,
-                               n, H->dense_ld, k, Hd, (const T *)X, ldx, nparts, P);
-        const int64_t total = n * k;
-        const unsigned cb = (unsigned)std::min<int64_t>((total + 255) / 256, 65536);
-        hipLaunchKernelGGL((dense_combine_kernel<T>), dim3(cb), dim3(256), 0, ctx->stream, n, k,
-                           nparts, P, (const T *)X, ldx, ctr, H->ct_col, ctv, (const T *)W,
-                           (T *)Y, ldy, (const T *)Z, ldz, alpha, beta, delta, use_beta,
-                           use_delta);
-        return;
-    }
     if (JT == 6 && k % (16 * JT) == 0 && ldx % 2 == 0 &&
         reinterpret_cast<uintptr_t>(X) % (2 * sizeof(T)) == 0)
         hipLaunchKernelGGL((dense_hx_kernel<T, JT, (JT == 6)>), grid, dim3(64 * kDenseWaves), 0,
@@ -834,19 +1090,16 @@ static void dense_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const T *Hd, const
 static int launch_dense_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx,
                              const void *W, void *Y, int64_t ldy, const void *Z, int64_t ldz,
                              int32_t k, int dtype, double alpha, double beta, double delta,
-                             int use_beta, int use_delta, double *P) {
-    // fewest workgroup columns of at most 96 states, then the fewest 16-state
-    // tiles that cover k in that many columns (each column streams H once)
-    const int ncol = (k + 95) / 96;
-    const int jt = (k + 16 * ncol - 1) / (16 * ncol);
+                             int use_beta, int use_delta, void *P, StepChain chain) {
+    const int jt = dense_tiling(H, k, dtype).jt;
 #define DENSE_CASE(JTV)                                                                         \
     case JTV:                                                                                   \
         if (dtype == TTDFT_F64)                                                                 \
             dense_launch<double, JTV>(ctx, H, H->dense64, H->ct_val64, X, ldx, W, Y, ldy, Z,    \
-                                      ldz, k, alpha, beta, delta, use_beta, use_delta, P);      \
+                                      ldz, k, alpha, beta, delta, use_beta, use_delta, P, chain);      \
         else                                                                                    \
             dense_launch<float, JTV>(ctx, H, H->dense32, H->ct_val32, X, ldx, W, Y, ldy, Z,     \
-                                     ldz, k, alpha, beta, delta, use_beta, use_delta, P);       \
+                                     ldz, k, alpha, beta, delta, use_beta, use_delta, P, chain);       \
         break;
     switch (jt) {
         DENSE_CASE(1)
@@ -866,7 +1119,7 @@ static int launch_dense_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X,
 int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, void *Y,
              int64_t ldy, const void *Z, int64_t ldz, int32_t k, int dtype, double alpha,
              double beta, double delta, int use_beta, int use_delta, void *ws,
-             size_t ws_bytes) {
+             size_t ws_bytes, StepChain chain) {
     const size_t es = dtype_size(dtype);
     const bool band = H->format == 1 && k >= 16 &&
                       (dtype == TTDFT_F64 ? H->mf64 != nullptr : H->mf32 != nullptr);
@@ -897,23 +1150,24 @@ int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, vo
         TT_TRY(launch_band_spmm(ctx, H, X, ldx, W, Y, ldy, Z ? Z : Y, Z ? ldz : ldy, k, dtype,
                                 alpha, beta, delta, use_beta, use_delta));
     else if (dense) {
-        // partial sums of the split product: after the projections in the
-        // caller's work space, else from the context.  When the caller's work
-        // space cannot hold them the product runs in one kernel (no partial
-        // sums; the same result up to the order of the additions).
-        double *P = nullptr;
-        if (dense_split_form(dtype) >= 1) {
-            const size_t need_p = (size_t)kDenseParts * H->n * k * sizeof(double);
+        // partial sums and fragments of the split product: after the
+        // projections in the caller's work space, else from the context.  When
+        // the caller's work space cannot hold them the product runs in one
+        // kernel (no partial sums; the same result up to the order of the
+        // additions).
+        void *P = nullptr;
+        if (dense_split_form() >= 1) {
+            const size_t need_p = dense_tiling(H, k, dtype).bytes;
             if (ws) {
                 const size_t off = W ? ((size_t)nl_workspace(H, k) * es + 255) / 256 * 256 : 0;
-                if (off + need_p <= ws_bytes) P = (double *)((char *)ws + off);
+                if (off + need_p <= ws_bytes) P = (char *)ws + off;
             } else {
                 TT_TRY(ctx->scratch[8].ensure(need_p));
-                P = (double *)ctx->scratch[8].ptr;
+                P = ctx->scratch[8].ptr;
             }
         }
         TT_TRY(launch_dense_spmm(ctx, H, X, ldx, W, Y, ldy, Z ? Z : Y, Z ? ldz : ldy, k, dtype,
-                                 alpha, beta, delta, use_beta, use_delta, P));
+                                 alpha, beta, delta, use_beta, use_delta, P, chain));
     }
     else
         TT_TRY(launch_spmm_fused(ctx, H, X, ldx, W, Y, ldy, Z ? Z : Y, Z ? ldz : ldy, k, dtype,
