@@ -401,6 +401,33 @@ def test_orth_matches_oracle_f64(ctx, k):
     assert rel(dX.to_host(), oracle.orth(X)) < 1e-11
 
 
+@pytest.mark.parametrize("k", [1, 31, 32, 33, 63, 65, 96, 97, 300, 513])
+def test_orth_block_columns_of_the_factorisation(ctx, k):
+    """Cholesky inverse by 32 columns a launch: one block, remainders of 1 and
+    31, many blocks, against numpy on a block of condition about 20 (squared
+    in the overlap: 400 eps, times the growth of sums over k)."""
+    n = k + 700
+    rng = np.random.default_rng(k)
+    X = rng.standard_normal((n, k)) * np.linspace(1.0, 0.1, k)
+    dX = dev(ctx, X)
+    ctx.orth(dX.ptr, k, n, k)
+    L = np.linalg.cholesky(X.T @ X)
+    assert rel(dX.to_host(), np.linalg.solve(L, X.T).T) < 1e-12
+
+
+@pytest.mark.parametrize("k,col", [(8, 5), (80, 0), (80, 31), (80, 32), (80, 79), (300, 290)])
+def test_orth_not_spd_in_any_block(ctx, k, col):
+    """A zero column gives an exactly zero pivot in whichever launch meets it;
+    X is left as it was."""
+    X = np.random.default_rng(2).standard_normal((600, k))
+    X[:, col] = 0.0
+    dX = dev(ctx, X)
+    with pytest.raises(E.TtdftError) as ei:
+        ctx.orth(dX.ptr, k, 600, k)
+    assert ei.value.status == E.ENOTSPD and f"minor {col + 1}" in str(ei.value)
+    assert np.array_equal(dX.to_host(), X)
+
+
 def test_orth_not_spd_reports_error(ctx):
     n, k = 300, 8
     X = np.random.default_rng(2).standard_normal((n, k))

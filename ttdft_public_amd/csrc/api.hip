@@ -34,7 +34,6 @@ int launch_cm_to_bm(ttdft_ctx ctx, const double *src, int64_t lda, int64_t n, in
                     void *dst, int64_t ldd, int dtype);
 int launch_bm_to_cm(ttdft_ctx ctx, const void *src, int64_t lds, int dtype, int64_t n,
                     int32_t k, double *dst, int64_t lda);
-int launch_lower_transpose(ttdft_ctx ctx, const double *L, double *LT, int32_t k);
 
 // ---- errors ----------------------------------------------------------------
 static thread_local std::string g_err;
@@ -388,34 +387,17 @@ void ctx_detach(ttdft_ctx ctx) {
 static int orth_once(ttdft_ctx ctx, void *X, int64_t ldx, int64_t n, int32_t k, int dtype,
                      int mode) {
     const int64_t kk = (int64_t)k * k;
-    TT_TRY(ctx->scratch[1].ensure((size_t)kk * 2 * sizeof(double)));
+    TT_TRY(ctx->scratch[1].ensure((size_t)kk * 3 * sizeof(double)));
     double *S = (double *)ctx->scratch[1].ptr;
     double *QT = S + kk;
     TT_TRY(launch_gram(ctx, X, ldx, X, ldx, n, k, dtype, mode, S));
-    if (small_dense_enabled(k)) {
-        TT_TRY(small_chol_inv(ctx, S, k, QT));
-        const size_t es = dtype_size(dtype);
-        TT_TRY(ctx->scratch[0].ensure((size_t)n * k * es));
-        void *Z = ctx->scratch[0].ptr;
-        TT_TRY(launch_rotate(ctx, X, ldx, Z, k, n, k, QT, dtype, mode));
-        TT_TRY(launch_copy_block(ctx, Z, k, dtype, X, ldx, dtype, n, k));
-        return TTDFT_OK;
-    }
-    rocblas_status st = rocsolver_dpotrf(ctx->blas, rocblas_fill_lower, k, S, k, ctx->d_info);
-    TT_CHECK(st == rocblas_status_success, TTDFT_ELIB, "rocsolver_dpotrf: status %d", (int)st);
-    int info = 0;
-    TT_HIP(hipMemcpyAsync(&info, ctx->d_info, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    TT_HIP(hipStreamSynchronize(ctx->stream));
-    TT_CHECK(info == 0, TTDFT_ENOTSPD, "overlap matrix not positive definite (minor %d)", info);
-    st = rocsolver_dtrtri(ctx->blas, rocblas_fill_lower, rocblas_diagonal_non_unit, k, S, k,
-                          ctx->d_info);
-    TT_CHECK(st == rocblas_status_success, TTDFT_ELIB, "rocsolver_dtrtri: status %d", (int)st);
-    // Q = L^{-T} (column-major, strictly lower part of L^{-T} zero)
-    TT_TRY(launch_lower_transpose(ctx, S, QT, k));
+    TT_TRY(chol_inv(ctx, S, QT + kk, k, QT));
     const size_t es = dtype_size(dtype);
     TT_TRY(ctx->scratch[0].ensure((size_t)n * k * es));
     void *Z = ctx->scratch[0].ptr;
+    // (X stays as it was until the factorisation is known to have succeeded)
     TT_TRY(launch_rotate(ctx, X, ldx, Z, k, n, k, QT, dtype, mode));
+    TT_TRY(chol_check(ctx));
     TT_TRY(launch_copy_block(ctx, Z, k, dtype, X, ldx, dtype, n, k));
     return TTDFT_OK;
 }

@@ -174,9 +174,13 @@ int build_band_device(ttdft_ctx ctx, ttdft_ham_s *H, int32_t rx, int32_t ry, int
                       int by, int bz, int copies);
 // Y = alpha*(H_loc X + C^T W) + beta*X + delta*Z   (Z may alias Y; flags select terms)
 // use_beta / use_delta select whether X / Z are read.
-// One-workgroup k x k factorisations for k <= 64 (small_dense.hip)
+// Q = L^{-T} (column-major, zero below the diagonal) of S = L L^T; S (lower
+// triangle read) and the k x k work are overwritten.  chol_check waits for it
+// and reports a matrix that is not positive definite; Q is then undefined.
+int chol_inv(ttdft_ctx ctx, double *S, double *work, int32_t k, double *Q);
+int chol_check(ttdft_ctx ctx);
+// One-workgroup eigensolve for k <= 64 (small_dense.hip)
 bool small_dense_enabled(int32_t k);
-int small_chol_inv(ttdft_ctx ctx, const double *S, int32_t k, double *QT);
 int small_syev(ttdft_ctx ctx, const double *A, int32_t k, double *evals, double *Q);
 // Orthonormal basis of an n x b column-major block in place (n b <= 18432, b <= 64)
 bool small_orth_fits(int32_t n, int32_t b);

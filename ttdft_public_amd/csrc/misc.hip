@@ -158,15 +158,6 @@ __global__ __launch_bounds__(256) void bm_to_cm_kernel(const S *__restrict__ src
     }
 }
 
-// LT = L^T for a lower-triangular L (entries above the diagonal of L ignored)
-__global__ void lower_transpose_kernel(const double *__restrict__ L, double *__restrict__ LT,
-                                       int32_t k) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)k * k) return;
-    const int a = (int)(idx % k), b = (int)(idx / k);
-    LT[a + (int64_t)k * b] = (b >= a) ? L[b + (int64_t)k * a] : 0.0;
-}
-
 }  // namespace
 
 int launch_initial_density(ttdft_ctx ctx, int32_t natoms, const double *d_xyz, int32_t nr,
@@ -278,14 +269,6 @@ int launch_bm_to_cm(ttdft_ctx ctx, const void *src, int64_t lds, int dtype, int6
     else
         hipLaunchKernelGGL((bm_to_cm_kernel<float>), grid, dim3(256), 0, ctx->stream,
                            (const float *)src, lds, n, k, dst, lda);
-    TT_LAUNCH_CHECK();
-    return TTDFT_OK;
-}
-
-int launch_lower_transpose(ttdft_ctx ctx, const double *L, double *LT, int32_t k) {
-    const int64_t kk = (int64_t)k * k;
-    hipLaunchKernelGGL(lower_transpose_kernel, dim3((unsigned)((kk + 255) / 256)), dim3(256), 0,
-                       ctx->stream, L, LT, k);
     TT_LAUNCH_CHECK();
     return TTDFT_OK;
 }

@@ -1,10 +1,9 @@
-// Dense k x k factorisations of the subspace iteration for small blocks
-// (k <= 64), each in one workgroup with the matrix held in LDS: the
-// Cholesky factor's inverse for Cholesky-QR (MultTm.cu:256-419, the
-// SOLVE_WITH_INVERSE variant) and the symmetric eigensolve of Rayleigh-Ritz
-// (EigenSolver.cc:30-184).  At these sizes the library routines spend their
-// time in launch latency (hundreds of small kernels per call); one launch
-// does the whole factorisation here.
+// Dense k x k factorisations of the subspace iteration: the Cholesky factor's
+// inverse for Cholesky-QR (MultTm.cu:256-419, the SOLVE_WITH_INVERSE variant)
+// for any k, and for small blocks (k <= 64) the symmetric eigensolve of
+// Rayleigh-Ritz (EigenSolver.cc:30-184) in one workgroup with the matrix held
+// in LDS.  At these sizes the library routines spend their time in launch
+// latency (tens to hundreds of small kernels per call).
 //
 // Matrices are column-major k x k, FP64.
 #include <cmath>
@@ -17,63 +16,181 @@ namespace {
 constexpr int kMax = 64;
 constexpr int kLd = kMax + 1;
 
-// QT = L^{-T} with S = L L^T (lower Cholesky of the symmetric S; only its
-// lower triangle is read); QT's strictly lower part is zero.  info = j + 1
-// when the leading minor of order j + 1 is not positive definite.
-__global__ __launch_bounds__(256) void small_chol_inv_kernel(const double *__restrict__ S, int k,
-                                                             double *__restrict__ QT,
-                                                             int *__restrict__ info) {
-    __shared__ double A[kMax * kLd];
-    __shared__ double Li[kMax * kLd];
-    __shared__ int bad;
-    const int t = threadIdx.x;
-    for (int e = t; e < k * k; e += 256) {
-        const int i = e % k, j = e / k;
-        A[i + kLd * j] = i >= j ? S[i + (int64_t)k * j] : 0.0;
-    }
-    if (t == 0) bad = 0;
+// Q = L^{-T} with S = L L^T, by blocks of 32 columns, one launch per block.
+//
+// What bounds it: latency.  At k = 300 the arithmetic is 0.02 GFLOP, and the
+// library's factorisation and triangular inverse took 0.76 + 0.25 ms in some
+// thirty launches.  Launch j eliminates block column j from the trailing
+// matrix and, at the same time, from the identity beside it (which becomes
+// L^{-1}): every workgroup owns one 32 x 32 tile, factorises the diagonal
+// block again for itself (32 pivots with one barrier each, 5 us) and
+// recomputes the one or two panel blocks its tile needs, so that tiles of a
+// launch depend only on the launch before.  k = 300: CHOL_MS.
+//
+//   T1  tile (i, l), j < l <= i:  S_il -= L_ij L_lj^T
+//   T2  tile (i, c), c <= j < i:  B_ic -= L_ij (Linv_jj B_jc)
+//   T3  tile (j, c), c <= j:      L^{-1}_jc = Linv_jj B_jc, stored transposed
+//       in Q, and zeros in Q's block below the diagonal
+// with L_ij = S_ij Linv_jj^T; B_jj = I and B_ij = 0 are implied.  Only S's
+// lower triangle is read; S is overwritten.
+constexpr int kNb = 32, kNbLd = kNb + 1;
+typedef double sd4 __attribute__((ext_vector_type(4)));
+
+// 32 x 32 x 32 product of LDS blocks, P Q^T: wave w's 16 x 16 tile (w / 2, w % 2);
+// element v of lane l is row l / 16 + 4 v, column l % 16 of the tile
+__device__ __forceinline__ sd4 block_pqt(const double *P, const double *Q, int wave, int lane) {
+    const double *p = P + (16 * (wave >> 1) + (lane & 15)) * kNbLd + (lane >> 4);
+    const double *q = Q + (16 * (wave & 1) + (lane & 15)) * kNbLd + (lane >> 4);
+    sd4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < kNb / 4; ++s)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(p[4 * s], q[4 * s], acc, 0, 0, 0);
+    return acc;
+}
+
+__global__ __launch_bounds__(256) void chol_inv_step_kernel(double *__restrict__ S,
+                                                            double *__restrict__ B,
+                                                            double *__restrict__ Q, int k, int j,
+                                                            int *__restrict__ info) {
+    __shared__ double Li[kNb * kNbLd];              // Linv_jj, row-major
+    __shared__ double pa[kNb * kNbLd], pb[kNb * kNbLd], pc[kNb * kNbLd];
+    __shared__ double rowb[2][2 * kNb], colb[2][kNb], piv[kNb];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    // An earlier launch found the matrix not positive definite (launch 0
+    // writes the word itself).  One thread reads it for all: workgroup 0 may
+    // write it meanwhile.
+    __shared__ int stop;
+    if (t == 0) stop = j > 0 ? *info : 0;
     __syncthreads();
-    // right-looking Cholesky, column j per step
-    for (int j = 0; j < k; ++j) {
-        const double d = A[j + kLd * j];
-        if (!(d > 0.0)) {  // uniform across the workgroup
-            if (t == 0) bad = j + 1;
-            break;
+    if (stop != 0) return;
+    const int64_t ld = k;
+    const int nb = (k + kNb - 1) / kNb, j0 = kNb * j;
+
+    // The diagonal block (identity past k) beside the identity: thread (row i,
+    // group g) keeps columns 8 g .. 8 g + 7 of the 64.  Step c subtracts
+    // multiples of row c from the rows below it; the next pivot row and column
+    // go through LDS, two buffers in turn.
+    const int i = t >> 3, g = t & 7;
+    double v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int c = 8 * (g & 3) + e;
+        if (g < 4) {
+            const int r = i > c ? i : c, cc = i > c ? c : i;
+            v[e] = j0 + r < k ? S[j0 + r + ld * (j0 + cc)] : (r == cc ? 1.0 : 0.0);
+        } else {
+            v[e] = i == c ? 1.0 : 0.0;
         }
-        const double ljj = sqrt(d);
-        __syncthreads();
-        if (t == 0) A[j + kLd * j] = ljj;
-        for (int i = j + 1 + t; i < k; i += 256) A[i + kLd * j] /= ljj;
-        __syncthreads();
-        // trailing update of the lower triangle: A[i][l] -= L[i][j] L[l][j], j < l <= i
-        const int m = k - j - 1;
-        for (int e = t; e < m * m; e += 256) {
-            const int i = j + 1 + e % m, l = j + 1 + e / m;
-            if (l <= i) A[i + kLd * l] -= A[i + kLd * j] * A[l + kLd * j];
-        }
-        __syncthreads();
     }
+    if (i == 0)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) rowb[0][8 * g + e] = v[e];
+    if (g == 0) colb[0][i] = v[0];
     __syncthreads();
-    if (bad) {
-        if (t == 0) *info = bad;
+    int bad = 0;
+    for (int co = 0; co < 4 && !bad; ++co)
+#pragma unroll
+        for (int ce = 0; ce < 8; ++ce) {
+            const int c = 8 * co + ce, p = c & 1;
+            const double d = colb[p][c];
+            if (!(d > 0.0)) {  // the same value for every thread
+                bad = c + 1;
+                break;
+            }
+            if (t == 0) piv[c] = d;
+            if (i > c) {
+                const double f = colb[p][i] / d;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] -= f * rowb[p][8 * g + e];
+            }
+            if (i == c + 1)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) rowb[p ^ 1][8 * g + e] = v[e];
+            if (g == (ce == 7 ? co + 1 : co)) colb[p ^ 1][i] = v[(ce + 1) & 7];
+            __syncthreads();
+        }
+    if (bad || j == 0) {
+        if (blockIdx.x == 0 && t == 0) *info = bad ? j0 + bad : 0;
+        if (bad) return;
+    }
+    if (g >= 4) {
+        const double r = 1.0 / sqrt(piv[i]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) Li[i * kNbLd + 8 * (g - 4) + e] = v[e] * r;
+    }
+
+    // this workgroup's tile
+    const int m = nb - 1 - j;
+    int w = blockIdx.x, kind, bi, bl;  // kind 1..3, block row, second block index
+    if (w < m * (m + 1) / 2) {
+        kind = 1;
+        int r = 0;
+        while (w > r) w -= ++r;
+        bi = j + 1 + r;
+        bl = j + 1 + w;
+    } else if ((w -= m * (m + 1) / 2) < m * (j + 1)) {
+        kind = 2;
+        bi = j + 1 + w / (j + 1);
+        bl = w % (j + 1);
+    } else {
+        kind = 3;
+        bi = j;
+        bl = w - m * (j + 1);
+    }
+    // block (r0, c0) of the column-major M into LDS, rows or columns first, zero past k
+    auto load = [&](double *dst, const double *M, int r0, int c0, bool transpose) {
+        for (int e = t; e < kNb * kNb; e += 256) {
+            const int r = e & (kNb - 1), c = e >> 5;
+            const double x = r0 + r < k && c0 + c < k ? M[r0 + r + ld * (c0 + c)] : 0.0;
+            dst[transpose ? c * kNbLd + r : r * kNbLd + c] = x;
+        }
+    };
+    auto rows_of = [&](int q) { return 16 * (wave >> 1) + (lane >> 4) + 4 * q; };
+    const int col = 16 * (wave & 1) + (lane & 15);
+    if (kind != 3) load(pa, S, kNb * bi, j0, false);
+    if (kind == 1) load(pb, S, kNb * bl, j0, false);
+    if (kind != 1 && bl < j) load(pb, B, j0, kNb * bl, true);  // B_jc^T
+    __syncthreads();
+    sd4 x = {0.0, 0.0, 0.0, 0.0}, y = x;
+    if (kind != 3) x = block_pqt(pa, Li, wave, lane);                    // L_ij
+    if (kind == 1) y = block_pqt(pb, Li, wave, lane);                    // L_lj
+    if (kind != 1) {
+        if (bl < j)
+            y = block_pqt(Li, pb, wave, lane);                           // Linv_jj B_jc
+        else
+#pragma unroll
+            for (int q = 0; q < 4; ++q) y[q] = Li[rows_of(q) * kNbLd + col];
+    }
+    if (kind == 3) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = j0 + rows_of(q), c = kNb * bl + col;
+            if (r >= k || c >= k) continue;
+            Q[c + ld * r] = y[q];
+            if (bl < j) Q[r + ld * c] = 0.0;
+        }
         return;
     }
-    // Linv by forward substitution, one column per thread: L Linv[:, c] = e_c
-    if (t < k) {
-        const int c = t;
-        for (int i = 0; i < k; ++i) {
-            double s = i == c ? 1.0 : 0.0;
-            for (int l = c; l < i; ++l) s -= A[i + kLd * l] * Li[l + kLd * c];
-            Li[i + kLd * c] = i < c ? 0.0 : s / A[i + kLd * i];
-        }
+    __syncthreads();  // every wave has read pa and pb
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        pa[rows_of(q) * kNbLd + col] = x[q];
+        if (kind == 1)
+            pb[rows_of(q) * kNbLd + col] = y[q];
+        else
+            pc[col * kNbLd + rows_of(q)] = y[q];
     }
     __syncthreads();
-    // QT[i][j] = Linv[j][i]
-    for (int e = t; e < k * k; e += 256) {
-        const int i = e % k, j = e / k;
-        QT[i + (int64_t)k * j] = Li[j + kLd * i];
+    const sd4 u = block_pqt(pa, kind == 1 ? pb : pc, wave, lane);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int r = kNb * bi + rows_of(q), c = kNb * bl + col;
+        if (r >= k || c >= k) continue;
+        if (kind == 1)
+            S[r + ld * c] -= u[q];
+        else
+            B[r + ld * c] = (bl < j ? B[r + ld * c] : 0.0) - u[q];
     }
-    if (t == 0) *info = 0;
 }
 
 // Pair t of round r of the round-robin (circle) order on m players: player 0
@@ -359,10 +476,19 @@ bool small_dense_enabled(int32_t k) {
     return !off && k >= 1 && k <= kMax;
 }
 
-int small_chol_inv(ttdft_ctx ctx, const double *S, int32_t k, double *QT) {
-    hipLaunchKernelGGL(small_chol_inv_kernel, dim3(1), dim3(256), 0, ctx->stream, S, k, QT,
-                       ctx->d_info);
+int chol_inv(ttdft_ctx ctx, double *S, double *work, int32_t k, double *Q) {
+    const int nb = (k + kNb - 1) / kNb;
+    for (int j = 0; j < nb; ++j) {
+        const int m = nb - 1 - j;
+        const unsigned tiles = (unsigned)(m * (m + 1) / 2 + (m + 1) * (j + 1));
+        hipLaunchKernelGGL(chol_inv_step_kernel, dim3(tiles), dim3(256), 0, ctx->stream, S, work,
+                           Q, k, j, ctx->d_info);
+    }
     TT_LAUNCH_CHECK();
+    return TTDFT_OK;
+}
+
+int chol_check(ttdft_ctx ctx) {
     int info = 0;
     TT_HIP(hipMemcpyAsync(&info, ctx->d_info, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     TT_HIP(hipStreamSynchronize(ctx->stream));
