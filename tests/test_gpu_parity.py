@@ -370,6 +370,26 @@ def test_rotate_bf16x3_shapes(ctx, n, k, ld):
     assert np.array_equal(got[:, k:], X[:, k:].astype(np.float64))
 
 
+@pytest.mark.parametrize("k", [1, 32, 33, 64, 65, 255, 319, 320, 321])
+@pytest.mark.parametrize("n", [1, 31, 33, 128, 129])
+def test_rotate_in_place_edges(ctx, n, k):
+    """The in-place form (up to 320 columns) at the edges of its 32-row waves,
+    128-row workgroups, 32-deep steps and 64-column variants, with aligned and
+    odd leading dimensions; columns past k stay as they are.  Split-BF16: a
+    value less its hi half is at most 2^-8 of it, so a product leaves out
+    lo lo' (2^-16) and the roundings of both lo halves (2^-17 each)."""
+    rng = np.random.default_rng(n * 1000 + k)
+    Q = rng.standard_normal((k, k))
+    for ld in (k, (k + 8) // 4 * 4, k + 1):
+        X = rng.standard_normal((n, ld)).astype(np.float32)
+        dX, dQ = dev(ctx, X, np.float32), dev(ctx, Q.T.copy())
+        print(f"rotate in place n={n} k={k} ld={ld}", flush=True)
+        ctx.rotate(dX.ptr, ld, n, k, dQ.ptr, E.F32, E.GEMM_BF16X3)
+        Z = dX.to_host().reshape(n, ld)
+        assert rel(Z[:, :k].astype(np.float64), X[:, :k].astype(np.float64) @ Q) < 2.0 ** -15
+        assert np.array_equal(Z[:, k:], X[:, k:])
+
+
 @pytest.mark.parametrize("mode", [E.GEMM_F64, E.GEMM_BF16X3])
 def test_rotate_and_orth(ctx, mode):
     n, k = 4000, 100

