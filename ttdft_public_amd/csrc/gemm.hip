@@ -359,7 +359,7 @@ __global__ __launch_bounds__(256, 1) void gram_f64_lds_kernel(
 // l = bj + 16 (ai/4), v = ai%4; for the f64 MFMA (P double) l = bj + 16 (ai%4),
 // v = ai/4.  Bound by the latency of a strided read per chunk: a workgroup
 // takes one tile, four quarters of the chunks at once (k = 300, 170 chunks:
-// 57 -> REDUCE_US us with one thread per entry of S before).
+// 57 -> 15 us with one thread per entry of S before).
 template <typename P_t>
 __global__ __launch_bounds__(1024) void reduce_tile_partials_kernel(
     const P_t *__restrict__ P, int nchunks, int32_t k, int32_t nt, int sym,
@@ -493,7 +493,7 @@ __global__ __launch_bounds__(256) void rotate_bf16x3_frag_kernel(
 // one wave that writes it, after its last read.  Q comes as hi/lo fragments
 // of 16x16x32 MFMA, 2 KB per tile and 32-deep step, loaded straight into two
 // LDS stages in turn and shared by the four waves; X's next step is loaded
-// into registers meanwhile.  0.32 -> ROT_MS ms.  Past 320 columns the
+// into registers meanwhile.  0.32 -> 0.083 ms.  Past 320 columns the
 // accumulators no longer fit the registers beside the operands.
 //
 // Fragments: step s, tile t, piece h (hi, lo), lane j + 16 q, eight BF16:

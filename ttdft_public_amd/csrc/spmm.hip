@@ -467,6 +467,15 @@ __device__ __forceinline__ void split_bf16(float x, float y, unsigned &a, unsign
                   ry - __builtin_bit_cast(float, b & 0xffff0000u));
 }
 
+// Sign that FP32 fragments of stage `st` carry in state c, undone as the
+// stage's sums are added up: (-1)^c times stage_sign.  A BF16 product rounds
+// its aligned terms towards minus infinity, so without it every sum of small
+// terms would err to the same side; a filter adds that up over its steps
+// (8,000 x 24, degree 20: error 1.2e-5 in place of 1.0e-6; FP32 products 4.9e-6).
+__device__ __forceinline__ unsigned stage_flip(int64_t st) {
+    return ((unsigned)st * 2654435761u) & 0x80000000u;
+}
+
 // Writes the fragment entries of rows 8 o .. 8 o + 7 of state c.
 __device__ __forceinline__ void store_fragment(const double (&y)[8], int64_t o, int c,
                                                int32_t ntiles, double *F) {
@@ -478,10 +487,14 @@ __device__ __forceinline__ void store_fragment(const double (&y)[8], int64_t o, 
 __device__ __forceinline__ void store_fragment(const float (&y)[8], int64_t o, int c,
                                                int32_t ntiles, float *F) {
     uv4 a, b, d;
+    const unsigned flip = stage_flip(o >> 2) ^ ((unsigned)(c & 1) << 31);
+    auto signed_y = [&](int i) {
+        return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, y[i]) ^ flip);
+    };
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         unsigned p, q, r;
-        split_bf16(y[2 * i], y[2 * i + 1], p, q, r);
+        split_bf16(signed_y(2 * i), signed_y(2 * i + 1), p, q, r);
         a[i] = p;
         b[i] = q;
         d[i] = r;
@@ -555,7 +568,7 @@ template <> struct RingH<float> {
 template <int JT>
 __device__ __forceinline__ void ring_products(const RingH<double> &cur, RingH<double> &next,
                                               const unsigned char *hnext, const unsigned char *xb,
-                                              int wave, int lane, dv4 (&acc)[1][JT]) {
+                                              int wave, int lane, int64_t, dv4 (&acc)[1][JT]) {
     typedef double v2 __attribute__((ext_vector_type(2)));
     const unsigned xa = lds_addr(xb) + lane * 16;
 #pragma unroll
@@ -577,15 +590,19 @@ __device__ __forceinline__ void ring_products(const RingH<double> &cur, RingH<do
 template <int JT>
 __device__ __forceinline__ void ring_products(const RingH<float> &cur, RingH<float> &next,
                                               const unsigned char *hnext, const unsigned char *xb,
-                                              int wave, int lane, fv4 (&acc)[2][JT]) {
+                                              int wave, int lane, int64_t st, fv4 (&acc)[2][JT]) {
     const unsigned xa = lds_addr(xb) + lane * 16;
     v4f_t xr[2][3];
     lds_read3<1024, 2048>(xa, xr[0][0], xr[0][1], xr[0][2]);
     next.read(hnext, wave, lane);
     // The stage's sums start from zero and are added to the running ones by
-    // vector adds: these round to nearest, where the accumulator of a BF16
-    // product is truncated, a bias that grows with the number of products
-    // (27,000 x 96, degree 20: error 5.9e-5 in place of 1.6e-5, as on FP32 products).
+    // vector instructions, which round to nearest, with the signs that the
+    // fragments carry.
+    const float even = __builtin_bit_cast(float, stage_flip(st) ^ 0x3f800000u);
+    auto add = [&](fv4 &c, const fv4 &s) {  // element v holds state 4 q + v of the tile
+#pragma unroll
+        for (int v = 0; v < 4; ++v) c[v] = __builtin_fmaf(v & 1 ? -even : even, s[v], c[v]);
+    };
     fv4 sum[2][2];
 #pragma unroll
     for (int jt = 0; jt < JT; ++jt) {
@@ -612,7 +629,7 @@ __device__ __forceinline__ void ring_products(const RingH<float> &cur, RingH<flo
         RING_MMA(x0, h0)
 #undef RING_MMA
         if (jt > 0)
-            for (int rt = 0; rt < 2; ++rt) acc[rt][jt - 1] += sum[(jt - 1) & 1][rt];
+            for (int rt = 0; rt < 2; ++rt) add(acc[rt][jt - 1], sum[(jt - 1) & 1][rt]);
         next.split(8 * jt / JT, 8 * (jt + 1) / JT);
         // one product, then three vector instructions of the adds and the
         // split, in turn
@@ -623,7 +640,7 @@ __device__ __forceinline__ void ring_products(const RingH<float> &cur, RingH<flo
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    for (int rt = 0; rt < 2; ++rt) acc[rt][JT - 1] += sum[(JT - 1) & 1][rt];
+    for (int rt = 0; rt < 2; ++rt) add(acc[rt][JT - 1], sum[(JT - 1) & 1][rt]);
 }
 
 template <typename T, int JT>
@@ -706,7 +723,7 @@ __global__ __launch_bounds__(64 * kRingWaves) void dense_ring_kernel(
         fetch_x(st + NB - 1, b == 0 ? NB - 1 : b - 1);
         fetch_h(st + NB, b);
         const int bn = b + 1 == NB ? 0 : b + 1;
-        ring_products<JT>(cur, next, place(bn), place(b) + HB, wave, lane, acc);
+        ring_products<JT>(cur, next, place(bn), place(b) + HB, wave, lane, st, acc);
         b = bn;
     };
     for (int64_t st = sb; st < se; st += 2) {
