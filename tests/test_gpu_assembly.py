@@ -257,3 +257,39 @@ def test_ham_assemble_tucker_matches_host_path(ctx, dims, rv, band, ranks, fmt, 
         for k in (1, 20, 64):
             Xk = np.ascontiguousarray(X[:, :k])
             assert np.array_equal(_apply(ctx, hd, Xk, dtype), _apply(ctx, hh, Xk, dtype))
+
+
+@pytest.mark.parametrize("dims,ranks", [((10, 9, 8), [2, 2]), ((11, 9, 7), []), ((13, 13, 13), [1]),
+                                        ((12, 4, 11), [3])])
+def test_dense_assembly_spectrum_bounds(ctx, dims, ranks):
+    """A matrix assembled straight into dense storage (rows and columns past
+    multiples of 16 and 32, entries dropped by the truncation, the projectors
+    folded in) has no CSR copy: products against the host path's bits and the
+    Lanczos bounds against the CSR rows of the same matrix (sums of up to 2,200
+    products in another order: 1e-13 of the norm a step, 20 steps)."""
+    hl = hloc_inputs(31, dims, (3, 4, 2), max(dims), sym=True)
+    proj = proj_inputs(32, dims, ranks) if ranks else None
+    p = len(ranks)
+    inv = np.linspace(-1.5, 2.0, p) if p else None
+    hd = ctx.ham_assemble_tucker(hl, 1e-2, proj, 1e-6, inv, E.HAM_F64 | E.HAM_F32)
+    rp, c, v = ctx.assemble_hloc(*hl, 1e-2)
+    n = int(np.prod(dims))
+    assert hd.format()[0] == 2 and hd.info()[1] == len(v) < n * n
+    crp, cc, cv = ctx.assemble_projectors(*proj, 1e-6) if p else (None, None, None)
+    hh = E.Hamiltonian(ctx, n, rp, c, v, p, crp, cc, cv, inv, E.HAM_F64 | E.HAM_F32, dims=dims)
+    X = np.random.default_rng(3).standard_normal((n, 20))
+    for dtype in (E.F64, E.F32):
+        assert np.array_equal(_apply(ctx, hd, X, dtype), _apply(ctx, hh, X, dtype))
+    H = np.zeros((n, n))
+    for i in range(n):
+        H[i, c[rp[i]:rp[i + 1]]] = v[rp[i]:rp[i + 1]]
+    if p:
+        C = np.zeros((p, n))
+        for i in range(p):
+            C[i, cc[crp[i]:crp[i + 1]]] = cv[crp[i]:crp[i + 1]]
+        H += C.T @ (inv[:, None] * C)
+    up, lo = ctx.lanczos_bounds(hd, 20, seed=11)
+    w = np.linalg.eigvalsh(0.5 * (H + H.T))
+    upo, loo = ctx.lanczos_bounds(hh, 20, seed=11)
+    assert up >= w[-1] - 1e-9 * abs(w).max()
+    assert abs(up - upo) < 1e-9 * abs(w).max() and abs(lo - loo) < 1e-9 * abs(w).max()

@@ -919,7 +919,8 @@ int ttdft_lanczos_bounds(ttdft_ctx ctx, ttdft_ham H, int32_t maxit, uint64_t see
                          double *lower) {
     clear_error();
     TT_CHECK(ctx && H && upper && lower && maxit >= 1, TTDFT_EBADARG, "lanczos: bad arguments");
-    TT_CHECK(H->val64, TTDFT_EBADARG, "lanczos needs the FP64 copy of H");
+    TT_CHECK(H->val64 || (H->format == 2 && H->dense64), TTDFT_EBADARG,
+             "lanczos needs the FP64 copy of H");
     const int64_t n = H->n;
     // EigenSolver.cc:186-388 with the start vector from the seeded generator
     std::vector<double> hv(n);

@@ -203,7 +203,11 @@ __global__ __launch_bounds__(256) void hloc_row_scan_kernel(const uint16_t *__re
 // the chip: the epilogue thresholds it, turns the keep bits into per-row
 // masks in LDS (wavefront ballots), and from the masks
 //   COUNT: cnt[row][y][z] = kept x of segment (pi, g);
-//   WRITE: each kept entry goes to rowptr[row] + rel[key] + (kept x' < x).
+//          and the Kronecker half-bandwidths of the kept entries (flags[1..3]);
+//   WRITE: each kept entry goes to rowptr[row] + rel[key] + (kept x' < x);
+//   DENSE: every entry goes to its place in the dense storage, 0 where it is
+//          dropped (13 atoms, n = 8,000: 205 us; the CSR arrays, their
+//          extents and the scatter from them to dense took 0.97 ms).
 struct FusedArgs {
     const double *A;  // Ae, (Mp rows) x (K4 + 8 planes), A[pi + Mp k], rows >= M zero
     const double *B;  // Be, (K4 + 8 planes) x ldb, B[k ldb + t], ldb >= ntup + 256
@@ -216,7 +220,10 @@ struct FusedArgs {
     int32_t *col;
     double *val;
     int32_t *flags;  // mismatch, half-bandwidths x, y, z
+    double *dense;   // dense storage, leading dimension dense_ld
+    int64_t dense_ld;
 };
+enum { kCount = 0, kWrite = 1, kDense = 2 };
 
 typedef double fd4_t __attribute__((ext_vector_type(4)));
 
@@ -235,7 +242,7 @@ __device__ inline int mask_popc(const uint16_t *m, int lo, int hi) {
     return c;
 }
 
-template <int WRITE>
+template <int PASS>
 __global__ __launch_bounds__(256, 2) void hloc_fused_kernel(FusedArgs a) {
     __shared__ uint16_t mask[64][16];
     __shared__ int64_t segbase[64 * kFusedGt];
@@ -291,6 +298,29 @@ __global__ __launch_bounds__(256, 2) void hloc_fused_kernel(FusedArgs a) {
         pb += 2 * sb;
     }
     if (ks < nks) mma(fa0, fb0);
+    if constexpr (PASS == kDense) {
+        const int64_t rxy = (int64_t)a.rx * a.ry;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int colj = 64 * w + 16 * j + li;
+            const int gl = colj / a.rx, x = colj - gl * a.rx;
+            const int g = (int)g0 + gl;
+            const int gy = g / a.rx, xI = g - gy * a.rx;
+            const int yI = gy / a.ry, y = gy - yI * a.ry;
+            double *d = a.dense + (xI + (int64_t)a.rx * yI) * a.dense_ld + x + a.rx * y;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int pi = pi0 + 16 * i + lk + 4 * v;
+                    if (colj >= ncols || pi >= a.M) continue;
+                    const int zI = pi / a.rz, z = pi - zI * a.rz;
+                    const double hv = acc[i][j][v];
+                    d[rxy * (zI * a.dense_ld + z)] = fabs(hv) > a.trunc ? hv : 0.0;
+                }
+        }
+        return;
+    }
     // ---- epilogue: keep bits -> row masks
     // lane (li, lk), tile (i, j), element v: row 16 i + lk + 4 v, column 64 w + 16 j + li
 #pragma unroll
@@ -311,6 +341,7 @@ __global__ __launch_bounds__(256, 2) void hloc_fused_kernel(FusedArgs a) {
     __syncthreads();
     // ---- segments (row, group): counts, and for WRITE the base offsets
     const int nseg = 64 * gcnt;
+    int ex = -1, ey = -1, ez = -1;
     for (int s = threadIdx.x; s < nseg; s += 256) {
         const int r = s % 64, gl = s / 64;
         const int pi = pi0 + r;
@@ -322,8 +353,17 @@ __global__ __launch_bounds__(256, 2) void hloc_fused_kernel(FusedArgs a) {
         const int yI = gy / a.ry, y = gy - yI * a.ry;
         const int64_t rowid = xI + (int64_t)a.rx * (yI + (int64_t)a.ry * zI);
         const int64_t key = (rowid * a.ry + y) * a.rz + z;
-        if (!WRITE) {
+        if (PASS == kCount) {
             a.cnt[key] = (uint16_t)kept;
+            if (kept > 0) {
+                const int lo = gl * a.rx;
+                int first = 0, last = a.rx - 1;
+                while (!(mask[r][(lo + first) >> 4] >> ((lo + first) & 15) & 1)) ++first;
+                while (!(mask[r][(lo + last) >> 4] >> ((lo + last) & 15) & 1)) --last;
+                ex = max(ex, max(xI - first, last - xI));
+                ey = max(ey, abs(y - yI));
+                ez = max(ez, abs(z - zI));
+            }
         } else {
             const int expect = a.cnt[key];
             if (kept != expect) a.flags[0] = 1;
@@ -331,7 +371,28 @@ __global__ __launch_bounds__(256, 2) void hloc_fused_kernel(FusedArgs a) {
             segcnt[r * kFusedGt + gl] = min(kept, expect);
         }
     }
-    if (!WRITE) return;
+    if (PASS == kCount) {
+        for (int o = 32; o > 0; o >>= 1) {
+            ex = max(ex, __shfl_xor(ex, o));
+            ey = max(ey, __shfl_xor(ey, o));
+            ez = max(ez, __shfl_xor(ez, o));
+        }
+        if (lane == 0) {
+            segcnt[w] = ex;
+            segcnt[4 + w] = ey;
+            segcnt[8 + w] = ez;
+        }
+        __syncthreads();
+        if (threadIdx.x < 3) {
+            int m = -1;
+            for (int q = 0; q < 4; ++q) m = max(m, segcnt[4 * threadIdx.x + q]);
+            // (most workgroups find the maximum already there)
+            if (m > __hip_atomic_load(a.flags + 1 + threadIdx.x, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT))
+                atomicMax(a.flags + 1 + threadIdx.x, m);
+        }
+        return;
+    }
     __syncthreads();
     // ---- scatter the kept entries (loops unrolled: acc stays in registers)
 #pragma unroll
@@ -569,7 +630,12 @@ int check_hloc(const HlocIn &a) {
 // H_loc rows.  Always: the row pointer (out.rp, out.nnz).  fill: the device
 // CSR (out.rowptr / col / val) and the Kronecker half-bandwidths of the kept
 // entries (ext, -1 when there are none).
-int hloc_run(ttdft_ctx ctx, const HlocIn &a, bool fill, DevCsr &out, int ext[3]) {
+//
+// With `dense` a matrix that has no band storage but qualifies for dense
+// storage is written there instead (*dense, leading dimension *dense_ld,
+// padding zero); out then holds only the row pointer.
+int hloc_run(ttdft_ctx ctx, const HlocIn &a, bool fill, DevCsr &out, int ext[3],
+             double **dense = nullptr, int64_t *dense_ld = nullptr) {
     const int32_t rx = a.rx, ry = a.ry, rz = a.rz, rvx = a.rvx, rvy = a.rvy, rvz = a.rvz;
     const int64_t n = (int64_t)rx * ry * rz;
     const int64_t rx2 = (int64_t)rx * rx, ry2 = (int64_t)ry * ry, rz2 = (int64_t)rz * rz;
@@ -660,7 +726,7 @@ int hloc_run(ttdft_ctx ctx, const HlocIn &a, bool fill, DevCsr &out, int ext[3])
             f.rowptr = drowptr;
             f.col = dcol;
             f.val = dval;
-            auto kern = write ? hloc_fused_kernel<1> : hloc_fused_kernel<0>;
+            auto kern = write ? hloc_fused_kernel<kWrite> : hloc_fused_kernel<kCount>;
             hipLaunchKernelGGL(kern, dim3((unsigned)f.nblocks), dim3(256), 0, ctx->stream, f);
             TT_LAUNCH_CHECK();
             return TTDFT_OK;
@@ -713,23 +779,43 @@ int hloc_run(ttdft_ctx ctx, const HlocIn &a, bool fill, DevCsr &out, int ext[3])
     TT_TRY(timing_end(ctx, &tm, 14.0 * n * ry * rz, flops));
     std::vector<int64_t> len(n);
     out.rp.assign(n + 1, 0);
+    int32_t flags[4];
     TT_HIP(hipMemcpyAsync(len.data(), drowlen.p, sizeof(int64_t) * n, hipMemcpyDeviceToHost,
                           ctx->stream));
+    TT_HIP(hipMemcpyAsync(flags, dflag.p, sizeof(flags), hipMemcpyDeviceToHost, ctx->stream));
     TT_HIP(hipStreamSynchronize(ctx->stream));
     for (int64_t i = 0; i < n; ++i) out.rp[i + 1] = out.rp[i] + len[i];
     out.nnz = out.rp[n];
     if (!fill) return TTDFT_OK;
+    if (fused) {  // the count pass left the half-bandwidths
+        for (int d = 0; d < 3; ++d) ext[d] = flags[1 + d];
+        if (dense && dense_storage_fits(n, out.nnz) &&
+            !(ext[0] >= 0 && band_storage_fits(rx, ry, rz, ext[0], ext[1], ext[2], out.nnz))) {
+            FusedArgs f = fa;
+            f.dense_ld = dense_leading_dim(n);
+            TT_TRY(dev_alloc(ctx, (void **)dense, sizeof(double) * dense_elements(n)));
+            f.dense = *dense;  // (the caller's from here on)
+            *dense_ld = f.dense_ld;
+            TT_TRY(timing_begin(ctx, TTDFT_KSTAT_ASSEMBLY, &tm));
+            TT_TRY(launch_dense_padding(ctx, n, *dense));
+            hipLaunchKernelGGL(hloc_fused_kernel<kDense>, dim3((unsigned)f.nblocks), dim3(256), 0,
+                               ctx->stream, f);
+            TT_LAUNCH_CHECK();
+            return timing_end(ctx, &tm, 8.0 * n2, flops);
+        }
+    }
     TT_TRY(upload_to(ctx, out.rowptr, out.rp.data(), sizeof(int64_t) * (n + 1)));
     TT_TRY(out.col.alloc(ctx, sizeof(int32_t) * out.nnz));
     TT_TRY(out.val.alloc(ctx, sizeof(double) * out.nnz));
     TT_TRY(timing_begin(ctx, TTDFT_KSTAT_ASSEMBLY, &tm));
     TT_TRY(run_pass(1, out.rowptr.as<int64_t>(), out.col.as<int32_t>(), out.val.as<double>()));
     TT_TRY(timing_end(ctx, &tm, 12.0 * out.nnz + 8.0 * (n + 1), flops));
-    hipLaunchKernelGGL(band_extent_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0,
-                       ctx->stream, out.rowptr.as<int64_t>(), out.col.as<int32_t>(), n, rx, ry,
-                       dflag.as<int32_t>() + 1);
-    TT_LAUNCH_CHECK();
-    int32_t flags[4];
+    if (!fused) {
+        hipLaunchKernelGGL(band_extent_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0,
+                           ctx->stream, out.rowptr.as<int64_t>(), out.col.as<int32_t>(), n, rx,
+                           ry, dflag.as<int32_t>() + 1);
+        TT_LAUNCH_CHECK();
+    }
     TT_HIP(hipMemcpyAsync(flags, dflag.p, sizeof(flags), hipMemcpyDeviceToHost, ctx->stream));
     TT_HIP(hipStreamSynchronize(ctx->stream));
     TT_CHECK(!flags[0], TTDFT_ELIB, "assemble_hloc: count and write passes disagree");
@@ -930,16 +1016,19 @@ static int ham_assemble(ttdft_ctx ctx, const HlocIn &a, int32_t p, const int32_t
     const int64_t n = (int64_t)a.rx * a.ry * a.rz;
     DevCsr h;
     int ext[3];
-    TT_TRY(hloc_run(ctx, a, true, h, ext));
     H->n = n;
+    TT_TRY(hloc_run(ctx, a, true, h, ext, &H->dense64, &H->dense_ld));
+    if (H->dense64) H->format = 2;
     H->nnz = h.nnz;
     H->copies = copies;
     for (int64_t i = 0; i < n; ++i)
         H->max_row_nnz = std::max<int32_t>(H->max_row_nnz, (int32_t)(h.rp[i + 1] - h.rp[i]));
-    H->rowptr = h.rowptr.release<int64_t>();
-    H->col = h.col.release<int32_t>();
-    H->val64 = h.val.release<double>();
-    if (copies & TTDFT_HAM_F32) {
+    if (H->format != 2) {
+        H->rowptr = h.rowptr.release<int64_t>();
+        H->col = h.col.release<int32_t>();
+        H->val64 = h.val.release<double>();
+    }
+    if (H->val64 && (copies & TTDFT_HAM_F32)) {
         TT_TRY(dev_alloc(ctx, (void **)&H->val32, sizeof(float) * std::max<int64_t>(1, h.nnz)));
         if (h.nnz) {
             hipLaunchKernelGGL(to_f32_kernel, dim3(blocks_for(h.nnz, 256)), dim3(256), 0,
@@ -947,8 +1036,8 @@ static int ham_assemble(ttdft_ctx ctx, const HlocIn &a, int32_t p, const int32_t
             TT_LAUNCH_CHECK();
         }
     }
-    if (ext[0] >= 0) TT_TRY(build_band_device(ctx, H, a.rx, a.ry, a.rz, ext[0], ext[1], ext[2],
-                                              copies));
+    if (H->format != 2 && ext[0] >= 0)
+        TT_TRY(build_band_device(ctx, H, a.rx, a.ry, a.rz, ext[0], ext[1], ext[2], copies));
     TT_TRY(maybe_build_dense(ctx, H, copies));
     if (!(copies & TTDFT_HAM_F64)) {
         TT_HIP(hipStreamSynchronize(ctx->stream));

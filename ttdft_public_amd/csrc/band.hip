@@ -878,6 +878,11 @@ int build_band(ttdft_ctx ctx, ttdft_ham_s *H, int32_t rx, int32_t ry, int32_t rz
     return TTDFT_OK;
 }
 
+bool band_storage_fits(int32_t rx, int32_t ry, int32_t rz, int bx, int by, int bz, int64_t nnz) {
+    BandShape b;
+    return band_shape(rx, ry, rz, bx, by, bz, nnz, &b);
+}
+
 int build_band_device(ttdft_ctx ctx, ttdft_ham_s *H, int32_t rx, int32_t ry, int32_t rz, int bx,
                       int by, int bz, int copies) {
     const int64_t n = (int64_t)rx * ry * rz;

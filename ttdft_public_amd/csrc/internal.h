@@ -172,6 +172,7 @@ int build_band(ttdft_ctx ctx, ttdft_ham_s *H, int32_t rx, int32_t ry, int32_t rz
                const int64_t *rowptr, const int32_t *colind, const double *val, int copies);
 int build_band_device(ttdft_ctx ctx, ttdft_ham_s *H, int32_t rx, int32_t ry, int32_t rz, int bx,
                       int by, int bz, int copies);
+bool band_storage_fits(int32_t rx, int32_t ry, int32_t rz, int bx, int by, int bz, int64_t nnz);
 // Y = alpha*(H_loc X + C^T W) + beta*X + delta*Z   (Z may alias Y; flags select terms)
 // use_beta / use_delta select whether X / Z are read.
 // Q = L^{-T} (column-major, zero below the diagonal) of S = L L^T; S (lower
@@ -190,6 +191,9 @@ int small_orth(ttdft_ctx ctx, double *Y, int32_t n, int32_t b);
 // Dense storage (format 2) of H_loc when it is nearly full and small enough
 // (no-op otherwise); drop_dense frees it.
 bool dense_storage_fits(int64_t n, int64_t nnz);
+int64_t dense_leading_dim(int64_t n);
+size_t dense_elements(int64_t n);  // padded rows times leading dimension
+int launch_dense_padding(ttdft_ctx ctx, int64_t n, double *D);  // zeroes the padding
 int maybe_build_dense(ttdft_ctx ctx, ttdft_ham_s *H, int copies);
 int finish_dense(ttdft_ctx ctx, ttdft_ham_s *H, int copies);
 // Device blocks that live and die with Hamiltonians, rebuilt every SCF

@@ -796,6 +796,42 @@ __global__ __launch_bounds__(256) void dense_combine_kernel(
     if (F) store_fragment(yv, o, c, ntiles, F);
 }
 
+__global__ __launch_bounds__(256) void dense_padding_kernel(int64_t n, int64_t ld, int64_t count,
+                                                            double *__restrict__ D) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= count) return;
+    const int64_t w = ld - n, cols = n * w;  // columns n .. ld - 1, then rows n ..
+    if (e < cols)
+        D[e / w * ld + n + e % w] = 0.0;
+    else
+        D[n * ld + e - cols] = 0.0;
+}
+
+// y = H x on the dense storage (+ C^T w where that is not folded in): one
+// wavefront per row, 16 bytes of H a lane; HBM-bound (8 n^2 bytes).
+__global__ __launch_bounds__(256) void dense_spmv_kernel(
+    int64_t n, int64_t ld, const double *__restrict__ D, const double *__restrict__ x,
+    const int64_t *__restrict__ ct_rowptr, const int32_t *__restrict__ ct_col,
+    const double *__restrict__ ct_val, const double *__restrict__ w, double *__restrict__ y) {
+    typedef double v2 __attribute__((ext_vector_type(2)));
+    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= n) return;
+    const double *d = D + row * ld;
+    double s = 0.0;
+    for (int64_t l = 2 * lane; l < n; l += 128) {  // (a pair past n meets the padding of the row)
+        const v2 h = *reinterpret_cast<const v2 *>(d + l);
+        s += h[0] * x[l];
+        if (l + 1 < n) s += h[1] * x[l + 1];
+    }
+    if (ct_rowptr)
+        for (int64_t e = ct_rowptr[row] + lane; e < ct_rowptr[row + 1]; e += 64)
+            s += ct_val[e] * w[ct_col[e]];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    if (lane == 0) y[row] = s;
+}
+
 __global__ __launch_bounds__(256) void dense_to_f32_kernel(const double *__restrict__ s,
                                                            float *__restrict__ d, int64_t n) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -889,16 +925,23 @@ int launch_spmm_fused(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_
 }
 
 int ham_spmv(ttdft_ctx ctx, const ttdft_ham_s *H, const double *x, double *y) {
-    TT_CHECK(H->val64, TTDFT_EBADARG, "no FP64 copy of H_loc uploaded");
+    const bool dense = H->format == 2 && H->dense64;
+    TT_CHECK(dense || H->val64, TTDFT_EBADARG, "no FP64 copy of H_loc uploaded");
+    const bool folded = dense && H->dense_nl;
     double *W = nullptr;
-    if (H->p > 0) {
+    if (H->p > 0 && !folded) {
         TT_TRY(ctx->scratch[3].ensure((size_t)nl_workspace(H, 1) * sizeof(double)));
         W = (double *)ctx->scratch[3].ptr;
         TT_TRY(launch_nl_project(ctx, H, x, 1, 1, TTDFT_F64, W));
     }
-    hipLaunchKernelGGL(spmv_kernel, dim3((unsigned)((H->n + 3) / 4)), dim3(256), 0, ctx->stream,
-                       H->n, H->rowptr, H->col, H->val64, x, H->p > 0 ? H->ct_rowptr : nullptr,
-                       H->ct_col, H->ct_val64, W, y);
+    const int64_t *ctr = H->p > 0 && !folded ? H->ct_rowptr : nullptr;
+    const dim3 grid((unsigned)((H->n + 3) / 4));
+    if (dense)
+        hipLaunchKernelGGL(dense_spmv_kernel, grid, dim3(256), 0, ctx->stream, H->n, H->dense_ld,
+                           H->dense64, x, ctr, H->ct_col, H->ct_val64, W, y);
+    else
+        hipLaunchKernelGGL(spmv_kernel, grid, dim3(256), 0, ctx->stream, H->n, H->rowptr, H->col,
+                           H->val64, x, ctr, H->ct_col, H->ct_val64, W, y);
     TT_LAUNCH_CHECK();
     return TTDFT_OK;
 }
@@ -922,13 +965,26 @@ bool dense_storage_fits(int64_t n, int64_t nnz) {
     return n >= 1 && 8.0 * (double)n * (double)n <= kDenseMaxBytes &&
            (double)nnz >= 0.2 * (double)n * (double)n;
 }
+// rows padded to 16 and the leading dimension to 32 (the product's tiles)
+int64_t dense_leading_dim(int64_t n) { return (n + 31) / 32 * 32; }
+size_t dense_elements(int64_t n) {
+    return (size_t)((n + 15) / 16 * 16) * (size_t)dense_leading_dim(n);
+}
+int launch_dense_padding(ttdft_ctx ctx, int64_t n, double *D) {
+    const int64_t ld = dense_leading_dim(n), rows = (n + 15) / 16 * 16;
+    const int64_t pad = n * (ld - n) + (rows - n) * ld;
+    if (pad == 0) return TTDFT_OK;
+    hipLaunchKernelGGL(dense_padding_kernel, dim3((unsigned)((pad + 255) / 256)), dim3(256), 0,
+                       ctx->stream, n, ld, pad, D);
+    TT_LAUNCH_CHECK();
+    return TTDFT_OK;
+}
 int maybe_build_dense(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
     (void)copies;
     const int64_t n = H->n;
     if (H->format != 0 || !dense_storage_fits(n, H->nnz)) return TTDFT_OK;
-    // rows padded to 16 and the leading dimension to 32 (the product's tiles)
-    const int64_t ld = (n + 31) / 32 * 32;
-    const size_t n2 = (size_t)((n + 15) / 16 * 16) * (size_t)ld;
+    const int64_t ld = dense_leading_dim(n);
+    const size_t n2 = dense_elements(n);
     const unsigned rows = (unsigned)((n + 3) / 4);
     if (H->val64) {
         TT_TRY(dev_alloc(ctx, (void **)&H->dense64, sizeof(double) * n2));
@@ -960,7 +1016,7 @@ int maybe_build_dense(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
 int finish_dense(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
     if (H->format != 2 || !H->dense64) return TTDFT_OK;
     const int64_t n = H->n, ld = H->dense_ld;
-    const size_t n2 = (size_t)((n + 15) / 16 * 16) * (size_t)ld;
+    const size_t n2 = dense_elements(n);
     if (H->p > 0 && H->c_val64 && H->ct_val64) {
         const int64_t p = H->p;
         double *A1 = nullptr, *A2 = nullptr;  // D C as p x n rows, C^T as n x p rows
