@@ -738,6 +738,60 @@ def test_dense_product_row_blocks_and_parts(ctx, monkeypatch, n, k):
     ham.free()
 
 
+@pytest.mark.parametrize("n,half", [(40, 2), (65, 4), (1030, 40), (1500, 9)])
+@pytest.mark.parametrize("k", [7, 8, 37, 96, 97])
+def test_csr_block_storage(ctx, n, half, k):
+    """CSR matrices whose 32 x 32 blocks are at least a tenth full run by
+    blocks from 8 states on: banded rows with holes (n past multiples of 16, 32
+    and 1024, blocks cut by the last column), a duplicate entry, rows without
+    entries, projectors, in a filter with its fused recurrence.  FP64 to 1e-13
+    (sums of up to 81 products), FP32 to 8 steps of 2^-24 sqrt(81)."""
+    rng = np.random.default_rng(n + k)
+    i, j = np.indices((n, n))
+    A = np.where((np.abs(i - j) <= half) & ((i * j) % 7 != 3), rng.standard_normal((n, n)), 0.0)
+    A = np.triu(A) + np.triu(A, 1).T
+    A[5], A[:, 5] = 0.0, 0.0  # a row without entries
+    rowptr, col, val = [0], [], []
+    for r in range(n):
+        c = np.nonzero(A[r])[0]
+        v = A[r, c]
+        if r == 3:  # its first entry in two parts
+            c, v = np.insert(c, 0, c[0]), np.insert(v, 0, 0.25)
+            v[1] -= 0.25
+        col += c.tolist()
+        val += v.tolist()
+        rowptr.append(len(col))
+    assert len(col) < 0.2 * n * n
+    C = np.zeros((2, n))
+    C[0, :9], C[1, n // 2:n // 2 + 5] = 0.3, -0.2
+    cc = [np.nonzero(C[q])[0] for q in range(2)]
+    inv = np.array([0.7, -0.4])
+    ham = E.Hamiltonian(ctx, n, np.array(rowptr), np.array(col, np.int32), np.array(val), 2,
+                        np.array([0, len(cc[0]), len(cc[0]) + len(cc[1])]),
+                        np.concatenate(cc).astype(np.int32),
+                        np.concatenate([C[0, cc[0]], C[1, cc[1]]]), inv,
+                        copies=E.HAM_F64 | E.HAM_F32)
+    H = A + C.T @ (inv[:, None] * C)
+    X = rng.standard_normal((n, k))
+    a, b, a0 = -2.0, 30.0, -10.0
+    e, c0 = (b - a) / 2, (b + a) / 2
+    for dtype, npdt, tol in ((E.F64, np.float64, 1e-13), (E.F32, np.float32, 8 * 2.0 ** -24 * 9)):
+        Xc = X.astype(npdt)
+        sigma = e / (a0 - c0)
+        gamma = 2.0 / sigma
+        prev = Xc.astype(np.float64)
+        cur = (sigma / e) * (H @ prev - c0 * prev)
+        for _ in range(2, 5):
+            nxt = 1.0 / (gamma - sigma)
+            prev, cur = cur, (2 * nxt / e) * (H @ cur - c0 * cur) - sigma * nxt * prev
+            sigma = nxt
+        dX = dev(ctx, Xc, npdt)
+        print(f"csr blocks n={n} half={half} k={k} dtype={dtype}", flush=True)
+        ctx.cheb_filter(ham, dX.ptr, k, k, 5, a, b, a0, 1, dtype)
+        assert rel(dX.to_host().astype(np.float64), cur) < tol
+    ham.free()
+
+
 def test_dense_storage_reuse_across_hamiltonians(ctx):
     """Hamiltonians of different sizes built and freed in turn on one context:
     the dense storage and the projector fold come from the context's block

