@@ -436,14 +436,17 @@ def test_orth_block_columns_of_the_factorisation(ctx, k):
 
 
 @pytest.mark.parametrize("k,col", [(8, 5), (80, 0), (80, 31), (80, 32), (80, 79), (300, 290)])
-def test_orth_not_spd_in_any_block(ctx, k, col):
+@pytest.mark.parametrize("f32", [False, True])
+def test_orth_not_spd_in_any_block(ctx, k, col, f32):
     """A zero column gives an exactly zero pivot in whichever launch meets it;
-    X is left as it was."""
-    X = np.random.default_rng(2).standard_normal((600, k))
+    X is left as it was, also where the rotation runs in place (FP32)."""
+    npdt = np.float32 if f32 else np.float64
+    X = np.random.default_rng(2).standard_normal((600, k)).astype(npdt)
     X[:, col] = 0.0
-    dX = dev(ctx, X)
+    dX = dev(ctx, X, npdt)
     with pytest.raises(E.TtdftError) as ei:
-        ctx.orth(dX.ptr, k, 600, k)
+        ctx.orth(dX.ptr, k, 600, k, E.F32 if f32 else E.F64,
+                 E.GEMM_BF16X3 if f32 else E.GEMM_F64)
     assert ei.value.status == E.ENOTSPD and f"minor {col + 1}" in str(ei.value)
     assert np.array_equal(dX.to_host(), X)
 

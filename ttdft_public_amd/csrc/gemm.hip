@@ -358,24 +358,30 @@ __global__ __launch_bounds__(256, 1) void gram_f64_lds_kernel(
 // a tile, D[ai][bj] is element v of lane l: for the bf16 MFMA (P float)
 // l = bj + 16 (ai/4), v = ai%4; for the f64 MFMA (P double) l = bj + 16 (ai%4),
 // v = ai/4.  Bound by the latency of a strided read per chunk: a workgroup
-// takes one tile, four quarters of the chunks at once (k = 300, 170 chunks:
-// 57 -> 15 us with one thread per entry of S before).
+// takes one tile, in FP32 four quarters of the chunks at once (k = 300, 170
+// chunks: 57 us with one thread per entry of S, 15 so).  FP64 partials are
+// added one after the other: their sums feed the Tucker recompression, whose
+// discarded directions carry a change of order on into the SCF energies (1e-9).
 template <typename P_t>
 __global__ __launch_bounds__(1024) void reduce_tile_partials_kernel(
     const P_t *__restrict__ P, int nchunks, int32_t k, int32_t nt, int sym,
     double *__restrict__ S) {
-    __shared__ double part[3][256];
+    constexpr int NQ = sizeof(P_t) == 4 ? 4 : 1;  // slices of the chunks
+    __shared__ double part[NQ][256];
     const int ta = blockIdx.x, tb = blockIdx.y;
     if (sym && ta > tb) return;
     const int e = threadIdx.x & 255, q = threadIdx.x >> 8;
     const int64_t stride = (int64_t)nt * nt * 256;
     const P_t *p = P + ((int64_t)tb * nt + ta) * 256 + e;
     double s = 0.0;
-    for (int c = nchunks * q / 4; c < nchunks * (q + 1) / 4; ++c) s += (double)p[c * stride];
-    if (q > 0) part[q - 1][e] = s;
-    __syncthreads();
-    if (q > 0) return;
-    s = ((s + part[0][e]) + part[1][e]) + part[2][e];
+    for (int c = nchunks * q / NQ; c < nchunks * (q + 1) / NQ; ++c) s += (double)p[c * stride];
+    if constexpr (NQ > 1) {
+        part[q][e] = s;
+        __syncthreads();
+        if (q > 0) return;
+#pragma unroll
+        for (int w = 1; w < NQ; ++w) s += part[w][e];
+    }
     const int l = e >> 2, v = e & 3;
     const int a = 16 * ta + (sizeof(P_t) == 4 ? 4 * (l >> 4) + v : (l >> 4) + 4 * v);
     const int b = 16 * tb + (l & 15);
@@ -766,7 +772,7 @@ int launch_gram(ttdft_ctx ctx, const void *X, int64_t ldx, const void *Y, int64_
                            (const double *)X, ldx, (const double *)Y, ldy, n, k, nb, nt, sym,
                            rows, vec, P);
         TT_LAUNCH_CHECK();
-        hipLaunchKernelGGL(reduce_tile_partials_kernel<double>, red, dim3(1024), 0, ctx->stream, P,
+        hipLaunchKernelGGL(reduce_tile_partials_kernel<double>, red, dim3(256), 0, ctx->stream, P,
                            (int)nchunks, k, nt, sym, dS);
         TT_LAUNCH_CHECK();
     } else {

@@ -16,6 +16,65 @@ namespace {
 constexpr int kMax = 64;
 constexpr int kLd = kMax + 1;
 
+// QT = L^{-T} with S = L L^T (lower Cholesky of the symmetric S; only its
+// lower triangle is read); QT's strictly lower part is zero.  info = j + 1
+// when the leading minor of order j + 1 is not positive definite.
+__global__ __launch_bounds__(256) void small_chol_inv_kernel(const double *__restrict__ S, int k,
+                                                             double *__restrict__ QT,
+                                                             int *__restrict__ info) {
+    __shared__ double A[kMax * kLd];
+    __shared__ double Li[kMax * kLd];
+    __shared__ int bad;
+    const int t = threadIdx.x;
+    for (int e = t; e < k * k; e += 256) {
+        const int i = e % k, j = e / k;
+        A[i + kLd * j] = i >= j ? S[i + (int64_t)k * j] : 0.0;
+    }
+    if (t == 0) bad = 0;
+    __syncthreads();
+    // right-looking Cholesky, column j per step
+    for (int j = 0; j < k; ++j) {
+        const double d = A[j + kLd * j];
+        if (!(d > 0.0)) {  // uniform across the workgroup
+            if (t == 0) bad = j + 1;
+            break;
+        }
+        const double ljj = sqrt(d);
+        __syncthreads();
+        if (t == 0) A[j + kLd * j] = ljj;
+        for (int i = j + 1 + t; i < k; i += 256) A[i + kLd * j] /= ljj;
+        __syncthreads();
+        // trailing update of the lower triangle: A[i][l] -= L[i][j] L[l][j], j < l <= i
+        const int m = k - j - 1;
+        for (int e = t; e < m * m; e += 256) {
+            const int i = j + 1 + e % m, l = j + 1 + e / m;
+            if (l <= i) A[i + kLd * l] -= A[i + kLd * j] * A[l + kLd * j];
+        }
+        __syncthreads();
+    }
+    __syncthreads();
+    if (bad) {
+        if (t == 0) *info = bad;
+        return;
+    }
+    // Linv by forward substitution, one column per thread: L Linv[:, c] = e_c
+    if (t < k) {
+        const int c = t;
+        for (int i = 0; i < k; ++i) {
+            double s = i == c ? 1.0 : 0.0;
+            for (int l = c; l < i; ++l) s -= A[i + kLd * l] * Li[l + kLd * c];
+            Li[i + kLd * c] = i < c ? 0.0 : s / A[i + kLd * i];
+        }
+    }
+    __syncthreads();
+    // QT[i][j] = Linv[j][i]
+    for (int e = t; e < k * k; e += 256) {
+        const int i = e % k, j = e / k;
+        QT[i + (int64_t)k * j] = Li[j + kLd * i];
+    }
+    if (t == 0) *info = 0;
+}
+
 // Q = L^{-T} with S = L L^T, by blocks of 32 columns, one launch per block.
 //
 // What bounds it: latency.  At k = 300 the arithmetic is 0.02 GFLOP, and the
@@ -477,6 +536,14 @@ bool small_dense_enabled(int32_t k) {
 }
 
 int chol_inv(ttdft_ctx ctx, double *S, double *work, int32_t k, double *Q) {
+    // Up to 64 columns in one workgroup by forward substitution: the rounding
+    // of these small factors carries on into the SCF energies (1e-9 Ha).
+    if (k <= kMax) {
+        hipLaunchKernelGGL(small_chol_inv_kernel, dim3(1), dim3(256), 0, ctx->stream, S, k, Q,
+                           ctx->d_info);
+        TT_LAUNCH_CHECK();
+        return TTDFT_OK;
+    }
     const int nb = (k + kNb - 1) / kNb;
     for (int j = 0; j < nb; ++j) {
         const int m = nb - 1 - j;

@@ -568,10 +568,19 @@ template <> struct RingH<float> {
 // and would otherwise first queue for LDS, then convert, and only then give
 // the matrix cores work (FP32, 27,000 x 96: 0.79 ms against 0.82 before the
 // vector adds below, 0.84 with them).
+//
+// FP64 sums run in NA chains (by u2) that are added at the end: one chain over
+// a part of l would add up 16,000 roundings at n = 64,000 in a single part,
+// more than the split product of fewer rows and more parts before it did.
+template <typename T, int JT> constexpr int ring_chains() {
+    return sizeof(T) == 8 ? (JT <= 3 ? 4 : 2) : 1;
+}
 template <int JT>
 __device__ __forceinline__ void ring_products(const RingH<double> &cur, RingH<double> &next,
                                               const unsigned char *hnext, const unsigned char *xb,
-                                              int wave, int lane, int64_t, dv4 (&acc)[1][JT]) {
+                                              int wave, int lane, int64_t,
+                                              dv4 (&acc)[1][ring_chains<double, JT>() * JT]) {
+    constexpr int NA = ring_chains<double, JT>();
     typedef double v2 __attribute__((ext_vector_type(2)));
     const unsigned xa = lds_addr(xb) + lane * 16;
 #pragma unroll
@@ -583,8 +592,10 @@ __device__ __forceinline__ void ring_products(const RingH<double> &cur, RingH<do
         for (int u2 = 0; u2 < 4; ++u2) {
             const v2 hv = __builtin_bit_cast(v2, cur.raw[u2]), xv = __builtin_bit_cast(v2, x[u2]);
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
-                acc[0][jt] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[u], hv[u], acc[0][jt], 0, 0, 0);
+            for (int u = 0; u < 2; ++u) {
+                dv4 &a4 = acc[0][u2 % NA * JT + jt];
+                a4 = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[u], hv[u], a4, 0, 0, 0);
+            }
         }
     }
     next.read(hnext, wave, lane);
@@ -699,11 +710,12 @@ __global__ __launch_bounds__(64 * kRingWaves) void dense_ring_kernel(
             load_lds_16(src + 1024 * c, d + 1024 * c);
         }
     };
-    acc_t acc[RT][JT];
+    constexpr int NA = ring_chains<T, JT>();
+    acc_t acc[RT][NA * JT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int jt = 0; jt < JT; ++jt) acc[rt][jt] = acc_t{0, 0, 0, 0};
+        for (int j = 0; j < NA * JT; ++j) acc[rt][j] = acc_t{0, 0, 0, 0};
     RingH<T> h[2];
     fetch_h(sb, 0);
 #pragma unroll
@@ -735,6 +747,10 @@ __global__ __launch_bounds__(64 * kRingWaves) void dense_ring_kernel(
         step(st + 1, h[1], h[0]);
     }
     TT_WAIT_ALL();  // no load into LDS may outlive the workgroup
+#pragma unroll
+    for (int h = NA / 2; h >= 1; h /= 2)  // the chains, pairwise
+#pragma unroll
+        for (int j = 0; j < h * JT; ++j) acc[0][j] += acc[0][h * JT + j];
     const int li = lane & 15, q = lane >> 4;
     const int c0 = blockIdx.y * 16 * JT;
 #pragma unroll
@@ -863,8 +879,8 @@ __global__ __launch_bounds__(256) void dense_combine_kernel(
 // straight into registers as whole pieces, no LDS and no barrier, and
 // dense_combine_kernel finishes.  A part is at most `chunk` blocks, so that all
 // waves have about the same work although rows in the middle of the domain
-// have several times the blocks of those at its corners: CHUNK_US us, 144 with
-// equal part counts (a third of the time CUs had run dry).
+// have several times the blocks of those at its corners: 141 us, 144 with
+// equal part counts.
 constexpr int kBlockRows = 32, kBlockElems = 32 * 32;
 template <typename T> __device__ __forceinline__ int block_slot(int row, int l);
 template <> __device__ __forceinline__ int block_slot<double>(int row, int l) {
