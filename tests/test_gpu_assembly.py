@@ -293,3 +293,40 @@ def test_dense_assembly_spectrum_bounds(ctx, dims, ranks):
     upo, loo = ctx.lanczos_bounds(hh, 20, seed=11)
     assert up >= w[-1] - 1e-9 * abs(w).max()
     assert abs(up - upo) < 1e-9 * abs(w).max() and abs(lo - loo) < 1e-9 * abs(w).max()
+
+
+def block_fill(rowptr, col, n):
+    """Share of the places of the 32 x 32 blocks that hold an entry."""
+    rows = np.repeat(np.arange(n, dtype=np.int64), np.diff(rowptr))
+    blocks = np.unique((rows // 32) * ((n + 31) // 32) + col // 32)
+    return len(col) / (1024.0 * len(blocks))
+
+
+@pytest.mark.parametrize("ranks", [[], [2, 1]])
+@pytest.mark.parametrize("copies", [E.HAM_F64, E.HAM_F32, E.HAM_F64 | E.HAM_F32])
+def test_csr_blocks_assembled_as_uploaded(ctx, ranks, copies):
+    """A CSR matrix with full 32 x 32 blocks (n = 1200, x reach 8 of 100, y and z
+    full) assembled on the device holds what the host path uploads: the same
+    bits from the row kernel (1 state) and from the blocks (8 and 40), and no
+    product in a precision that was not asked for."""
+    dims, p = (100, 4, 3), len(ranks)
+    hl = hloc_inputs(41, dims, (2, 2, 2), 8, sym=True)
+    proj = proj_inputs(42, dims, ranks) if ranks else None
+    inv = np.linspace(-1.5, 2.0, p) if p else None
+    hd = ctx.ham_assemble_tucker(hl, 0.0, proj, 1e-6, inv, copies)
+    rp, c, v = ctx.assemble_hloc(*hl, 0.0)
+    n = int(np.prod(dims))
+    assert block_fill(rp, c, n) >= 0.15 and len(c) < 0.2 * n * n
+    crp, cc, cv = ctx.assemble_projectors(*proj, 1e-6) if p else (None, None, None)
+    hh = E.Hamiltonian(ctx, n, rp, c, v, p, crp, cc, cv, inv, copies, dims=dims)
+    assert hd.format() == hh.format() and hd.format()[0] == 0
+    X = np.random.default_rng(3).standard_normal((n, 40))
+    for dtype, copy in ((E.F64, E.HAM_F64), (E.F32, E.HAM_F32)):
+        for k in (1, 8, 40):
+            Xk = np.ascontiguousarray(X[:, :k])
+            if copies & copy:
+                assert np.array_equal(_apply(ctx, hd, Xk, dtype), _apply(ctx, hh, Xk, dtype))
+                continue
+            for h in (hd, hh):
+                with pytest.raises(E.TtdftError):
+                    _apply(ctx, h, Xk, dtype)

@@ -737,7 +737,7 @@ int ttdft_ham_upload(ttdft_ctx ctx, int64_t n, const int64_t *rowptr, const int3
                      int copies, ttdft_ham *out) {
     TT_TRY(ham_upload(ctx, n, rowptr, colind, val, p, c_rowptr, c_colind, c_val, inv_c_lm, copies,
                       out));
-    return ham_upload_end(out, build_blocks(ctx, *out));
+    return ham_upload_end(out, build_blocks(ctx, *out, copies));
 }
 
 int ttdft_ham_upload_tucker(ttdft_ctx ctx, int32_t rx, int32_t ry, int32_t rz,
@@ -752,7 +752,7 @@ int ttdft_ham_upload_tucker(ttdft_ctx ctx, int32_t rx, int32_t ry, int32_t rz,
                       out));
     int rc = build_band(ctx, *out, rx, ry, rz, rowptr, colind, val, copies);
     if (rc == TTDFT_OK && (*out)->format == 1) drop_dense(*out);
-    if (rc == TTDFT_OK) rc = build_blocks(ctx, *out);
+    if (rc == TTDFT_OK) rc = build_blocks(ctx, *out, copies);
     return ham_upload_end(out, rc);
 }
 

@@ -197,7 +197,7 @@ int dev_fill_uniform(ttdft_ctx ctx, double *f, int64_t n, uint64_t seed, double 
 int small_orth(ttdft_ctx ctx, double *Y, int32_t n, int32_t b);
 // Dense storage (format 2) of H_loc when it is nearly full and small enough
 // (no-op otherwise); drop_dense frees it.
-int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H);
+int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H, int copies);
 void drop_blocks(ttdft_ham_s *H);
 bool dense_storage_fits(int64_t n, int64_t nnz);
 int64_t dense_leading_dim(int64_t n);

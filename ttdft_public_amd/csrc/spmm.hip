@@ -1498,11 +1498,15 @@ void drop_blocks(ttdft_ham_s *H) {
 // takes 43 ps (up to 64 states), per 32 x 32 block the block kernel about
 // 1.7 ns for its 8 KB and 0.4 ns per 16 states: even at 7% of a block's 1,024
 // places.  Stored from 10% on, where the storage (8 bytes a place against 12
-// an entry) is at most 7 times that of the rows.
-int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H) {
+// an entry) is at most 7 times that of the rows.  Only the precisions asked
+// for are built: a device assembly still holds its FP64 rows here when FP32
+// alone was.
+int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
     const int64_t n = H->n;
     const int64_t words = (n + 1023) / 1024, tiles = (n + kBlockRows - 1) / kBlockRows;
-    if (H->format != 0 || (!H->val64 && !H->val32) || H->nnz < 1 || words > 4096) return TTDFT_OK;
+    const bool f64 = H->val64 && (copies & TTDFT_HAM_F64);
+    const bool f32 = H->val32 && (copies & TTDFT_HAM_F32);
+    if (H->format != 0 || (!f64 && !f32) || H->nnz < 1 || words > 4096) return TTDFT_OK;
     int32_t *dcount = nullptr;
     TT_TRY(dev_alloc(ctx, (void **)&dcount, sizeof(int32_t) * tiles));
     const size_t lds = sizeof(unsigned) * 2 * (size_t)words;
@@ -1530,14 +1534,14 @@ int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H) {
     TT_HIP(hipMemcpyAsync(H->blk_ptr, ptr.data(), sizeof(int64_t) * (tiles + 1),
                           hipMemcpyHostToDevice, ctx->stream));
     TT_HIP(hipStreamSynchronize(ctx->stream));  // ptr goes out of scope
-    if (H->val64) {
+    if (f64) {
         TT_TRY(dev_alloc(ctx, (void **)&H->blk64, sizeof(double) * kBlockElems * nblk));
         TT_HIP(hipMemsetAsync(H->blk64, 0, sizeof(double) * kBlockElems * nblk, ctx->stream));
         hipLaunchKernelGGL((block_build_kernel<1, double>), dim3((unsigned)tiles), dim3(256), lds,
                            ctx->stream, n, (int32_t)words, H->rowptr, H->col, H->val64, nullptr,
                            H->blk_ptr, H->blk_col, H->blk64);
     }
-    if (H->val32) {
+    if (f32) {
         TT_TRY(dev_alloc(ctx, (void **)&H->blk32, sizeof(float) * kBlockElems * nblk));
         TT_HIP(hipMemsetAsync(H->blk32, 0, sizeof(float) * kBlockElems * nblk, ctx->stream));
         hipLaunchKernelGGL((block_build_kernel<1, float>), dim3((unsigned)tiles), dim3(256), lds,
