@@ -795,6 +795,57 @@ def test_csr_block_storage(ctx, n, half, k):
     ham.free()
 
 
+def banded_csr(n, half, seed, rows=()):
+    """Symmetric banded CSR with holes; `rows` are full rows (not mirrored)."""
+    rng = np.random.default_rng(seed)
+    rowptr, col, val = [0], [], []
+    for r in range(n):
+        c = np.arange(n) if r in rows else np.arange(max(0, r - half), min(n, r + half + 1))
+        c = c if r in rows else c[(r * c) % 7 != 3]
+        col.append(c)
+        val.append(rng.standard_normal(len(c)))
+        rowptr.append(rowptr[-1] + len(c))
+    return np.array(rowptr, np.int64), np.concatenate(col).astype(np.int32), np.concatenate(val)
+
+
+def csr_product(n, rowptr, col, val, X):
+    """H X in FP64, a row's products added in its order."""
+    Y = np.zeros((n, X.shape[1]))
+    for r in range(n):
+        Y[r] = val[rowptr[r]:rowptr[r + 1]] @ X[col[rowptr[r]:rowptr[r + 1]]]
+    return Y
+
+
+@pytest.mark.parametrize("copies", [E.HAM_F64, E.HAM_F32, E.HAM_F64 | E.HAM_F32])
+def test_csr_without_room_for_blocks(monkeypatch, copies):
+    """Block storage (2.3 MB an FP64 copy here, 1.1 MB FP32) that finds no
+    memory is left out: the CSR rows (0.7 MB at most an array) apply, with the
+    row kernel's bits, as seven columns (always the row kernel) show."""
+    n, k = 3000, 20
+    rowptr, col, val = banded_csr(n, 15, 5)
+    X = np.random.default_rng(6).standard_normal((n, k))
+    monkeypatch.setenv("TTDFT_ALLOC_LIMIT", str(1 << 20))
+    c = E.Context(0)
+    try:
+        ham = E.Hamiltonian(c, n, rowptr, col, val, 0, None, None, None, None, copies=copies)
+        ref = csr_product(n, rowptr, col, val, X)
+        for dtype, npdt, copy, tol in ((E.F64, np.float64, E.HAM_F64, 1e-13),
+                                       (E.F32, np.float32, E.HAM_F32, 1e-5)):
+            if not copies & copy:
+                continue
+            got = {}
+            for kk in (7, k):
+                dX = dev(c, X[:, :kk], npdt)
+                dY = E.DeviceArray(c, (n, kk), npdt)
+                c.ham_apply(ham, dX.ptr, kk, dY.ptr, kk, kk, dtype)
+                got[kk] = dY.to_host()
+            assert rel(got[k].astype(np.float64), ref) < tol
+            assert np.array_equal(got[k][:, :7], got[7])
+        ham.free()
+    finally:
+        c.close()
+
+
 def test_dense_storage_reuse_across_hamiltonians(ctx):
     """Hamiltonians of different sizes built and freed in turn on one context:
     the dense storage and the projector fold come from the context's block

@@ -48,6 +48,21 @@ void set_error(const char *fmt, ...) {
 }
 void clear_error() { g_err.clear(); }
 
+// hipMalloc of a device block.  TTDFT_ALLOC_LIMIT refuses blocks above that many
+// bytes, as a full device would: the paths that go on without an optional
+// block can be tested without filling the card.
+static hipError_t dev_malloc(void **p, size_t bytes) {
+    *p = nullptr;
+    const char *env = std::getenv("TTDFT_ALLOC_LIMIT");
+    if (env && bytes > std::strtoull(env, nullptr, 10)) return hipErrorOutOfMemory;
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError();  // a later launch check must not see this error
+    }
+    return e;
+}
+
 // ---- scratch ---------------------------------------------------------------
 int Scratch::ensure(size_t need) {
     if (need <= bytes) return TTDFT_OK;
@@ -60,13 +75,12 @@ int Scratch::ensure(size_t need) {
         ptr = nullptr;
         bytes = 0;
     }
-    hipError_t e = hipMalloc(&ptr, need);
+    hipError_t e = dev_malloc(&ptr, need);
     if (e != hipSuccess && owner && !owner->blk_free.empty()) {
         dev_cache_clear(owner);
-        e = hipMalloc(&ptr, need);
+        e = dev_malloc(&ptr, need);
     }
     if (e != hipSuccess) {
-        ptr = nullptr;
         set_error("scratch allocation of %zu bytes failed: %s", need, hipGetErrorString(e));
         return TTDFT_ENOMEM;
     }
@@ -309,13 +323,12 @@ int dev_alloc(ttdft_ctx ctx, void **p, size_t bytes) {
         ctx->blk_free.erase(it);
         ctx->blk_free_bytes -= c;
     } else {
-        hipError_t e = hipMalloc(p, c);
+        hipError_t e = dev_malloc(p, c);
         if (e != hipSuccess && !ctx->blk_free.empty()) {  // give the cached blocks back, retry
             dev_cache_clear(ctx);
-            e = hipMalloc(p, c);
+            e = dev_malloc(p, c);
         }
         if (e != hipSuccess) {
-            *p = nullptr;
             set_error("hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
             return TTDFT_ENOMEM;
         }

@@ -1501,7 +1501,7 @@ void drop_blocks(ttdft_ham_s *H) {
 // an entry) is at most 7 times that of the rows.  Only the precisions asked
 // for are built: a device assembly still holds its FP64 rows here when FP32
 // alone was.
-int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
+static int try_build_blocks(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
     const int64_t n = H->n;
     const int64_t words = (n + 1023) / 1024, tiles = (n + kBlockRows - 1) / kBlockRows;
     const bool f64 = H->val64 && (copies & TTDFT_HAM_F64);
@@ -1549,6 +1549,16 @@ int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
                            H->blk_ptr, H->blk_col, H->blk32);
     }
     TT_LAUNCH_CHECK();
+    return TTDFT_OK;
+}
+
+// The rows are whole without the blocks: where these find no memory, the row
+// kernel takes every product.
+int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
+    const int rc = try_build_blocks(ctx, H, copies);
+    if (rc != TTDFT_OK) drop_blocks(H);
+    if (rc != TTDFT_ENOMEM) return rc;
+    clear_error();
     return TTDFT_OK;
 }
 
