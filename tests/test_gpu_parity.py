@@ -846,6 +846,32 @@ def test_csr_without_room_for_blocks(monkeypatch, copies):
         c.close()
 
 
+def test_csr_block_parts_are_bounded(monkeypatch):
+    """One row tile that meets every column block among short ones (n = 40,000,
+    32 full rows): the block product's partial sums stay within 16 parts of the
+    block (350 MB with the operand; by the average list alone, 313 parts and
+    6.4 GB), so that it runs, and adds in another order than the row kernel,
+    where no more than 400 MiB are to be had."""
+    n, k = 40000, 64
+    rowptr, col, val = banded_csr(n, 6, 7, rows=range(64, 96))
+    X = np.random.default_rng(8).standard_normal((n, k))
+    monkeypatch.setenv("TTDFT_ALLOC_LIMIT", str(400 << 20))
+    c = E.Context(0)
+    try:
+        ham = E.Hamiltonian(c, n, rowptr, col, val, 0, None, None, None, None)
+        got = {}
+        for kk in (7, k):
+            dX, dY = dev(c, X[:, :kk]), E.DeviceArray(c, (n, kk))
+            c.ham_apply(ham, dX.ptr, kk, dY.ptr, kk, kk, E.F64)
+            got[kk] = dY.to_host()
+        assert not np.array_equal(got[k][:, :7], got[7])
+        # sums of up to 40,000 products of unit normal numbers
+        assert rel(got[k], csr_product(n, rowptr, col, val, X)) < 1e-12
+        ham.free()
+    finally:
+        c.close()
+
+
 def test_dense_storage_reuse_across_hamiltonians(ctx):
     """Hamiltonians of different sizes built and freed in turn on one context:
     the dense storage and the projector fold come from the context's block

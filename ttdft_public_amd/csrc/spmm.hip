@@ -1343,7 +1343,7 @@ int finish_dense(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
     return TTDFT_OK;
 }
 
-constexpr int kDenseParts = 16;  // most parts of l in the split dense product
+constexpr int kDenseParts = 16;  // most parts of the split dense and the block product
 
 // 0: one-kernel dense product; 1: form and parts picked; 2..16: split product
 // with that many parts
@@ -1562,13 +1562,17 @@ int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
     return TTDFT_OK;
 }
 
-// State tiles, parts and work space of the block product: about four waves'
-// chunks of blocks per SIMD, four blocks at least
+// State tiles, parts and work space of the block product: chunks of blocks for
+// about four waves per SIMD, four blocks at least, and as long as keeps the
+// longest list to kDenseParts parts: every part has a place for all rows, so
+// one full row tile in a sparse matrix would otherwise take gigabytes (200,000
+// rows x 64 states with 32 full rows: 91 GB).
 static DenseTiling block_tiling(const ttdft_ham_s *H, int32_t k, int dtype) {
     DenseTiling d;
     d.ncol = (k + 95) / 96;
     d.jt = (k + 16 * d.ncol - 1) / (16 * d.ncol);
-    d.chunk = (int)std::max<int64_t>((H->nblk * d.ncol + 4095) / 4096, 4);
+    d.chunk = (int)std::max<int64_t>({(H->nblk * d.ncol + 4095) / 4096, 4,
+                                      (H->blk_most + kDenseParts - 1) / kDenseParts});
     d.nparts = (int)((H->blk_most + d.chunk - 1) / d.chunk);
     d.partial_bytes = ((size_t)d.nparts * H->n * k * dtype_size(dtype) + 255) / 256 * 256;
     d.bytes = d.partial_bytes + (size_t)(dense_leading_dim(H->n) / 32) * d.ncol * d.jt * 1024 *
