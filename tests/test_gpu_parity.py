@@ -872,6 +872,43 @@ def test_csr_block_parts_are_bounded(monkeypatch):
         c.close()
 
 
+@pytest.mark.parametrize("form", ["blocks", "dense"])
+def test_filter_without_room_for_partial_sums(monkeypatch, form):
+    """Where the split products find no work space (1 MiB at most here; 1.2 MB
+    and more needed) the filter runs on the one-kernel products: the row
+    kernel's bits, as a Hamiltonian without block storage gives them, or the
+    one-kernel dense form's."""
+    if form == "blocks":
+        n, k = 3000, 20
+        rowptr, col, val = banded_csr(n, 15, 5)
+    else:
+        n, k = 300, 96
+        A = np.random.default_rng(9).standard_normal((n, n)) / np.sqrt(n)
+        rowptr, col = np.arange(n + 1, dtype=np.int64) * n, np.tile(np.arange(n, dtype=np.int32), n)
+        val = (A + A.T).reshape(-1)
+    X = np.random.default_rng(10).standard_normal((n, k))
+    got = []
+    for limited in (False, True):
+        c = E.Context(0)
+        try:
+            if form == "blocks" and not limited:  # no block storage: the row kernel
+                monkeypatch.setenv("TTDFT_ALLOC_LIMIT", str(1 << 20))
+            ham = E.Hamiltonian(c, n, rowptr, col, val, 0, None, None, None, None)
+            monkeypatch.delenv("TTDFT_ALLOC_LIMIT", raising=False)
+            dX = dev(c, X)
+            if form == "dense":
+                monkeypatch.setenv("TTDFT_DENSE_LDS", "16" if limited else "0")
+            if limited:
+                monkeypatch.setenv("TTDFT_ALLOC_LIMIT", str(1 << 20))
+            c.cheb_filter(ham, dX.ptr, k, k, 5, -2.0, 30.0, -10.0, 1, E.F64)
+            got.append(dX.to_host())
+            monkeypatch.delenv("TTDFT_ALLOC_LIMIT", raising=False)
+            ham.free()
+        finally:
+            c.close()
+    assert np.array_equal(got[0], got[1])
+
+
 def test_dense_storage_reuse_across_hamiltonians(ctx):
     """Hamiltonians of different sizes built and freed in turn on one context:
     the dense storage and the projector fold come from the context's block

@@ -870,9 +870,11 @@ int ttdft_cheb_filter(ttdft_ctx ctx, ttdft_ham H, void *X, int64_t ldx, int32_t 
         double sigma = e / (a0 - c);
         const double sigma1 = sigma, gamma = 2.0 / sigma1;
         double alpha = sigma1 / e, beta = alpha * (-c);
+        StepChain chain;
+        chain.want = target > 1;
         // Y_1 = alpha H X + beta X   -> B
         TT_TRY(ham_step(ctx, H, Ac, ldx, Bc, ldx, nullptr, 0, cols, dtype, alpha, beta, 0.0, 1,
-                        0, nullptr, 0, {false, target > 1}));
+                        0, nullptr, 0, &chain));
         char *cur = Bc, *prev = Ac;
         for (int it = 2; it <= target; ++it) {
             const double sigma2 = 1.0 / (gamma - sigma);
@@ -880,8 +882,9 @@ int ttdft_cheb_filter(ttdft_ctx ctx, ttdft_ham H, void *X, int64_t ldx, int32_t 
             beta = -c * alpha;
             const double delta = -sigma * sigma2;
             // Y_it = alpha H Y_{it-1} + beta Y_{it-1} + delta Y_{it-2}, written over Y_{it-2}
+            chain.want = it < target;
             TT_TRY(ham_step(ctx, H, cur, ldx, prev, ldx, prev, ldx, cols, dtype, alpha, beta,
-                            delta, 1, 1, nullptr, 0, {true, it < target}));
+                            delta, 1, 1, nullptr, 0, &chain));
             char *t = cur;
             cur = prev;
             prev = t;

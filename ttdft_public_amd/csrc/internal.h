@@ -238,8 +238,9 @@ int launch_band_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t
 // Consecutive applications of one H, each to the result of the one before
 // (same states, leading dimensions and work space, nothing else using that
 // work space between them): have: the previous step left its result in the
-// product's own operand layout there; want: do so for the next one.  Storage
-// forms without such a layout ignore it.
+// product's own operand layout there; want: do so for the next one.  A step
+// sets have for the next: a product without such a layout, or one that found
+// no work space, leaves nothing.
 struct StepChain {
     bool have = false, want = false;
 };
@@ -249,7 +250,7 @@ struct StepChain {
 int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, void *Y,
              int64_t ldy, const void *Z, int64_t ldz, int32_t k, int dtype, double alpha,
              double beta, double delta, int use_beta, int use_delta, void *ws = nullptr,
-             size_t ws_bytes = 0, StepChain chain = StepChain());
+             size_t ws_bytes = 0, StepChain *chain = nullptr);
 
 // S = X^T Y, k x k column-major FP64 (device)
 int launch_gram(ttdft_ctx ctx, const void *X, int64_t ldx, const void *Y, int64_t ldy,

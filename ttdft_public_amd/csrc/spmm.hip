@@ -1638,7 +1638,7 @@ static int launch_block_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X,
 int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, void *Y,
              int64_t ldy, const void *Z, int64_t ldz, int32_t k, int dtype, double alpha,
              double beta, double delta, int use_beta, int use_delta, void *ws,
-             size_t ws_bytes, StepChain chain) {
+             size_t ws_bytes, StepChain *chain) {
     const size_t es = dtype_size(dtype);
     const bool band = H->format == 1 && k >= 16 &&
                       (dtype == TTDFT_F64 ? H->mf64 != nullptr : H->mf32 != nullptr);
@@ -1674,9 +1674,9 @@ int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, vo
     else {
         // Partial sums and fragments of the split dense and the block product:
         // after the projections in the caller's work space, else from the
-        // context.  When the caller's work space cannot hold them the product
-        // runs in one kernel (no partial sums; the same result up to the order
-        // of the additions).
+        // context.  Where the caller's work space cannot hold them, or the
+        // context finds no memory, the product runs in one kernel (no partial
+        // sums; the same result up to the order of the additions).
         void *P = nullptr;
         if (blocks || (dense && dense_split(H->n, k, dtype))) {
             const size_t need_p =
@@ -1684,19 +1684,23 @@ int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, vo
             if (ws) {
                 const size_t off = W ? ((size_t)nl_workspace(H, k) * es + 255) / 256 * 256 : 0;
                 if (off + need_p <= ws_bytes) P = (char *)ws + off;
-            } else {
-                TT_TRY(ctx->scratch[8].ensure(need_p));
+            } else if (ctx->scratch[8].ensure(need_p) == TTDFT_OK) {
                 P = ctx->scratch[8].ptr;
+            } else {
+                clear_error();
             }
         }
+        StepChain now;  // what this step finds and is to leave
+        if (chain && P) now = *chain;
+        if (chain) chain->have = P && chain->want;
         const void *Zp = Z ? Z : Y;
         const int64_t ldzp = Z ? ldz : ldy;
         if (dense)
             TT_TRY(launch_dense_spmm(ctx, H, X, ldx, W, Y, ldy, Zp, ldzp, k, dtype, alpha, beta,
-                                     delta, use_beta, use_delta, P, chain));
+                                     delta, use_beta, use_delta, P, now));
         else if (blocks && P)
             TT_TRY(launch_block_spmm(ctx, H, X, ldx, W, Y, ldy, Zp, ldzp, k, dtype, alpha, beta,
-                                     delta, use_beta, use_delta, P, chain));
+                                     delta, use_beta, use_delta, P, now));
         else
             TT_TRY(launch_spmm_fused(ctx, H, X, ldx, W, Y, ldy, Zp, ldzp, k, dtype, alpha, beta,
                                      delta, use_beta, use_delta));
