@@ -191,9 +191,10 @@ int ttdft_ham_apply(ttdft_ctx ctx, ttdft_ham ham, const void *X, int64_t ldx,
  * capture, tight serving loops).  The nonlocal projections go to a static
  * device work space of 32 MiB per GPU (held until the process ends): the
  * call fails with TTDFT_EBADARG when p * k * (1 + splits) * sizeof(dtype)
- * exceeds it (k = 300 and p = 172 need at most 2.5 MB in FP64).  A product on
- * dense storage also keeps its partial sums there (4 n k doubles) when they
- * fit (n k up to about 1e6); above that it runs in one kernel, which agrees
+ * exceeds it (k = 300 and p = 172 need at most 2.5 MB in FP64).  The split
+ * products on dense storage and on CSR blocks keep X's operand fragments and up
+ * to 16 parts of partial sums there (n k numbers each); a call that has room for
+ * fewer parts than ttdft_ham_apply takes, or for none (one kernel then), agrees
  * with ttdft_ham_apply up to the order of the additions.  Every call on one
  * GPU shares that work space, so calls that overlap on one GPU (different
  * contexts or streams) race; calls on one context are stream-ordered and

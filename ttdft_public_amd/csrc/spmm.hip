@@ -1372,35 +1372,60 @@ static bool dense_split(int64_t n, int32_t k, int dtype) {
 // (each column streams H once).
 struct DenseTiling {
     int ncol, jt, nparts, chunk = 0;  // chunk: most blocks of a part (block product)
-    size_t partial_bytes, bytes;  // partial sums; with the fragments of X behind them
+    // one part's sums, all parts' (rounded up to 256 bytes), the fragments of X
+    // behind them, and the whole
+    size_t part_bytes, partial_bytes, fragment_bytes, bytes;
+    DenseTiling(const ttdft_ham_s *H, int32_t k, int dtype) {
+        ncol = (k + 95) / 96;
+        jt = (k + 16 * ncol - 1) / (16 * ncol);
+        part_bytes = (size_t)H->n * k * dtype_size(dtype);
+        fragment_bytes = (size_t)((H->n + kRingStep - 1) / kRingStep) * ncol * jt * 1024 *
+                         (dtype == TTDFT_F64 ? RingCfg<double>::PIECES : RingCfg<float>::PIECES);
+        set_parts(1);
+    }
+    void set_parts(int p) {
+        nparts = p;
+        partial_bytes = (p * part_bytes + 255) / 256 * 256;
+        bytes = partial_bytes + fragment_bytes;
+    }
+    // most parts that fit `limit` bytes with the fragments (0: none)
+    int parts_within(size_t limit) const {
+        if (limit < fragment_bytes + 256) return 0;
+        return (int)std::min<size_t>((limit - fragment_bytes - 255) / part_bytes, 1 << 20);
+    }
 };
-static DenseTiling dense_tiling(const ttdft_ham_s *H, int32_t k, int dtype) {
-    DenseTiling d;
-    d.ncol = (k + 95) / 96;
-    d.jt = (k + 16 * d.ncol - 1) / (16 * d.ncol);
+// (limit: bytes of work space; nparts is 0 where it holds no part)
+static DenseTiling dense_tiling(const ttdft_ham_s *H, int32_t k, int dtype,
+                                size_t limit = SIZE_MAX) {
+    DenseTiling d(H, k, dtype);
     const int rows = dtype == TTDFT_F64 ? ring_rows<double>() : ring_rows<float>();
     const int64_t nst = H->dense_ld / kRingStep, wgs = (H->n + rows - 1) / rows * d.ncol;
     // Parts of l: one workgroup fills a CU (its LDS stages), so parts p take
     // ceil(wgs p / 256) rounds of nst / p stages and about four to fill and
     // drain the ring; a part's sums cost n k / (64 rows) stages of the chip's
-    // bandwidth (written and read back).  The cheapest count is taken.
-    double best = 0.0;
-    d.nparts = 1;
+    // bandwidth (written and read back).  The cheapest count is taken.  Where
+    // the work space holds only dearer ones, the one-kernel form takes over from
+    // 1.25 times the cheapest on in FP64, 2.5 times in FP32 (8,000 and 15,625
+    // rows, 96 to 180 states: one kernel 1.4-1.6 and 1.9-3.3 times the split,
+    // half the parts 1.9 and 1.5 times).
+    const int within = d.parts_within(limit);
+    const int form = dense_split_form();
+    if (form > 1) {
+        d.set_parts((int)std::min<int64_t>({form, kDenseParts, nst, within}));
+        return d;
+    }
+    double best = 0.0, best_within = 0.0;
+    int nparts = 0;
     for (int p = 1; p <= kDenseParts && p <= nst; ++p) {
         const double cost = (double)((wgs * p + 255) / 256) * (double)((nst + p - 1) / p + 4) +
                             p * (double)H->n * k / (256.0 * 16 * rows);
-        if (p == 1 || cost < best) {
-            best = cost;
-            d.nparts = p;
+        if (p == 1 || cost < best) best = cost;
+        if (p <= within && (p == 1 || cost < best_within)) {
+            best_within = cost;
+            nparts = p;
         }
     }
-    const int form = dense_split_form();
-    if (form > 1) d.nparts = (int)std::min<int64_t>(std::min(form, kDenseParts), nst);
-    const size_t es = dtype_size(dtype);
-    d.partial_bytes = ((size_t)d.nparts * H->n * k * es + 255) / 256 * 256;
-    d.bytes = d.partial_bytes + (size_t)nst * d.ncol * d.jt * 1024 *
-                                    (dtype == TTDFT_F64 ? RingCfg<double>::PIECES
-                                                        : RingCfg<float>::PIECES);
+    d.set_parts(best_within <= (dtype == TTDFT_F64 ? 1.25 : 2.5) * best ? nparts : 0);
     return d;
 }
 
@@ -1408,7 +1433,8 @@ template <typename T, int JT>
 static void dense_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const T *Hd, const T *ctv,
                          const void *X, int64_t ldx, const void *W, void *Y, int64_t ldy,
                          const void *Z, int64_t ldz, int32_t k, double alpha, double beta,
-                         double delta, int use_beta, int use_delta, void *P, StepChain chain) {
+                         double delta, int use_beta, int use_delta, const DenseTiling &d, void *P,
+                         StepChain chain) {
     const int64_t n = H->n;
     const dim3 grid((unsigned)((n + 15) / 16), (unsigned)((k + 16 * JT - 1) / (16 * JT)));
     const int64_t *ctr = H->p > 0 && !H->dense_nl ? H->ct_rowptr : nullptr;
@@ -1418,7 +1444,6 @@ static void dense_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const T *Hd, const
     // 8,000 x 24 0.108 + 0.007 against 0.153.  TTDFT_DENSE_LDS=0 turns the split
     // off, 1 picks the form and the parts, 2..16 splits into that many.
     if (P) {
-        const DenseTiling d = dense_tiling(H, k, sizeof(T) == 8 ? TTDFT_F64 : TTDFT_F32);
         const int ntiles = d.ncol * JT;
         T *Pt = (T *)P, *F = (T *)((char *)P + d.partial_bytes);
         const unsigned cb = (unsigned)((H->dense_ld / 8 * k + 255) / 256);
@@ -1456,18 +1481,20 @@ static void dense_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const T *Hd, const
 static int launch_dense_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx,
                              const void *W, void *Y, int64_t ldy, const void *Z, int64_t ldz,
                              int32_t k, int dtype, double alpha, double beta, double delta,
-                             int use_beta, int use_delta, void *P, StepChain chain) {
-    const int jt = dense_tiling(H, k, dtype).jt;
+                             int use_beta, int use_delta, const DenseTiling &d, void *P,
+                             StepChain chain) {
 #define DENSE_CASE(JTV)                                                                         \
     case JTV:                                                                                   \
         if (dtype == TTDFT_F64)                                                                 \
             dense_launch<double, JTV>(ctx, H, H->dense64, H->ct_val64, X, ldx, W, Y, ldy, Z,    \
-                                      ldz, k, alpha, beta, delta, use_beta, use_delta, P, chain);      \
+                                      ldz, k, alpha, beta, delta, use_beta, use_delta, d, P,    \
+                                      chain);                                                   \
         else                                                                                    \
             dense_launch<float, JTV>(ctx, H, H->dense32, H->ct_val32, X, ldx, W, Y, ldy, Z,     \
-                                     ldz, k, alpha, beta, delta, use_beta, use_delta, P, chain);       \
+                                     ldz, k, alpha, beta, delta, use_beta, use_delta, d, P,     \
+                                     chain);                                                    \
         break;
-    switch (jt) {
+    switch (d.jt) {
         DENSE_CASE(1)
         DENSE_CASE(2)
         DENSE_CASE(3)
@@ -1567,17 +1594,17 @@ int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
 // longest list to kDenseParts parts: every part has a place for all rows, so
 // one full row tile in a sparse matrix would otherwise take gigabytes (200,000
 // rows x 64 states with 32 full rows: 91 GB).
-static DenseTiling block_tiling(const ttdft_ham_s *H, int32_t k, int dtype) {
-    DenseTiling d;
-    d.ncol = (k + 95) / 96;
-    d.jt = (k + 16 * d.ncol - 1) / (16 * d.ncol);
-    d.chunk = (int)std::max<int64_t>({(H->nblk * d.ncol + 4095) / 4096, 4,
-                                      (H->blk_most + kDenseParts - 1) / kDenseParts});
-    d.nparts = (int)((H->blk_most + d.chunk - 1) / d.chunk);
-    d.partial_bytes = ((size_t)d.nparts * H->n * k * dtype_size(dtype) + 255) / 256 * 256;
-    d.bytes = d.partial_bytes + (size_t)(dense_leading_dim(H->n) / 32) * d.ncol * d.jt * 1024 *
-                                    (dtype == TTDFT_F64 ? RingCfg<double>::PIECES
-                                                        : RingCfg<float>::PIECES);
+static DenseTiling block_tiling(const ttdft_ham_s *H, int32_t k, int dtype,
+                                size_t limit = SIZE_MAX) {
+    DenseTiling d(H, k, dtype);
+    const int64_t most = std::min(kDenseParts, d.parts_within(limit));
+    if (most < 1) {
+        d.set_parts(0);
+        return d;
+    }
+    d.chunk = (int)std::max<int64_t>(
+        {(H->nblk * d.ncol + 4095) / 4096, 4, (H->blk_most + most - 1) / most});
+    d.set_parts((int)((H->blk_most + d.chunk - 1) / d.chunk));
     return d;
 }
 
@@ -1607,8 +1634,8 @@ static void block_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const DenseTiling 
 static int launch_block_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx,
                              const void *W, void *Y, int64_t ldy, const void *Z, int64_t ldz,
                              int32_t k, int dtype, double alpha, double beta, double delta,
-                             int use_beta, int use_delta, void *P, StepChain chain) {
-    const DenseTiling d = block_tiling(H, k, dtype);
+                             int use_beta, int use_delta, const DenseTiling &d, void *P,
+                             StepChain chain) {
 #define BLOCK_CASE(JTV)                                                                        \
     case JTV:                                                                                  \
         if (dtype == TTDFT_F64)                                                                \
@@ -1673,18 +1700,19 @@ int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, vo
                                 alpha, beta, delta, use_beta, use_delta));
     else {
         // Partial sums and fragments of the split dense and the block product:
-        // after the projections in the caller's work space, else from the
-        // context.  Where the caller's work space cannot hold them, or the
-        // context finds no memory, the product runs in one kernel (no partial
-        // sums; the same result up to the order of the additions).
+        // after the projections in the caller's work space, in as many parts as
+        // that holds, else from the context.  Where the caller's work space
+        // holds no part, or the context finds no memory, the product runs in one
+        // kernel.  (The same result up to the order of the additions.)
         void *P = nullptr;
+        DenseTiling tiling(H, k, dtype);
         if (blocks || (dense && dense_split(H->n, k, dtype))) {
-            const size_t need_p =
-                blocks ? block_tiling(H, k, dtype).bytes : dense_tiling(H, k, dtype).bytes;
+            const size_t off = W ? ((size_t)nl_workspace(H, k) * es + 255) / 256 * 256 : 0;
+            const size_t limit = !ws ? SIZE_MAX : off < ws_bytes ? ws_bytes - off : 0;
+            tiling = blocks ? block_tiling(H, k, dtype, limit) : dense_tiling(H, k, dtype, limit);
             if (ws) {
-                const size_t off = W ? ((size_t)nl_workspace(H, k) * es + 255) / 256 * 256 : 0;
-                if (off + need_p <= ws_bytes) P = (char *)ws + off;
-            } else if (ctx->scratch[8].ensure(need_p) == TTDFT_OK) {
+                if (tiling.nparts > 0) P = (char *)ws + off;
+            } else if (ctx->scratch[8].ensure(tiling.bytes) == TTDFT_OK) {
                 P = ctx->scratch[8].ptr;
             } else {
                 clear_error();
@@ -1697,10 +1725,10 @@ int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, vo
         const int64_t ldzp = Z ? ldz : ldy;
         if (dense)
             TT_TRY(launch_dense_spmm(ctx, H, X, ldx, W, Y, ldy, Zp, ldzp, k, dtype, alpha, beta,
-                                     delta, use_beta, use_delta, P, now));
+                                     delta, use_beta, use_delta, tiling, P, now));
         else if (blocks && P)
             TT_TRY(launch_block_spmm(ctx, H, X, ldx, W, Y, ldy, Zp, ldzp, k, dtype, alpha, beta,
-                                     delta, use_beta, use_delta, P, now));
+                                     delta, use_beta, use_delta, tiling, P, now));
         else
             TT_TRY(launch_spmm_fused(ctx, H, X, ldx, W, Y, ldy, Zp, ldzp, k, dtype, alpha, beta,
                                      delta, use_beta, use_delta));
