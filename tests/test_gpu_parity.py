@@ -816,6 +816,49 @@ def csr_product(n, rowptr, col, val, X):
     return Y
 
 
+@pytest.mark.parametrize("form", ["blocks", "dense"])
+@pytest.mark.parametrize("dtype", [E.F64, E.F32])
+def test_split_products_keep_the_rows_infinities(ctx, monkeypatch, form, dtype):
+    """Infinities, NaN, the largest numbers and states 2^-115 small through the
+    block and the split dense product: every result is what the row's own
+    entries give (an infinite state reaches no row without an entry there, and
+    stays infinite), and a small state keeps its precision (rounding of sums of
+    `most` products in the type, 8 sqrt(most) eps)."""
+    npdt, eps = (np.float64, 2.0 ** -53) if dtype == E.F64 else (np.float32, 2.0 ** -24)
+    if form == "blocks":
+        n, most = 1000, 19
+        rowptr, col, val = banded_csr(n, 9, 11)
+    else:
+        n, most = 300, 300
+        rowptr, col = np.arange(n + 1, dtype=np.int64) * n, np.tile(np.arange(n, dtype=np.int32), n)
+        val = np.random.default_rng(12).standard_normal(n * n)
+        monkeypatch.setenv("TTDFT_DENSE_LDS", "2")
+    val = val.astype(npdt).astype(np.float64)
+    ham = E.Hamiltonian(ctx, n, rowptr, col, val, 0, None, None, None, None,
+                        copies=E.HAM_F64 if dtype == E.F64 else E.HAM_F32)
+    k = 40
+    X = np.random.default_rng(13).standard_normal((n, k)).astype(npdt)
+    X[n // 2, 3] = np.inf
+    X[n // 5, 5] = np.nan
+    X[n // 3, 7], X[n // 3 + 4, 7] = -np.inf, np.inf
+    X[n - 1, 9] = np.finfo(npdt).max
+    X[:, 11] *= npdt(2.0 ** -115)
+    dX, dY = dev(ctx, X, npdt), dev(ctx, np.full((n, k), 7.0), npdt)
+    ctx.ham_apply(ham, dX.ptr, k, dY.ptr, k, k, dtype)
+    with np.errstate(all="ignore"):
+        ref = csr_product(n, rowptr, col, val, X.astype(np.float64)).astype(npdt)
+    got = dY.to_host().reshape(n, k)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    assert np.array_equal(np.isfinite(got), np.isfinite(ref))
+    for c in range(k):
+        f = np.isfinite(ref[:, c])
+        g, r = got[f, c].astype(np.longdouble), ref[f, c].astype(np.longdouble)
+        if len(r):
+            assert np.abs(g - r).max() <= 8 * eps * np.sqrt(most) * np.abs(r).max(), c
+    ham.free()
+
+
 @pytest.mark.parametrize("copies", [E.HAM_F64, E.HAM_F32, E.HAM_F64 | E.HAM_F32])
 def test_csr_without_room_for_blocks(monkeypatch, copies):
     """Block storage (2.3 MB an FP64 copy here, 1.1 MB FP32) that finds no

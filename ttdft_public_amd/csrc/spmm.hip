@@ -428,7 +428,11 @@ __global__ __launch_bounds__(512) void dense_hx_kernel(
 // x2 = x - x0 - x1); the products h0 x0, h0 x1, h1 x0, h1 x1, h0 x2, h2 x0
 // on 16x16x32 BF16 MFMA with FP32 accumulation leave out terms below 2^-24 of
 // |h x|, the rounding of one FP32 product.  H stays in FP32 in memory and is
-// split in registers after the LDS read, X once per product.
+// split in registers after the LDS read, X once per product, times 2^16 so that
+// the third piece of every normal number is one too (H's entries keep their 24
+// bits from 2^-110 on).  A value that the pieces cannot hold (infinities, X from
+// 2^111 on) makes the sum infinite or NaN; dense_combine_kernel then adds up that
+// row again in plain FP32.
 //
 // dense_combine_kernel: Y = alpha (sum_p P[p] + C^T W) (+ beta X) (+ delta Z),
 // the parts summed in FP64 in a fixed order.
@@ -469,6 +473,9 @@ __device__ __forceinline__ void split_bf16(float x, float y, unsigned &a, unsign
                   ry - __builtin_bit_cast(float, b & 0xffff0000u));
 }
 
+// Factor of the FP32 fragments, undone where their sums are complete
+constexpr float kFragScale = 65536.0f;
+
 // Sign that FP32 fragments of stage `st` carry in state c, undone as the
 // stage's sums are added up: (-1)^c times stage_sign.  A BF16 product rounds
 // its aligned terms towards minus infinity, so without it every sum of small
@@ -489,14 +496,13 @@ __device__ __forceinline__ void store_fragment(const double (&y)[8], int64_t o, 
 __device__ __forceinline__ void store_fragment(const float (&y)[8], int64_t o, int c,
                                                int32_t ntiles, float *F) {
     uv4 a, b, d;
-    const unsigned flip = stage_flip(o >> 2) ^ ((unsigned)(c & 1) << 31);
-    auto signed_y = [&](int i) {
-        return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, y[i]) ^ flip);
-    };
+    const float scale =
+        __builtin_bit_cast(float, __builtin_bit_cast(unsigned, kFragScale) ^ stage_flip(o >> 2) ^
+                                      ((unsigned)(c & 1) << 31));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         unsigned p, q, r;
-        split_bf16(signed_y(2 * i), signed_y(2 * i + 1), p, q, r);
+        split_bf16(y[2 * i] * scale, y[2 * i + 1] * scale, p, q, r);
         a[i] = p;
         b[i] = q;
         d[i] = r;
@@ -773,15 +779,38 @@ __device__ __forceinline__ int block_parts(int64_t cnt, int32_t chunk) {
     return (int)((cnt + chunk - 1) / chunk);
 }
 
+// The matrix behind the partial sums as rows, for sums that are not finite: CSR,
+// or dense rows of leading dimension ldh (rowptr null).  val null: the partial
+// sums stand.
+template <typename T> struct RowSource {
+    const int64_t *rowptr;
+    const int32_t *col;
+    const T *val;
+    __device__ __forceinline__ double sum(int64_t r, int64_t n, int64_t ldh, const T *x,
+                                          int64_t ldx) const {
+        const int64_t e0 = rowptr ? rowptr[r] : r * ldh, e1 = rowptr ? rowptr[r + 1] : e0 + n;
+        T s = T(0);
+        for (int64_t e = e0; e < e1 && s == s; ++e)  // (a NaN stays)
+            s += val[e] * x[(rowptr ? (int64_t)col[e] : e - e0) * ldx];
+        return (double)s;
+    }
+};
+
 // One thread per eight rows of one state (the rows of a fragment entry).  With
 // blk_ptr the part count is that of the rows' block list (none: no sum).
+//
+// An infinity or NaN among the states reaches what the rows say: a block's
+// zeros times an infinity, or its BF16 pieces, would make NaN of rows without an
+// entry there and of infinite results.  Sums that are not finite are therefore
+// added up again from the matrix, one entry after the other.
 template <typename T>
 __global__ __launch_bounds__(256) void dense_combine_kernel(
     int64_t n, int64_t ldh, int32_t k, int32_t nparts, const T *__restrict__ P, const T *X,
     int64_t ldx, const int64_t *__restrict__ ct_rowptr, const int32_t *__restrict__ ct_col,
     const T *__restrict__ ct_val, const T *__restrict__ W, T *Y, int64_t ldy, const T *Z,
     int64_t ldz, double alpha, double beta, double delta, int use_beta, int use_delta,
-    int32_t ntiles, T *__restrict__ F, const int64_t *__restrict__ blk_ptr, int32_t chunk) {
+    int32_t ntiles, T *__restrict__ F, const int64_t *__restrict__ blk_ptr, int32_t chunk,
+    RowSource<T> rows) {
     // (fewer than 2^32 threads: k <= 1024, n < 2^25)
     const unsigned e = blockIdx.x * 256u + threadIdx.x;
     const unsigned oc = e / (unsigned)k;
@@ -820,6 +849,18 @@ __global__ __launch_bounds__(256) void dense_combine_kernel(
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 if (p + u < nparts) s[i] += (double)v[u][i];
+    }
+    if (rows.val) {
+        bool finite = true;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) finite = finite && __builtin_isfinite(s[i]);
+        if constexpr (sizeof(T) == 4)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s[i] *= 1.0 / kFragScale;
+        if (!finite)
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (!__builtin_isfinite(s[i])) s[i] = rows.sum(row(i), n, ldh, X + c, ldx);
     }
     if (ct_rowptr) {
         // entry t of all eight rows together: a row by itself is a serial chain
@@ -1457,7 +1498,8 @@ static void dense_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const T *Hd, const
         hipLaunchKernelGGL((dense_combine_kernel<T>), dim3(cb), dim3(256), 0, ctx->stream, n,
                            H->dense_ld, k, d.nparts, Pt, (const T *)X, ldx, ctr, H->ct_col, ctv,
                            (const T *)W, (T *)Y, ldy, (const T *)Z, ldz, alpha, beta, delta,
-                           use_beta, use_delta, ntiles, chain.want ? F : nullptr, nullptr, 0);
+                           use_beta, use_delta, ntiles, chain.want ? F : nullptr, nullptr, 0,
+                           RowSource<T>{nullptr, nullptr, sizeof(T) == 4 ? Hd : nullptr});
         return;
     }
     // six-state runs per lane, fetched as pairs, when every tile is full and
@@ -1609,8 +1651,8 @@ static DenseTiling block_tiling(const ttdft_ham_s *H, int32_t k, int dtype,
 }
 
 template <typename T, int JT>
-static void block_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const DenseTiling &d, const T *bval,
-                         const T *ctv, const void *X, int64_t ldx, const void *W, void *Y,
+static void block_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const DenseTiling &d, const T *val,
+                         const T *bval, const T *ctv, const void *X, int64_t ldx, const void *W, void *Y,
                          int64_t ldy, const void *Z, int64_t ldz, int32_t k, double alpha,
                          double beta, double delta, int use_beta, int use_delta, void *P,
                          StepChain chain) {
@@ -1628,7 +1670,7 @@ static void block_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const DenseTiling 
                        d.nparts, Pt, (const T *)X, ldx, H->p > 0 ? H->ct_rowptr : nullptr,
                        H->ct_col, ctv, (const T *)W, (T *)Y, ldy, (const T *)Z, ldz, alpha, beta,
                        delta, use_beta, use_delta, ntiles, chain.want ? F : nullptr, H->blk_ptr,
-                       d.chunk);
+                       d.chunk, RowSource<T>{H->rowptr, H->col, val});
 }
 
 static int launch_block_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx,
@@ -1639,12 +1681,12 @@ static int launch_block_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X,
 #define BLOCK_CASE(JTV)                                                                        \
     case JTV:                                                                                  \
         if (dtype == TTDFT_F64)                                                                \
-            block_launch<double, JTV>(ctx, H, d, H->blk64, H->ct_val64, X, ldx, W, Y, ldy, Z,  \
-                                      ldz, k, alpha, beta, delta, use_beta, use_delta, P,      \
+            block_launch<double, JTV>(ctx, H, d, H->val64, H->blk64, H->ct_val64, X, ldx, W, Y, \
+                                      ldy, Z, ldz, k, alpha, beta, delta, use_beta, use_delta, P,      \
                                       chain);                                                  \
         else                                                                                   \
-            block_launch<float, JTV>(ctx, H, d, H->blk32, H->ct_val32, X, ldx, W, Y, ldy, Z,   \
-                                     ldz, k, alpha, beta, delta, use_beta, use_delta, P,       \
+            block_launch<float, JTV>(ctx, H, d, H->val32, H->blk32, H->ct_val32, X, ldx, W, Y,  \
+                                     ldy, Z, ldz, k, alpha, beta, delta, use_beta, use_delta, P,       \
                                      chain);                                                   \
         break;
     switch (d.jt) {
