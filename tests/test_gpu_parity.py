@@ -743,12 +743,13 @@ def test_dense_product_row_blocks_and_parts(ctx, monkeypatch, n, k):
 
 @pytest.mark.parametrize("n,half", [(40, 2), (65, 4), (1030, 40), (1500, 9)])
 @pytest.mark.parametrize("k", [7, 8, 37, 96, 97])
-def test_csr_block_storage(ctx, n, half, k):
+def test_csr_block_storage(ctx, monkeypatch, n, half, k):
     """CSR matrices whose 32 x 32 blocks are at least a tenth full run by
     blocks from 8 states on: banded rows with holes (n past multiples of 16, 32
     and 1024, blocks cut by the last column), a duplicate entry, rows without
     entries, projectors, in a filter with its fused recurrence.  FP64 to 1e-13
     (sums of up to 81 products), FP32 to 8 steps of 2^-24 sqrt(81)."""
+    monkeypatch.setenv("TTDFT_CSR_BLOCKS", "1")
     rng = np.random.default_rng(n + k)
     i, j = np.indices((n, n))
     A = np.where((np.abs(i - j) <= half) & ((i * j) % 7 != 3), rng.standard_normal((n, n)), 0.0)
@@ -887,6 +888,36 @@ def test_csr_without_room_for_blocks(monkeypatch, copies):
         ham.free()
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("dtype,fewest", [(E.F64, 64), (E.F32, 128)])
+def test_csr_product_form_by_states(ctx, monkeypatch, dtype, fewest):
+    """Blocks just over a tenth full: few states go by blocks, from `fewest` on
+    (one more pass of the row kernel's 64 states or the blocks' 96 aside) by
+    rows, each with the bits of the form that the switch takes."""
+    n = 4000
+    rowptr, col, val = banded_csr(n, 6, 14)
+    rows, keep = np.repeat(np.arange(n), np.diff(rowptr)), np.arange(len(col)) % 9 != 0
+    rows, col, val = rows[keep], col[keep], val[keep]
+    rowptr = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))])
+    blocks = len(np.unique(rows // 32 * 125 + col // 32))
+    assert 0.1 < len(col) / (1024.0 * blocks) < 0.11
+    npdt = np.float64 if dtype == E.F64 else np.float32
+    ham = E.Hamiltonian(ctx, n, rowptr, col, val, 0, None, None, None, None,
+                        copies=E.HAM_F64 if dtype == E.F64 else E.HAM_F32)
+    for k in (8, 16, fewest):
+        X = np.random.default_rng(k).standard_normal((n, k)).astype(npdt)
+        dX, got = dev(ctx, X, npdt), {}
+        for form in (None, "0", "1"):
+            if form is not None:
+                monkeypatch.setenv("TTDFT_CSR_BLOCKS", form)
+            dY = E.DeviceArray(ctx, (n, k), npdt)
+            ctx.ham_apply(ham, dX.ptr, k, dY.ptr, k, k, dtype)
+            got[form] = dY.to_host()
+            monkeypatch.delenv("TTDFT_CSR_BLOCKS", raising=False)
+        assert not np.array_equal(got["0"], got["1"])
+        assert np.array_equal(got[None], got["0" if k == fewest else "1"]), k
+    ham.free()
 
 
 def test_csr_block_parts_are_bounded(monkeypatch):

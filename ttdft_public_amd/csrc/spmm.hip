@@ -913,9 +913,9 @@ __global__ __launch_bounds__(256) void dense_combine_kernel(
 //   FP32: two 1 KB pieces of four floats per lane, H[row][8 q + 4 i + 0..3],
 // row = lane % 16, q = lane / 16, as the fragments of X have them.
 //
-// The row kernel above gathers a whole row of X per entry (12,167 x 37, 690
+// The row kernel above gathers a whole row of X per entry (12,167 x 37, 836
 // entries a row: 359 us, bound by those gathers from L2); here an entry costs
-// its share of a block on the matrix cores.  One wave takes 32 rows' blocks,
+// its share of a block (18% full) on the matrix cores.  One wave takes 32 rows' blocks,
 // or a part of them, by 16 JT states: H from HBM and X from L2 both come
 // straight into registers as whole pieces, no LDS and no barrier, and
 // dense_combine_kernel finishes.  A part is at most `chunk` blocks, so that all
@@ -1563,13 +1563,11 @@ void drop_blocks(ttdft_ham_s *H) {
     H->nblk = 0;
 }
 
-// Blocks of a CSR H_loc when they are full enough.  Per entry the row kernel
-// takes 43 ps (up to 64 states), per 32 x 32 block the block kernel about
-// 1.7 ns for its 8 KB and 0.4 ns per 16 states: even at 7% of a block's 1,024
-// places.  Stored from 10% on, where the storage (8 bytes a place against 12
-// an entry) is at most 7 times that of the rows.  Only the precisions asked
-// for are built: a device assembly still holds its FP64 rows here when FP32
-// alone was.
+// Blocks of a CSR H_loc when they are full enough: from 10% of their places on,
+// where the products of most state counts gain (block_product_pays) and the
+// storage (8 bytes a place against 12 an entry) is at most 7 times that of the
+// rows.  Only the precisions asked for are built: a device assembly still holds
+// its FP64 rows here when FP32 alone was.
 static int try_build_blocks(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
     const int64_t n = H->n;
     const int64_t words = (n + 1023) / 1024, tiles = (n + kBlockRows - 1) / kBlockRows;
@@ -1631,11 +1629,34 @@ int build_blocks(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
     return TTDFT_OK;
 }
 
+// Does a product of k states run by blocks?  Both forms' times go with what they
+// read: the row kernel's with its entries, once per 64 states (FP64 33 ps each
+// time, FP32 12 ps and 9 ps each time), the block kernel's with its blocks, once
+// per column of at most 96 states, and their 16-state tiles (1.6 ns and 0.55 ns a
+// tile in FP64, 0.8 and 0.31 in FP32).  Measured, rows / blocks in us:
+//   15,625 rows, blocks 10% full: FP64 16 states 203 / 147, 64 207 / 225, 96
+//   385 / 347; FP32 16 147 / 83, 64 148 / 134, 128 179 / 230;
+//   21,952 rows, 16% full: FP64 64 609 / 401, 300 3,902 / 1,891; FP32 64
+//   426 / 243, 300 1,075 / 1,136;
+//   12,167 rows, 18% full: FP64 16 364 / 150, 300 1,806 / 854; FP32 16
+//   265 / 81, 300 701 / 463.
+// TTDFT_CSR_BLOCKS=0 takes the rows, 1 the blocks wherever they are stored.
+static bool block_product_pays(const ttdft_ham_s *H, int32_t k, int dtype) {
+    if (const char *env = std::getenv("TTDFT_CSR_BLOCKS")) return std::atoi(env) != 0;
+    const DenseTiling d(H, k, dtype);
+    const int nc = (k + 63) / 64;
+    const bool f64 = dtype == TTDFT_F64;
+    const double entry = f64 ? 0.033 * nc : 0.012 + 0.009 * nc;
+    const double block = d.ncol * (f64 ? 1.6 + 0.55 * d.jt : 0.8 + 0.31 * d.jt);
+    return entry * (double)H->nnz >= block * (double)H->nblk;
+}
+
 // State tiles, parts and work space of the block product: chunks of blocks for
-// about four waves per SIMD, four blocks at least, and as long as keeps the
-// longest list to kDenseParts parts: every part has a place for all rows, so
-// one full row tile in a sparse matrix would otherwise take gigabytes (200,000
-// rows x 64 states with 32 full rows: 91 GB).
+// about four waves per SIMD in FP64, two in FP32 (there the partial sums weigh
+// more: 12,167 x 64 119 us against 139), four blocks at least, and as long as
+// keeps the longest list to kDenseParts parts: every part has a place for all
+// rows, so one full row tile in a sparse matrix would otherwise take gigabytes
+// (200,000 rows x 64 states with 32 full rows: 91 GB).
 static DenseTiling block_tiling(const ttdft_ham_s *H, int32_t k, int dtype,
                                 size_t limit = SIZE_MAX) {
     DenseTiling d(H, k, dtype);
@@ -1644,8 +1665,9 @@ static DenseTiling block_tiling(const ttdft_ham_s *H, int32_t k, int dtype,
         d.set_parts(0);
         return d;
     }
+    const int64_t waves = dtype == TTDFT_F64 ? 4096 : 2048;
     d.chunk = (int)std::max<int64_t>(
-        {(H->nblk * d.ncol + 4095) / 4096, 4, (H->blk_most + most - 1) / most});
+        {(H->nblk * d.ncol + waves - 1) / waves, 4, (H->blk_most + most - 1) / most});
     d.set_parts((int)((H->blk_most + d.chunk - 1) / d.chunk));
     return d;
 }
@@ -1715,7 +1737,8 @@ int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, vo
                                                             : H->dense32 != nullptr);
     // (from 8 states on: below, a block's columns are mostly padding)
     const bool blocks = H->format == 0 && k >= 8 && k <= 1024 &&
-                        (dtype == TTDFT_F64 ? H->blk64 != nullptr : H->blk32 != nullptr);
+                        (dtype == TTDFT_F64 ? H->blk64 != nullptr : H->blk32 != nullptr) &&
+                        block_product_pays(H, k, dtype);
     void *W = nullptr;
     if (H->p > 0 && !(dense && H->dense_nl)) {  // folded into the dense storage otherwise
         const size_t need = (size_t)nl_workspace(H, k) * es;
