@@ -203,7 +203,9 @@ __global__ __launch_bounds__(256) void hloc_row_scan_kernel(const uint16_t *__re
 // the chip: the epilogue thresholds it, turns the keep bits into per-row
 // masks in LDS (wavefront ballots), and from the masks
 //   COUNT: cnt[row][y][z] = kept x of segment (pi, g);
-//          and the Kronecker half-bandwidths of the kept entries (flags[1..3]);
+//   COUNT_EXTENT: the same, and the Kronecker half-bandwidths of the kept entries
+//          (flags[1..3]), where n lets dense storage be chosen by them (they cost
+//          the pass 12% at 21,952 rows; elsewhere band_extent_kernel reads them);
 //   WRITE: each kept entry goes to rowptr[row] + rel[key] + (kept x' < x);
 //   DENSE: every entry goes to its place in the dense storage, 0 where it is
 //          dropped (13 atoms, n = 8,000: 205 us; the CSR arrays, their
@@ -223,7 +225,7 @@ struct FusedArgs {
     double *dense;   // dense storage, leading dimension dense_ld
     int64_t dense_ld;
 };
-enum { kCount = 0, kWrite = 1, kDense = 2 };
+enum { kCount = 0, kWrite = 1, kDense = 2, kCountExtent = 3 };
 
 typedef double fd4_t __attribute__((ext_vector_type(4)));
 
@@ -240,6 +242,20 @@ __device__ inline int mask_popc(const uint16_t *m, int lo, int hi) {
         c += __popc(bits);
     }
     return c;
+}
+
+// first and last bit of [lo, hi) that is set (one is)
+__device__ inline int mask_first(const uint16_t *m, int lo, int hi) {
+    int wi = lo >> 4;
+    unsigned w = m[wi] & (0xffffu << (lo & 15));
+    while (!w && 16 * (wi + 1) < hi) w = m[++wi];
+    return 16 * wi + __ffs(w) - 1;
+}
+__device__ inline int mask_last(const uint16_t *m, int lo, int hi) {
+    int wi = (hi - 1) >> 4;
+    unsigned w = m[wi] & (0xffffu >> (15 - ((hi - 1) & 15)));
+    while (!w && 16 * wi > lo) w = m[--wi];
+    return 16 * wi + 31 - __clz(w);
 }
 
 template <int PASS>
@@ -353,13 +369,12 @@ __global__ __launch_bounds__(256, 2) void hloc_fused_kernel(FusedArgs a) {
         const int yI = gy / a.ry, y = gy - yI * a.ry;
         const int64_t rowid = xI + (int64_t)a.rx * (yI + (int64_t)a.ry * zI);
         const int64_t key = (rowid * a.ry + y) * a.rz + z;
-        if (PASS == kCount) {
+        if (PASS != kWrite) {
             a.cnt[key] = (uint16_t)kept;
-            if (kept > 0) {
+            if (PASS == kCountExtent && kept > 0) {
                 const int lo = gl * a.rx;
-                int first = 0, last = a.rx - 1;
-                while (!(mask[r][(lo + first) >> 4] >> ((lo + first) & 15) & 1)) ++first;
-                while (!(mask[r][(lo + last) >> 4] >> ((lo + last) & 15) & 1)) --last;
+                const int first = mask_first(mask[r], lo, lo + a.rx) - lo;
+                const int last = mask_last(mask[r], lo, lo + a.rx) - lo;
                 ex = max(ex, max(xI - first, last - xI));
                 ey = max(ey, abs(y - yI));
                 ez = max(ez, abs(z - zI));
@@ -371,7 +386,8 @@ __global__ __launch_bounds__(256, 2) void hloc_fused_kernel(FusedArgs a) {
             segcnt[r * kFusedGt + gl] = min(kept, expect);
         }
     }
-    if (PASS == kCount) {
+    if (PASS == kCount) return;
+    if (PASS == kCountExtent) {
         for (int o = 32; o > 0; o >>= 1) {
             ex = max(ex, __shfl_xor(ex, o));
             ey = max(ey, __shfl_xor(ey, o));
@@ -720,13 +736,17 @@ int hloc_run(ttdft_ctx ctx, const HlocIn &a, bool fill, DevCsr &out, int ext[3],
                  "assemble_hloc: %lld workgroups exceed the grid limit",
                  (long long)fa.nblocks);
     }
+    // only a matrix of at most so many rows may go to dense storage
+    const bool extents = fused && dense && dense_storage_fits(n, n * n);
     auto run_pass = [&](int write, const int64_t *drowptr, int32_t *dcol, double *dval) -> int {
         if (fused) {
             FusedArgs f = fa;
             f.rowptr = drowptr;
             f.col = dcol;
             f.val = dval;
-            auto kern = write ? hloc_fused_kernel<kWrite> : hloc_fused_kernel<kCount>;
+            auto kern = write ? hloc_fused_kernel<kWrite>
+                              : extents ? hloc_fused_kernel<kCountExtent>
+                                        : hloc_fused_kernel<kCount>;
             hipLaunchKernelGGL(kern, dim3((unsigned)f.nblocks), dim3(256), 0, ctx->stream, f);
             TT_LAUNCH_CHECK();
             return TTDFT_OK;
@@ -787,9 +807,9 @@ int hloc_run(ttdft_ctx ctx, const HlocIn &a, bool fill, DevCsr &out, int ext[3],
     for (int64_t i = 0; i < n; ++i) out.rp[i + 1] = out.rp[i] + len[i];
     out.nnz = out.rp[n];
     if (!fill) return TTDFT_OK;
-    if (fused) {  // the count pass left the half-bandwidths
+    if (extents) {  // the count pass left the half-bandwidths
         for (int d = 0; d < 3; ++d) ext[d] = flags[1 + d];
-        if (dense && dense_storage_fits(n, out.nnz) &&
+        if (dense_storage_fits(n, out.nnz) &&
             !(ext[0] >= 0 && band_storage_fits(rx, ry, rz, ext[0], ext[1], ext[2], out.nnz))) {
             FusedArgs f = fa;
             f.dense_ld = dense_leading_dim(n);
@@ -810,7 +830,7 @@ int hloc_run(ttdft_ctx ctx, const HlocIn &a, bool fill, DevCsr &out, int ext[3],
     TT_TRY(timing_begin(ctx, TTDFT_KSTAT_ASSEMBLY, &tm));
     TT_TRY(run_pass(1, out.rowptr.as<int64_t>(), out.col.as<int32_t>(), out.val.as<double>()));
     TT_TRY(timing_end(ctx, &tm, 12.0 * out.nnz + 8.0 * (n + 1), flops));
-    if (!fused) {
+    if (!extents) {
         hipLaunchKernelGGL(band_extent_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0,
                            ctx->stream, out.rowptr.as<int64_t>(), out.col.as<int32_t>(), n, rx,
                            ry, dflag.as<int32_t>() + 1);
