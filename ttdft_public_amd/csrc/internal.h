@@ -146,7 +146,8 @@ struct ttdft_ham_s {
     // enough: block lists per 32 rows, column blocks, operand fragments
     int64_t nblk = 0, blk_most = 0;  // in all; most of a list
     int64_t *blk_ptr = nullptr;
-    int32_t *blk_col = nullptr;
+    int32_t *blk_col = nullptr, *blk_count = nullptr;
+    std::vector<int64_t> blk_ptr_host;
     double *blk64 = nullptr;
     float *blk32 = nullptr;
     // dense storage of H_loc (format 2) for small, nearly full matrices:

@@ -932,46 +932,73 @@ template <> __device__ __forceinline__ int block_slot<float>(int row, int l) {
 }
 
 // Blocks of one 32-row tile per workgroup: bit b of the LDS map is column
-// block b.  PASS 0 counts them; PASS 1 lists them and scatters the values
-// (duplicate entries add up, as in the row kernel).
+// block b.  PASS 0 counts them and notes (count negative) a row whose columns do
+// not ascend; PASS 1 lists them and scatters the values.  Duplicate entries add
+// up, as in the row kernel: with atomics, in tiles that may hold any.
+//
+// Bound by latency: a matrix of this size has a few hundred tiles.  Sixteen
+// waves take two rows each, and of a run of entries in one block only the first
+// sets the map's bit (12,167 rows x 836: count 29 us, FP64 blocks 173, FP32 127;
+// 64, 358 and 282 with four waves and atomics for every entry).  With the clear
+// and the host's wait for the count an FP64 assembly of that matrix takes 1.61 ms
+// in place of 1.25; two products of 37 states (0.19 in place of 0.36 ms each)
+// repay that.
+constexpr int kBuildThreads = 1024;
 template <int PASS, typename T>
-__global__ __launch_bounds__(256) void block_build_kernel(
+__global__ __launch_bounds__(kBuildThreads) void block_build_kernel(
     int64_t n, int32_t words, const int64_t *__restrict__ rowptr, const int32_t *__restrict__ col,
     const T *__restrict__ val, int32_t *__restrict__ count, const int64_t *__restrict__ ptr,
     int32_t *__restrict__ bcol, T *__restrict__ bval) {
+    constexpr int NW = kBuildThreads / 64;
     extern __shared__ unsigned block_map[];  // words map words, then their prefix counts
     unsigned *map = block_map, *pre = block_map + words;
-    __shared__ int total;
+    __shared__ int total, disorder;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int64_t tile = blockIdx.x;
-    for (int w = t; w < words; w += 256) map[w] = 0;
-    if (t == 0) total = 0;
+    for (int w = t; w < words; w += kBuildThreads) map[w] = 0;
+    if (t == 0) total = disorder = 0;
     __syncthreads();
-    for (int r = wave; r < kBlockRows; r += 4) {
+    for (int r = wave; r < kBlockRows; r += NW) {
         const int64_t row = kBlockRows * tile + r;
         if (row >= n) break;
-        for (int64_t e = rowptr[row] + lane; e < rowptr[row + 1]; e += 64)
-            atomicOr(&map[col[e] >> 10], 1u << ((col[e] >> 5) & 31));
+        const int64_t e1 = rowptr[row + 1];
+        int last = -1;  // column of the entry before the chunk's first
+        for (int64_t base = rowptr[row]; base < e1; base += 64) {
+            const bool on = base + lane < e1;
+            const int c = on ? col[base + lane] : 0;
+            int before = __shfl_up(c, 1);
+            if (lane == 0) before = last;
+            if (on && (before < 0 || (before >> 5) != (c >> 5)))
+                atomicOr(&map[c >> 10], 1u << ((c >> 5) & 31));
+            if (PASS == 0 && on && before >= c) disorder = 1;
+            last = __shfl(c, 63);
+        }
     }
     __syncthreads();
     if (PASS == 0) {
         int c = 0;
-        for (int w = t; w < words; w += 256) c += __popc(map[w]);
-        atomicAdd(&total, c);
+        for (int w = t; w < words; w += kBuildThreads) c += __popc(map[w]);
+        if (c) atomicAdd(&total, c);
         __syncthreads();
-        if (t == 0) count[tile] = total;
+        if (t == 0) count[tile] = disorder ? -total : total;
         return;
     }
-    if (t == 0) {
-        unsigned c = 0;
-        for (int w = 0; w < words; ++w) {
-            pre[w] = c;
-            c += __popc(map[w]);
+    if (wave == 0) {  // prefix counts, 64 words at a time
+        int sum = 0;
+        for (int w0 = 0; w0 < words; w0 += 64) {
+            const int w = w0 + lane, c = w < words ? __popc(map[w]) : 0;
+            int s = c;
+            for (int o = 1; o < 64; o *= 2) {
+                const int x = __shfl_up(s, o);
+                if (lane >= o) s += x;
+            }
+            if (w < words) pre[w] = sum + s - c;
+            sum += __shfl(s, 63);
         }
     }
     __syncthreads();
     const int64_t base = ptr[tile];
-    for (int w = t; w < words; w += 256) {
+    for (int w = t; w < words; w += kBuildThreads) {
         unsigned m = map[w];
         for (int64_t b = base + pre[w]; m; ++b) {
             const int bit = __ffs(m) - 1;
@@ -979,13 +1006,18 @@ __global__ __launch_bounds__(256) void block_build_kernel(
             bcol[b] = 32 * w + bit;
         }
     }
-    for (int r = wave; r < kBlockRows; r += 4) {
+    const bool add = count[tile] < 0;
+    for (int r = wave; r < kBlockRows; r += NW) {
         const int64_t row = kBlockRows * tile + r;
         if (row >= n) break;
         for (int64_t e = rowptr[row] + lane; e < rowptr[row + 1]; e += 64) {
             const int c = col[e], w = c >> 10, bit = (c >> 5) & 31;
             const int64_t b = base + pre[w] + __popc(map[w] & ((1u << bit) - 1u));
-            atomicAdd(bval + b * kBlockElems + block_slot<T>(r, c & 31), val[e]);
+            T *d = bval + b * kBlockElems + block_slot<T>(r, c & 31);
+            if (add)
+                atomicAdd(d, val[e]);
+            else
+                *d = val[e];
         }
     }
 }
@@ -1556,6 +1588,8 @@ void drop_blocks(ttdft_ham_s *H) {
     dev_release(H->ctx, H->blk_col);
     dev_release(H->ctx, H->blk64);
     dev_release(H->ctx, H->blk32);
+    dev_release(H->ctx, H->blk_count);
+    H->blk_count = nullptr;
     H->blk_ptr = nullptr;
     H->blk_col = nullptr;
     H->blk64 = nullptr;
@@ -1574,46 +1608,48 @@ static int try_build_blocks(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
     const bool f64 = H->val64 && (copies & TTDFT_HAM_F64);
     const bool f32 = H->val32 && (copies & TTDFT_HAM_F32);
     if (H->format != 0 || (!f64 && !f32) || H->nnz < 1 || words > 4096) return TTDFT_OK;
-    int32_t *dcount = nullptr;
-    TT_TRY(dev_alloc(ctx, (void **)&dcount, sizeof(int32_t) * tiles));
+    TT_TRY(dev_alloc(ctx, (void **)&H->blk_count, sizeof(int32_t) * tiles));
     const size_t lds = sizeof(unsigned) * 2 * (size_t)words;
-    hipLaunchKernelGGL((block_build_kernel<0, double>), dim3((unsigned)tiles), dim3(256), lds,
-                       ctx->stream, n, (int32_t)words, H->rowptr, H->col, nullptr, dcount,
-                       nullptr, nullptr, nullptr);
+    const dim3 grid((unsigned)tiles), block(kBuildThreads);
+    hipLaunchKernelGGL((block_build_kernel<0, double>), grid, block, lds, ctx->stream, n,
+                       (int32_t)words, H->rowptr, H->col, nullptr, H->blk_count, nullptr, nullptr,
+                       nullptr);
+    TT_LAUNCH_CHECK();
     std::vector<int32_t> cnt(tiles);
-    std::vector<int64_t> ptr(tiles + 1, 0);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(cnt.data(), dcount, sizeof(int32_t) * tiles, hipMemcpyDeviceToHost,
-                           ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    dev_release(ctx, dcount);
-    TT_CHECK(e == hipSuccess, TTDFT_EHIP, "build_blocks: %s", hipGetErrorString(e));
-    for (int64_t t = 0; t < tiles; ++t) ptr[t + 1] = ptr[t] + cnt[t];
-    H->blk_most = *std::max_element(cnt.begin(), cnt.end());
+    TT_HIP(hipMemcpyAsync(cnt.data(), H->blk_count, sizeof(int32_t) * tiles,
+                          hipMemcpyDeviceToHost, ctx->stream));
+    TT_HIP(hipStreamSynchronize(ctx->stream));
+    std::vector<int64_t> &ptr = H->blk_ptr_host;  // (read by the copy below after the return)
+    ptr.assign(tiles + 1, 0);
+    for (int64_t t = 0; t < tiles; ++t) {
+        const int64_t c = std::abs(cnt[t]);
+        ptr[t + 1] = ptr[t] + c;
+        H->blk_most = std::max(H->blk_most, c);
+    }
     const int64_t nblk = ptr[tiles];
     if ((double)H->nnz < 0.1 * kBlockElems * (double)nblk ||
-        8.0 * kBlockElems * (double)nblk > kDenseMaxBytes)
+        8.0 * kBlockElems * (double)nblk > kDenseMaxBytes) {
+        drop_blocks(H);
         return TTDFT_OK;
+    }
     H->nblk = nblk;
     TT_TRY(dev_alloc(ctx, (void **)&H->blk_ptr, sizeof(int64_t) * (tiles + 1)));
     TT_TRY(dev_alloc(ctx, (void **)&H->blk_col, sizeof(int32_t) * nblk));
     TT_HIP(hipMemcpyAsync(H->blk_ptr, ptr.data(), sizeof(int64_t) * (tiles + 1),
                           hipMemcpyHostToDevice, ctx->stream));
-    TT_HIP(hipStreamSynchronize(ctx->stream));  // ptr goes out of scope
     if (f64) {
         TT_TRY(dev_alloc(ctx, (void **)&H->blk64, sizeof(double) * kBlockElems * nblk));
         TT_HIP(hipMemsetAsync(H->blk64, 0, sizeof(double) * kBlockElems * nblk, ctx->stream));
-        hipLaunchKernelGGL((block_build_kernel<1, double>), dim3((unsigned)tiles), dim3(256), lds,
-                           ctx->stream, n, (int32_t)words, H->rowptr, H->col, H->val64, nullptr,
-                           H->blk_ptr, H->blk_col, H->blk64);
+        hipLaunchKernelGGL((block_build_kernel<1, double>), grid, block, lds, ctx->stream, n,
+                           (int32_t)words, H->rowptr, H->col, H->val64, H->blk_count, H->blk_ptr,
+                           H->blk_col, H->blk64);
     }
     if (f32) {
         TT_TRY(dev_alloc(ctx, (void **)&H->blk32, sizeof(float) * kBlockElems * nblk));
         TT_HIP(hipMemsetAsync(H->blk32, 0, sizeof(float) * kBlockElems * nblk, ctx->stream));
-        hipLaunchKernelGGL((block_build_kernel<1, float>), dim3((unsigned)tiles), dim3(256), lds,
-                           ctx->stream, n, (int32_t)words, H->rowptr, H->col, H->val32, nullptr,
-                           H->blk_ptr, H->blk_col, H->blk32);
+        hipLaunchKernelGGL((block_build_kernel<1, float>), grid, block, lds, ctx->stream, n,
+                           (int32_t)words, H->rowptr, H->col, H->val32, H->blk_count, H->blk_ptr,
+                           H->blk_col, H->blk32);
     }
     TT_LAUNCH_CHECK();
     return TTDFT_OK;
