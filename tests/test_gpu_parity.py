@@ -983,6 +983,29 @@ def test_filter_without_room_for_partial_sums(monkeypatch, form):
     assert np.array_equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("dtype", [E.F64, E.F32])
+@pytest.mark.parametrize("k,blocks", [(64, 2), (48, 3), (102, 2)])
+def test_band_filter_in_column_blocks(ctx, dtype, k, blocks):
+    """A band filter in column blocks narrower than the kernel's state tiles (32,
+    16 and 51 states): blocks past the first start inside the rows, and the
+    last one's rows end where the block's memory ends (2 MiB to the byte for
+    4,096 x 64 FP64).  Against the filter in one block and the oracle's."""
+    s = E.SynthHam(16, 16, 16, 3, 3, 3, 4, seed=51)
+    ham = ctx.ham_upload(s, E.HAM_F64 | E.HAM_F32, tucker=True)
+    assert ham.format()[0] == 1
+    npdt = np.float64 if dtype == E.F64 else np.float32
+    X = np.random.default_rng(k).standard_normal((s.n, k)).astype(npdt)
+    got = []
+    for b in (1, blocks):
+        dX = dev(ctx, X, npdt)
+        ctx.cheb_filter(ham, dX.ptr, k, k, 6, -0.5, 30.0, -3.0, b, dtype)
+        got.append(dX.to_host())
+    assert rel(got[1].astype(np.float64), got[0].astype(np.float64)) < 10 * np.finfo(npdt).eps
+    ref = oracle.cheb_filter(oracle.Ham.from_synth(s), X.astype(np.float64), 6, -0.5, 30.0, -3.0, 1)
+    assert rel(got[1].astype(np.float64), ref) < (1e-12 if dtype == E.F64 else 5e-5)
+    ham.free()
+
+
 def test_dense_storage_reuse_across_hamiltonians(ctx):
     """Hamiltonians of different sizes built and freed in turn on one context:
     the dense storage and the projector fold come from the context's block

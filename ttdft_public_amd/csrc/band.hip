@@ -280,9 +280,13 @@ __global__ __launch_bounds__(G > 1 ? 64 * G * GXM : 1024) void brick_spmm_kernel
     // q = wl + i nw (i < NQ; past the last chunk it repeats the last one,
     // which writes the same bytes again).  A lane's byte offset inside the
     // line of X is the same for every line: computed once.  Rows outside
-    // 0..rx-1 and states past the end load clamped, finite values; the A
+    // 0..rx-1 and states past the last load clamped, finite values; the A
     // fragments are zero against those rows and those states are never
-    // stored.
+    // stored.  The last state, not the row's end, is the limit: X may start at a
+    // column of a wider block, whose last row ends that much earlier.  (The last
+    // lane-load may pass state k - 1, but as rows are whole numbers of loads
+    // where it holds more than one state, not the row.)
+    const int smax = (a.k - 1) / VE * VE;
     int32_t goff[NQ];
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
@@ -294,7 +298,7 @@ __global__ __launch_bounds__(G > 1 ? 64 * G * GXM : 1024) void brick_spmm_kernel
         const int xp = xw0 + row;
         const int xpc = xp < 0 ? 0 : (xp >= a.rx ? a.rx - 1 : xp);
         int st = s0 + s;
-        if (st > (int)a.ldx - VE) st = (int)a.ldx - VE;
+        if (st > smax) st = smax;
         goff[i] = (xpc * (int)a.ldx + st) * ES + (off % ES);
     }
     auto line_of = [&](int li_, int &yy, int &zz) {
