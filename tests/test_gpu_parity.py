@@ -675,24 +675,30 @@ def test_dense_storage_matches_oracle(ctx, tucker):
     assert rel(dX.to_host().astype(np.float64), ref) < 5e-5
 
 
+@pytest.mark.parametrize("form", ["0", "-1", "3"])
 @pytest.mark.parametrize("dims", [(4, 3, 5), (9, 8, 7), (11, 10, 13)])
 @pytest.mark.parametrize("k", [1, 8, 16, 24, 33, 64, 80, 96, 100, 150, 192])
-def test_dense_product_tilings(ctx, dims, k):
+def test_dense_product_tilings(ctx, monkeypatch, dims, k, form):
     """The dense product over its state tilings (16 to 96 states per
     workgroup, one or two workgroup columns, partial tiles), leading dimension
-    of the block above k, and n
-    not a multiple of 32 (n = 60: six of the eight waves get no l range;
-    n = 1430: the last wave's range is shorter)."""
+    of the block above k, and n not a multiple of 32, in one kernel (n = 60: six
+    of the eight waves get no l range; n = 1430: the last wave's range is
+    shorter) and split into one part of up to 45 stages and into three (n = 60:
+    two).  An FP32-only matrix keeps its projectors apart."""
     rx, ry, rz = dims
     s = E.SynthHam(rx, ry, rz, rx - 1, ry - 1, rz - 1, 3, seed=k)
     H = oracle.Ham.from_synth(s)
-    ham = ctx.ham_upload(s, E.HAM_F64 | E.HAM_F32, tucker=False)
-    assert ham.format()[0] == 2
-    print(f"dense product n={s.n} k={k}", flush=True)
+    monkeypatch.setenv("TTDFT_DENSE_LDS", form)
+    print(f"dense product n={s.n} k={k} form={form}", flush=True)
     # an odd and an even leading dimension (96-state multiples with an even
     # one take the six-consecutive-states layout)
-    for ld, dtype, npdt, tol in ((k + 3, E.F64, np.float64, 1e-13), (k + 3, E.F32, np.float32, 1e-5),
-                                 (k + 4, E.F64, np.float64, 1e-13), (k + 4, E.F32, np.float32, 1e-5)):
+    for copies, ld, dtype, npdt, tol in (
+            (E.HAM_F64 | E.HAM_F32, k + 3, E.F64, np.float64, 1e-13),
+            (E.HAM_F64 | E.HAM_F32, k + 3, E.F32, np.float32, 1e-5),
+            (E.HAM_F64, k + 4, E.F64, np.float64, 1e-13),
+            (E.HAM_F32, k + 4, E.F32, np.float32, 1e-5)):
+        ham = ctx.ham_upload(s, copies, tucker=False)
+        assert ham.format()[0] == 2
         X = np.random.default_rng(k).standard_normal((s.n, ld)).astype(npdt)
         dX, dY = dev(ctx, X, npdt), dev(ctx, np.full((s.n, ld), 7.0), npdt)
         ctx.ham_apply(ham, dX.ptr, ld, dY.ptr, ld, k, dtype)
@@ -700,6 +706,7 @@ def test_dense_product_tilings(ctx, dims, k):
         ref = oracle.ham_apply(H, X[:, :k].astype(np.float64))
         assert rel(Y[:, :k], ref) < tol
         assert np.all(Y[:, k:] == 7.0)  # columns past k untouched
+        ham.free()
 
 
 @pytest.mark.parametrize("n", [1, 31, 33, 127, 129, 255, 257, 300])
@@ -732,7 +739,7 @@ def test_dense_product_row_blocks_and_parts(ctx, monkeypatch, n, k):
             nxt = 1.0 / (gamma - sigma)
             prev, cur = cur, (2 * nxt / e) * (A_c @ cur - c * cur) - sigma * nxt * prev
             sigma = nxt
-        for parts in ("1", "2", "3"):
+        for parts in ("-1", "2", "3"):
             monkeypatch.setenv("TTDFT_DENSE_LDS", parts)
             dX = dev(ctx, Xc, npdt)
             print(f"dense row blocks n={n} k={k} dtype={dtype} parts={parts}", flush=True)
@@ -741,58 +748,81 @@ def test_dense_product_row_blocks_and_parts(ctx, monkeypatch, n, k):
     ham.free()
 
 
-@pytest.mark.parametrize("n,half", [(40, 2), (65, 4), (1030, 40), (1500, 9)])
-@pytest.mark.parametrize("k", [7, 8, 37, 96, 97])
-def test_csr_block_storage(ctx, monkeypatch, n, half, k):
-    """CSR matrices whose 32 x 32 blocks are at least a tenth full run by
-    blocks from 8 states on: banded rows with holes (n past multiples of 16, 32
-    and 1024, blocks cut by the last column), a duplicate entry, rows without
-    entries, projectors, in a filter with its fused recurrence.  FP64 to 1e-13
-    (sums of up to 81 products), FP32 to 8 steps of 2^-24 sqrt(81)."""
+@pytest.mark.parametrize("n", [40, 65, 1030, 1500])
+@pytest.mark.parametrize("k", [7, 8, 17, 37, 80, 96, 97])
+def test_csr_block_storage(ctx, monkeypatch, n, k):
+    """CSR matrices whose 32 x 32 blocks are at least a tenth full, by blocks
+    from 8 states on: one and two clumps in a matrix of two and three row tiles,
+    one of them empty or of one row (n = 40, 65); bands with holes, a row and a
+    whole row tile without entries, n past multiples of 16, 32 and 1024, blocks
+    cut by the last column (1030); full rows in one tile, 12 parts of partial
+    sums (1500); a duplicate entry, a row whose columns descend, projectors; a
+    filter with its fused recurrence, leading dimension above k.  FP64 to 1e-13
+    (sums of `most` products), FP32 to 8 steps of 2^-24 sqrt(most)."""
     monkeypatch.setenv("TTDFT_CSR_BLOCKS", "1")
     rng = np.random.default_rng(n + k)
     i, j = np.indices((n, n))
-    A = np.where((np.abs(i - j) <= half) & ((i * j) % 7 != 3), rng.standard_normal((n, n)), 0.0)
-    A = np.triu(A) + np.triu(A, 1).T
-    A[5], A[:, 5] = 0.0, 0.0  # a row without entries
+    if n < 100:
+        on = ((i < 16) & (j < 16)) | ((n > 64) & (i // 16 == 2) & (j // 16 == 2)) | \
+            ((n > 64) & (i == 64) & (j == 64))
+    else:
+        on = (np.abs(i - j) <= (40 if n == 1030 else 9)) & ((i * j) % 7 != 3)
+        on &= (i != 5) & (j != 5)
+        on &= (i // 32 != 4) & (j // 32 != 4)
+        on |= (n == 1500) & (i // 8 == 9)
+    A = np.where(on, rng.standard_normal((n, n)), 0.0)
+    most = int(on.sum(1).max())
     rowptr, col, val = [0], [], []
     for r in range(n):
-        c = np.nonzero(A[r])[0]
+        c = np.nonzero(on[r])[0]
         v = A[r, c]
         if r == 3:  # its first entry in two parts
             c, v = np.insert(c, 0, c[0]), np.insert(v, 0, 0.25)
             v[1] -= 0.25
+        if r == 9 or r == n - 2:
+            c, v = c[::-1], v[::-1]
         col += c.tolist()
         val += v.tolist()
         rowptr.append(len(col))
-    assert len(col) < 0.2 * n * n
+    col = np.array(col, np.int32)
+    tiles = np.repeat(np.arange(n), np.diff(rowptr)) // 32
+    blocks = np.unique(tiles * 100 + col // 32)
+    assert 0.1 * 1024 * len(blocks) <= len(col) < 0.2 * n * n
+    assert n == 65 or len(np.unique(tiles)) < (n + 31) // 32  # an empty tile
+    # (a part holds four blocks at least)
+    assert n != 1500 or np.bincount(blocks // 100).max() > 44
     C = np.zeros((2, n))
     C[0, :9], C[1, n // 2:n // 2 + 5] = 0.3, -0.2
     cc = [np.nonzero(C[q])[0] for q in range(2)]
     inv = np.array([0.7, -0.4])
-    ham = E.Hamiltonian(ctx, n, np.array(rowptr), np.array(col, np.int32), np.array(val), 2,
+    ham = E.Hamiltonian(ctx, n, np.array(rowptr), col, np.array(val), 2,
                         np.array([0, len(cc[0]), len(cc[0]) + len(cc[1])]),
                         np.concatenate(cc).astype(np.int32),
                         np.concatenate([C[0, cc[0]], C[1, cc[1]]]), inv,
                         copies=E.HAM_F64 | E.HAM_F32)
+    assert ham.format()[0] == 0
     H = A + C.T @ (inv[:, None] * C)
-    X = rng.standard_normal((n, k))
+    ld = k + 3
+    X = rng.standard_normal((n, ld))
     a, b, a0 = -2.0, 30.0, -10.0
     e, c0 = (b - a) / 2, (b + a) / 2
-    for dtype, npdt, tol in ((E.F64, np.float64, 1e-13), (E.F32, np.float32, 8 * 2.0 ** -24 * 9)):
+    for dtype, npdt, tol in ((E.F64, np.float64, 1e-13),
+                             (E.F32, np.float32, 8 * 2.0 ** -24 * np.sqrt(most))):
         Xc = X.astype(npdt)
         sigma = e / (a0 - c0)
         gamma = 2.0 / sigma
-        prev = Xc.astype(np.float64)
+        prev = Xc[:, :k].astype(np.float64)
         cur = (sigma / e) * (H @ prev - c0 * prev)
         for _ in range(2, 5):
             nxt = 1.0 / (gamma - sigma)
             prev, cur = cur, (2 * nxt / e) * (H @ cur - c0 * cur) - sigma * nxt * prev
             sigma = nxt
         dX = dev(ctx, Xc, npdt)
-        print(f"csr blocks n={n} half={half} k={k} dtype={dtype}", flush=True)
-        ctx.cheb_filter(ham, dX.ptr, k, k, 5, a, b, a0, 1, dtype)
-        assert rel(dX.to_host().astype(np.float64), cur) < tol
+        print(f"csr blocks n={n} k={k} dtype={dtype}", flush=True)
+        ctx.cheb_filter(ham, dX.ptr, ld, k, 5, a, b, a0, 1, dtype)
+        got = dX.to_host().reshape(n, ld)
+        assert rel(got[:, :k].astype(np.float64), cur) < tol
+        assert np.array_equal(got[:, k:], Xc[:, k:])
     ham.free()
 
 

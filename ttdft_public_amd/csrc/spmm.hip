@@ -1418,8 +1418,8 @@ int finish_dense(ttdft_ctx ctx, ttdft_ham_s *H, int copies) {
 
 constexpr int kDenseParts = 16;  // most parts of the split dense and the block product
 
-// 0: one-kernel dense product; 1: form and parts picked; 2..16: split product
-// with that many parts
+// 0: one-kernel dense product; 1: form and parts picked; 2..16 and -1..-16:
+// split product with that many parts
 static int dense_split_form() {
     const char *env = std::getenv("TTDFT_DENSE_LDS");
     return env ? std::atoi(env) : 1;
@@ -1435,7 +1435,7 @@ static int dense_split_form() {
 // 2,744 x 90: 375 / 308; 4,096 x 30: 200 / 245; 8,000 x 24: 739 / 473.
 static bool dense_split(int64_t n, int32_t k, int dtype) {
     const int form = dense_split_form();
-    if (form != 1) return form > 1;
+    if (form != 1) return form != 0;
     const bool f64 = dtype == TTDFT_F64;
     return n > (k <= (f64 ? 32 : 48) ? 4096 : (f64 ? 1024 : 1728));
 }
@@ -1483,8 +1483,8 @@ static DenseTiling dense_tiling(const ttdft_ham_s *H, int32_t k, int dtype,
     // half the parts 1.9 and 1.5 times).
     const int within = d.parts_within(limit);
     const int form = dense_split_form();
-    if (form > 1) {
-        d.set_parts((int)std::min<int64_t>({form, kDenseParts, nst, within}));
+    if (form != 1) {
+        d.set_parts((int)std::min<int64_t>({std::abs(form), kDenseParts, nst, within}));
         return d;
     }
     double best = 0.0, best_within = 0.0;
@@ -1515,7 +1515,7 @@ static void dense_launch(ttdft_ctx ctx, const ttdft_ham_s *H, const T *Hd, const
     // and callers whose work space cannot hold the partial sums: FP32
     // 27,000 x 96 0.84 + 0.03 (sum of the parts) against 2.54 ms, FP64
     // 8,000 x 24 0.108 + 0.007 against 0.153.  TTDFT_DENSE_LDS=0 turns the split
-    // off, 1 picks the form and the parts, 2..16 splits into that many.
+    // off, 1 picks the form and the parts, 2..16 and -1..-16 split into that many.
     if (P) {
         const int ntiles = d.ncol * JT;
         T *Pt = (T *)P, *F = (T *)((char *)P + d.partial_bytes);
