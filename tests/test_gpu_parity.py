@@ -1014,6 +1014,30 @@ def test_filter_without_room_for_partial_sums(monkeypatch, form):
 
 
 @pytest.mark.parametrize("dtype", [E.F64, E.F32])
+@pytest.mark.parametrize("p", [4, 60])
+@pytest.mark.parametrize("bx,k,ld", [(3, 300, 300), (3, 250, 251), (7, 260, 260)])
+def test_band_epilogue_over_projector_rows(ctx, dtype, p, bx, k, ld):
+    """The state-group forms of the band product (aligned rows, unaligned rows,
+    the widest band) with rows of up to four entries of C^T on average and with
+    more, in a filter, so that the recurrence is in the epilogue too."""
+    s = E.SynthHam(18, 10, 9, bx, 3, 3, p, seed=61)
+    assert (s.nnz_c > 4 * s.n) == (p == 60)
+    ham = ctx.ham_upload(s, E.HAM_F64 | E.HAM_F32, tucker=True)
+    assert ham.format()[0] == 1
+    npdt, tol = (np.float64, 1e-12) if dtype == E.F64 else (np.float32, 5e-5)
+    X = np.random.default_rng(k).standard_normal((s.n, ld)).astype(npdt)
+    dX = dev(ctx, X, npdt)
+    ctx.cheb_filter(ham, dX.ptr, ld, k, 4, -0.5, 30.0, -3.0, 1, dtype)
+    got = dX.to_host().reshape(s.n, ld)
+    ref = oracle.cheb_filter(oracle.Ham.from_synth(s),
+                             np.ascontiguousarray(X[:, :k]).astype(np.float64), 4, -0.5, 30.0,
+                             -3.0, 1)
+    assert rel(got[:, :k].astype(np.float64), ref) < tol
+    assert np.array_equal(got[:, k:], X[:, k:])
+    ham.free()
+
+
+@pytest.mark.parametrize("dtype", [E.F64, E.F32])
 @pytest.mark.parametrize("k,blocks", [(64, 2), (48, 3), (102, 2)])
 def test_band_filter_in_column_blocks(ctx, dtype, k, blocks):
     """A band filter in column blocks narrower than the kernel's state tiles (32,

@@ -81,6 +81,8 @@ struct BrickArgs {
     T alpha, beta, delta;
     int use_beta, use_delta;
     int32_t light_last;  // ragged last x-chunk's units after all full ones, per XCD
+    int32_t slast;       // state where the last lane-load of a row starts
+    int32_t long_rows;   // rows of C^T have more than a few entries
 };
 
 // N LDS loads of T from byte offsets OFF0 + i STRIDE past p, completed inside
@@ -168,7 +170,10 @@ __device__ __forceinline__ void lds_read_n(const T *p, T (&v)[N]) {
 // halves.  A line only a plane outside the band of z' is skipped for that
 // plane; each plane sees its lines in the same order as with ZB = 1, so
 // the sums are bitwise the same.
-template <typename T, int KS, int NST, int DB, int DEPTH, int GXM, int G, int ZB = 1>
+// TILES: the epilogue finishes one state tile at a time (rows of C^T with few
+// entries; see there).
+template <typename T, int KS, int NST, int DB, int DEPTH, int GXM, int G, int ZB = 1,
+          bool TILES = false>
 __global__ __launch_bounds__(G > 1 ? 64 * G * GXM : 1024) void brick_spmm_kernel(BrickArgs<T> a) {
     typedef typename Acc4<T>::type acc_t;
     constexpr int S = 16 * NST;                  // states per wave
@@ -286,7 +291,6 @@ __global__ __launch_bounds__(G > 1 ? 64 * G * GXM : 1024) void brick_spmm_kernel
     // column of a wider block, whose last row ends that much earlier.  (The last
     // lane-load may pass state k - 1, but as rows are whole numbers of loads
     // where it holds more than one state, not the row.)
-    const int smax = (a.k - 1) / VE * VE;
     int32_t goff[NQ];
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
@@ -298,7 +302,7 @@ __global__ __launch_bounds__(G > 1 ? 64 * G * GXM : 1024) void brick_spmm_kernel
         const int xp = xw0 + row;
         const int xpc = xp < 0 ? 0 : (xp >= a.rx ? a.rx - 1 : xp);
         int st = s0 + s;
-        if (st > smax) st = smax;
+        if (st > a.slast) st = a.slast;
         goff[i] = (xpc * (int)a.ldx + st) * ES + (off % ES);
     }
     auto line_of = [&](int li_, int &yy, int &zz) {
@@ -486,6 +490,9 @@ __global__ __launch_bounds__(G > 1 ? 64 * G * GXM : 1024) void brick_spmm_kernel
     // tiles, so a step of that serial chain (entry, then its rows of W) loads
     // NST values and the row's next entry together (172 atoms, 172
     // projectors: FP64 product 7.07 -> 6.08 ms, FP32 4.35 -> 3.49).
+    // With TILES a tile at a time: the compiler unrolls over the entries and
+    // stays within 64 registers, as the joint walk does, but not both in one
+    // kernel (108).
 #pragma unroll
     for (int zi = 0; zi < ZB; ++zi) {
         const int z = z0 + zi;
@@ -496,6 +503,24 @@ __global__ __launch_bounds__(G > 1 ? 64 * G * GXM : 1024) void brick_spmm_kernel
             const int x = 4 * g + (i & 3), y = y0 + (i >> 2);
             if (x >= a.rx || y >= a.ry) continue;
             const int64_t row = x + (int64_t)a.rx * (y + (int64_t)a.ry * z);
+            if constexpr (TILES) {
+#pragma unroll
+                for (int st = 0; st < NST; ++st) {
+                    const int sc = s0 + sgw * S + 16 * st + li;
+                    if (sc >= a.k) break;
+                    T val = acc[zi][st][v];
+                    if (a.ct_rowptr) {
+                        const int64_t f0 = a.ct_rowptr[row], f1 = a.ct_rowptr[row + 1];
+                        for (int64_t e = f0; e < f1; ++e)
+                            val += a.ct_val[e] * a.Wnl[(int64_t)a.ct_col[e] * a.ldw + sc];
+                    }
+                    T out = val * a.alpha;
+                    if (a.use_beta) out = out + a.beta * a.X[row * a.ldx + sc];
+                    if (a.use_delta) out = out + a.delta * a.Z[row * a.ldz + sc];
+                    a.Y[row * a.ldy + sc] = out;
+                }
+                continue;
+            }
             int s[NST];
             bool on[NST];
             T val[NST], xb[NST], zb[NST];
@@ -588,6 +613,18 @@ int launch_db(ttdft_ctx ctx, const BrickArgs<T> &a, int cogroups) {
                 return TTDFT_OK;
             }
         }
+        // Rows of up to four entries of C^T on average: a tile at a time in the
+        // one-plane FP32 form (343,000 x 900, 2 entries a row: 37.0 ms against
+        // 38.9; 64,000 x 300, 7 a row: 3.18 against 2.92).
+        if constexpr (sizeof(T) == 4 && ZB == 1) {
+            if (!a.long_rows) {
+                hipLaunchKernelGGL(
+                    (brick_spmm_kernel<T, KS, NST, DB, C::DEPTH, C::GXM, C::G, ZB, true>),
+                    dim3((unsigned)blocks), dim3(64 * C::G * C::GXM), 0, ctx->stream, a);
+                TT_LAUNCH_CHECK();
+                return TTDFT_OK;
+            }
+        }
         hipLaunchKernelGGL((brick_spmm_kernel<T, KS, NST, DB, C::DEPTH, C::GXM, C::G, ZB>),
                            dim3((unsigned)blocks), dim3(64 * C::G * C::GXM), 0, ctx->stream, a);
         TT_LAUNCH_CHECK();
@@ -619,12 +656,14 @@ bool band_wide_loads(const BrickArgs<T> &a) {
 }
 
 template <typename T, int KS>
-int launch_ks(ttdft_ctx ctx, const BrickArgs<T> &a, int cogroups, int zb) {
+int launch_ks(ttdft_ctx ctx, BrickArgs<T> a, int cogroups, int zb) {
     TT_CHECK(a.gxb >= 1 && (cogroups ? CoShape<T, 0>::G * a.gxb : a.gxb + a.nsplit) <= 16,
              TTDFT_EBADARG, "band SpMM: %d x-bricks per chunk", a.gxb);
     TT_CHECK((int64_t)a.rx * a.ldx * (int64_t)sizeof(T) < ((int64_t)1 << 31), TTDFT_EBADARG,
              "band SpMM: one x-line of X exceeds 2 GiB");
     const bool wide = band_wide_loads(a);
+    const int ve = wide ? 16 / (int)sizeof(T) : 1;
+    a.slast = (a.k - 1) / ve * ve;
     if constexpr (two_planes_fit(KS)) {
         if (zb == 2) {
             TT_CHECK(wide && cogroups, TTDFT_EBADARG, "band SpMM: no two-plane form here");
@@ -717,6 +756,7 @@ int launch_band_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t
                             (const double *)W, k, (double *)Y, ldy, (const double *)Z, ldz,
                             k, H->rx, H->ry, H->rz, H->bx, H->by, H->bz, H->gxn, H->hyn,
                             H->gxb, H->nxc, 0, 0, 0, alpha, beta, delta, use_beta, use_delta};
+        a.long_rows = H->nnz_c > 4 * H->n;
         return launch_brick<double>(ctx, a, H->ks);
     }
     TT_CHECK(H->mf32, TTDFT_EBADARG, "no FP32 band copy of H_loc uploaded");
@@ -726,6 +766,7 @@ int launch_band_spmm(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t
                        k, H->rx, H->ry, H->rz, H->bx, H->by, H->bz, H->gxn, H->hyn,
                        H->gxb, H->nxc, 0, 0, 0, (float)alpha, (float)beta, (float)delta,
                        use_beta, use_delta};
+    a.long_rows = H->nnz_c > 4 * H->n;
     return launch_brick<float>(ctx, a, H->ks);
 }
 
