@@ -1015,11 +1015,13 @@ def test_filter_without_room_for_partial_sums(monkeypatch, form):
 
 @pytest.mark.parametrize("dtype", [E.F64, E.F32])
 @pytest.mark.parametrize("p", [4, 60])
-@pytest.mark.parametrize("bx,k,ld", [(3, 300, 300), (3, 250, 251), (7, 260, 260)])
+@pytest.mark.parametrize("bx,k,ld", [(3, 300, 300), (3, 250, 251), (7, 260, 260), (3, 16, 16),
+                                     (2, 16, 17)])
 def test_band_epilogue_over_projector_rows(ctx, dtype, p, bx, k, ld):
     """The state-group forms of the band product (aligned rows, unaligned rows,
-    the widest band) with rows of up to four entries of C^T on average and with
-    more, in a filter, so that the recurrence is in the epilogue too."""
+    the widest band) and one tile of states, the last x-brick's tiles split over
+    two waves, with rows of up to four entries of C^T on average and with more,
+    in a filter, so that the recurrence is in the epilogue too."""
     s = E.SynthHam(18, 10, 9, bx, 3, 3, p, seed=61)
     assert (s.nnz_c > 4 * s.n) == (p == 60)
     ham = ctx.ham_upload(s, E.HAM_F64 | E.HAM_F32, tucker=True)
