@@ -374,6 +374,7 @@ __global__ __launch_bounds__(1024) void reduce_tile_partials_kernel(
     const int64_t stride = (int64_t)nt * nt * 256;
     const P_t *p = P + ((int64_t)tb * nt + ta) * 256 + e;
     double s = 0.0;
+#pragma unroll 8
     for (int c = nchunks * q / NQ; c < nchunks * (q + 1) / NQ; ++c) s += (double)p[c * stride];
     if constexpr (NQ > 1) {
         part[q][e] = s;
