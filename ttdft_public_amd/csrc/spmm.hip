@@ -1425,26 +1425,12 @@ static int dense_split_form() {
     return env ? std::atoi(env) : 1;
 }
 
-// Does the dense product of k states run as the split product?  It takes two
-// launches, and a small matrix gives its row blocks too few workgroups: up to
-// 4,096 rows (two state tiles in FP64, three in FP32) or 1,024 and 1,728 (more
-// tiles) the one-kernel form, 16 rows a workgroup, is faster.  Filters of nine
-// products, one kernel against split, us:  FP64 n = 512, k = 16: 64 / 125;
-// 1,000 x 90: 221 / 245; 1,331 x 50: 232 / 221; 4,096 x 30: 310 / 321;
-// 8,000 x 24: 1,342 / 948.  FP32 1,000 x 90: 162 / 202; 1,728 x 90: 252 / 257;
-// 2,744 x 90: 375 / 308; 4,096 x 30: 200 / 245; 8,000 x 24: 739 / 473.
-static bool dense_split(int64_t n, int32_t k, int dtype) {
-    const int form = dense_split_form();
-    if (form != 1) return form != 0;
-    const bool f64 = dtype == TTDFT_F64;
-    return n > (k <= (f64 ? 32 : 48) ? 4096 : (f64 ? 1024 : 1728));
-}
-
 // Tiling of the dense product of k states: fewest columns of at most 96
 // states, then the fewest 16-state tiles that cover k in that many columns
 // (each column streams H once).
 struct DenseTiling {
     int ncol, jt, nparts, chunk = 0;  // chunk: most blocks of a part (block product)
+    double stages = 0.0;  // cost of the cheapest dense split, in ring stages
     // one part's sums, all parts' (rounded up to 256 bytes), the fragments of X
     // behind them, and the whole
     size_t part_bytes, partial_bytes, fragment_bytes, bytes;
@@ -1499,7 +1485,43 @@ static DenseTiling dense_tiling(const ttdft_ham_s *H, int32_t k, int dtype,
         }
     }
     d.set_parts(best_within <= (dtype == TTDFT_F64 ? 1.25 : 2.5) * best ? nparts : 0);
+    d.stages = best;
     return d;
+}
+
+// Does the dense product of k states run as the split product?  From 8,192 rows
+// on (8,000 x 24 FP64 1,344 us in one kernel, 953 split, a filter of nine
+// products; 8,000 x 1 FP32 391 / 488).  Below, the cheaper of two costs in us, by
+// 16-state tiles and type:  the split's two further launches and its ring
+// stages (dense_tiling), against the one kernel's rounds of 256 workgroups of 16
+// rows, one a CU, that each walk all of l.  Fitted to filters of 512 to 8,000
+// rows with 1 to 400 states, of which it loses 0.3% against the better form.
+// One kernel / split, us, FP64: 512 x 16 64 / 131; 1,331 x 200 246 / 339;
+// 1,728 x 200 537 / 419; 4,096 x 96 563 / 637; 4,913 x 16 520 / 359.
+// FP32: 1,728 x 96 224 / 293, x 300 435 / 337; 2,744 x 80 313 / 302; 4,096 x 24
+// 201 / 235, x 96 461 / 393.
+static bool dense_split(const ttdft_ham_s *H, int32_t k, int dtype) {
+    const int form = dense_split_form();
+    if (form != 1) return form != 0;
+    if (H->n > 8192) return true;
+    static const struct {
+        double split, stage, one, row;
+    } cost[2][6] = {{{8.2, 1.13, 3.8, 0.0056},
+                     {9.3, 1.31, 4.6, 0.0078},
+                     {8.2, 1.74, 6.1, 0.0103},
+                     {7.2, 2.11, 7.0, 0.0135},
+                     {2.9, 2.66, 7.1, 0.0146},
+                     {4.0, 2.67, 5.7, 0.0162}},
+                    {{6.5, 1.25, 3.8, 0.0024},
+                     {8.2, 1.20, 3.6, 0.0048},
+                     {8.6, 1.40, 4.4, 0.0067},
+                     {11.5, 1.49, 4.4, 0.0098},
+                     {12.3, 1.70, 4.4, 0.0118},
+                     {12.7, 1.87, 3.7, 0.0135}}};
+    const DenseTiling d = dense_tiling(H, k, dtype);
+    const auto &c = cost[dtype == TTDFT_F64 ? 0 : 1][d.jt - 1];
+    const int64_t rounds = ((H->n + 15) / 16 * d.ncol + 255) / 256;
+    return c.split + c.stage * d.stages < c.one + c.row * (double)(rounds * H->dense_ld);
 }
 
 template <typename T, int JT>
@@ -1807,7 +1829,7 @@ int ham_step(ttdft_ctx ctx, const ttdft_ham_s *H, const void *X, int64_t ldx, vo
         // kernel.  (The same result up to the order of the additions.)
         void *P = nullptr;
         DenseTiling tiling(H, k, dtype);
-        if (blocks || (dense && dense_split(H->n, k, dtype))) {
+        if (blocks || (dense && dense_split(H, k, dtype))) {
             const size_t off = W ? ((size_t)nl_workspace(H, k) * es + 255) / 256 * 256 : 0;
             const size_t limit = !ws ? SIZE_MAX : off < ws_bytes ? ws_bytes - off : 0;
             tiling = blocks ? block_tiling(H, k, dtype, limit) : dense_tiling(H, k, dtype, limit);
