@@ -615,9 +615,10 @@ int launch_db(ttdft_ctx ctx, const BrickArgs<T> &a, int cogroups) {
             }
         }
         // Rows of up to four entries of C^T on average: a tile at a time in the
-        // one-plane FP32 form (343,000 x 900, 2 entries a row: 37.0 ms against
-        // 38.9; 64,000 x 300, 7 a row: 3.18 against 2.92).
-        if constexpr (sizeof(T) == 4 && ZB == 1) {
+        // one-plane FP32 form of the widest bands (343,000 x 900, 2 entries a row:
+        // 37.0 ms against 38.9; 64,000 x 600, 1.5 a row: 5.18 against 5.39).
+        // Narrower ones walk together (85,184 x 263, 1.1 a row: 2.73 against 2.95).
+        if constexpr (sizeof(T) == 4 && ZB == 1 && !two_planes_fit(KS)) {
             if (!a.long_rows) {
                 hipLaunchKernelGGL(
                     (brick_spmm_kernel<T, KS, NST, DB, C::DEPTH, C::GXM, C::G, ZB, true>),
