@@ -91,7 +91,7 @@ struct ttdft_ctx_s {
     std::vector<ttdft::PendingTiming> *pending = nullptr;
     // scratch: [0] second X block for the filter / rotation, [1] small k x k
     // work, [2] Gram partials, [3] nonlocal projections, [4..7] misc, [8] partial
-    // sums of the split dense product
+    // sums and operand fragments of the split dense and the block product
     ttdft::Scratch scratch[9];
     // network-layer work: [0] transformed weights, [1] weight-gradient partials
     ttdft::Scratch nn_scratch[2];
